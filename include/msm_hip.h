@@ -345,6 +345,7 @@ int msm_set_option(msm_sim* sim, int option, int value);
 #define MSM_PASS_LDS_TABLE   4  /* global list, table window in LDS */
 #define MSM_PASS_BRICK_TABLE 5  /* LDS-staged positions and table window in LDS */
 #define MSM_PASS_STAGED      6  /* staged bricks: halo images resolved once, slots per pair */
+#define MSM_PASS_WIDE        7  /* 8 to 32 lanes per atom, global list and table (small boxes) */
 /* Current value of an option (every MSM_OPT_* above). */
 int msm_get_option(msm_sim* sim, int option, int* value);
 

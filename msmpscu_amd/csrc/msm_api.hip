@@ -57,9 +57,10 @@ struct msm_sim {
     // force table
     bool has_table = false;
     TabDev tab{};
-    double2* d_b2 = nullptr;
+    double* d_b1 = nullptr;
+    double2 *d_b2 = nullptr, *d_f2 = nullptr;
     double4 *d_f4 = nullptr, *d_e4 = nullptr, *d_m4 = nullptr;
-    size_t cap_b2 = 0, cap_f4 = 0, cap_e4 = 0, cap_m4 = 0;  // elements allocated
+    size_t cap_b1 = 0, cap_f2 = 0, cap_b2 = 0, cap_f4 = 0, cap_e4 = 0, cap_m4 = 0;  // elements allocated
     int tab_ngroup = 0;
 
     // control
@@ -73,6 +74,7 @@ struct msm_sim {
     std::vector<BoxDev> boxes;
     BoxDev* d_boxes = nullptr;
     int ncell_total = 0;
+    double half_min = 0.0;  // half the shortest periodic box length
 
     // atoms
     int n = 0, n_alloc = 0;
@@ -116,6 +118,7 @@ struct msm_sim {
     int force_lanes = 0;   // lanes per atom of the LDS-table force pass (0: as force_path)
     int cell_brick = 1;    // cells are numbered in bricks of cell_brick^3 (1: row-major)
     msm::LtShape lt{1024, 1, 1024, 1};  // block / workgroups per CU of the LDS-table passes
+    int auto_pass = 1;     // no pass option set: lanes and table placement by size (walk_plan)
     int compact = 0;       // global-list path: force pass reads the density pass's in-cutoff list
 
     // adjoint scratch (allocated on first use)
@@ -146,6 +149,7 @@ struct msm_sim {
     int nl_wide = 0;   // bricks planned for the wide list kernel
     int list_sidx = 0; // the current list holds halo slots (written for the brick passes)
     int tuning = 0;    // msm_autotune is running: lists carry halo slots for every candidate
+    double kmean = 0.0;       // list length expected from the largest box's density (at upload)
     std::vector<double> occ;  // mean atoms per non-empty cell, per box (at upload)
     int* d_brick_box = nullptr;
 
@@ -525,6 +529,14 @@ int plan_bricks(msm_sim* s, const double* xp, int n) {
             }
         s->occ[bidx] = nonempty ? static_cast<double>(occ) / nonempty : 1.0;
     }
+    size_t big = 0;
+    for (size_t b = 0; b < s->boxes.size(); ++b)
+        if (s->boxes[b].natoms > s->boxes[big].natoms) big = b;
+    const BoxDev& b = s->boxes[big];
+    double rnl = 0.0, cell = 1.0;
+    for (double r : s->nb_rm) rnl = std::max(rnl, r);
+    for (int k = 0; k < 3; ++k) cell *= b.len[k] / b.ncell[k];
+    s->kmean = s->occ[big] * (4.0 / 3.0) * 3.14159265358979 * rnl * rnl * rnl / cell;
     return replan_bricks(s);
 }
 
@@ -546,6 +558,11 @@ int eff_path(const msm_sim* s) { return s->force_path == 5 ? 2 : s->force_path; 
 
 int lt_force_lanes(const msm_sim* s) {
     return (s->force_lanes > 0 && eff_path(s) != 3) ? s->force_lanes : eff_path(s);
+}
+
+// Both list-walk passes hold the upper half of the table in LDS.
+bool walk_lds_ok(const msm_sim* s) {
+    return msm::walk_window_ok(s->tab, 0, s->lt.wgs_d) && msm::walk_window_ok(s->tab, 1, s->lt.wgs_f);
 }
 
 bool use_lds_table(const msm_sim* s) {
@@ -571,9 +588,60 @@ bool use_brick_table(const msm_sim* s) {
            p.cap_f > 0;
 }
 
+// Lanes per atom of a pass when no option fixes the kernel (MSM_OPT_FORCE_PATH and the other
+// pass options leave s->auto_pass): enough that the pass holds about 120,000 lanes (twice that
+// for long lists), at least 2 (4).  Measured, density + force + 1/10 list per step: 2,000 W atoms
+// (26 neighbours) 37.9 us at 2 lanes, 21.2 / 19.5 / 19.2 at 8 / 16 / 32; 16,000 atoms 38.0 at 2,
+// 23.3 / 24.7 / 30.1; 54,000 atoms 30.1 / 32.0 / 38.1 at 2 / 4 / 8, 137,000 48.7 / 51.0 / 64.1;
+// Cu-Ni (86 neighbours) 42,600 atoms 131.9 / 100.5 / 93.8 at 2 / 4 / 8, 442,000 atoms 377.7 /
+// 374.8 / 421.6.
+int auto_lanes(const msm_sim* s) {
+    const bool lng = s->kmean >= 48.0;
+    int lanes = lng ? 4 : 2;
+    while (lanes < 32 && static_cast<double>(s->n) * lanes < (lng ? 240000.0 : 120000.0))
+        lanes *= 2;
+    return lanes;
+}
+
+// The list-walk pass (msm_walk.hip) and its shape; false: another kernel runs.
+bool walk_plan(const msm_sim* s, int force, msm::WalkPlan& p) {
+    if (s->n >= msm::kWalkMaxAtoms || s->compact) return false;
+    const int fp = eff_path(s);
+    if (fp != 1 && fp != 2 && fp != 4) return false;
+    p.block = force ? s->lt.block_f : s->lt.block_d;
+    p.wgs = force ? s->lt.wgs_f : s->lt.wgs_d;
+    p.sweep = s->lt.sweep;
+    // inner units skip the minimum image; worth it when half a box is well beyond the list radius
+    double rnl = 0.0;
+    for (double r : s->nb_rm) rnl = std::max(rnl, r);
+    p.margin = rnl;
+    p.kimg = 0;
+    if (s->half_min >= 1.25 * rnl) {
+        const double k = std::floor(std::sqrt(s->half_min * (1.0 - 1.0e-9)) * s->tab.csi);
+        p.kimg = k < 1.0e9 ? static_cast<int>(k) : 1000000000;
+    }
+    if (!s->auto_pass) {
+        p.tl = 1;
+        p.lanes = force ? lt_force_lanes(s) : fp;
+        return s->table_lds && walk_lds_ok(s);
+    }
+    p.lanes = auto_lanes(s);
+    // filling the LDS window costs more than the global lookups it saves below about 10^6 pairs:
+    // 16,000 W atoms at 8 lanes 25.6 us with it, 23.3 without; 54,000 at 4 lanes 31.0, at 8 lanes
+    // from global memory 38.7; 42,600 Cu-Ni atoms at 8 lanes 93.8 with it, 108.4 without
+    p.tl = p.lanes <= 8 && s->n * s->kmean >= 8.0e5 && msm::walk_window_ok(s->tab, force, p.wgs);
+    if (!p.tl) {
+        // a table too large for the LDS on a large box: the two-lane global-table pass
+        if (s->n * s->kmean >= 8.0e6) return false;
+        p.lanes = std::max(p.lanes, 8);
+    }
+    return true;
+}
+
 void enqueue_density(msm_sim* s) {
     TimedScope ts(s, MSM_KCLASS_DENSITY);
     AtomsDev a = atoms_view(s, s->scur, s->pcur);
+    msm::WalkPlan wp{};
     if (use_staged(s))
         msm::launch_density_sb(s->lt, s->nbricks, s->d_brick_box, a, list_view(s), s->tab,
                                s->d_boxes, s->sb.start, s->ncell_total, s->d_err, s->stream);
@@ -581,6 +649,9 @@ void enqueue_density(msm_sim* s) {
         msm::launch_density_bt(s->bt_lanes, s->lt, s->nbricks, s->d_brick_box, a, list_view(s),
                                s->tab, s->d_boxes, s->sb.start, s->ncell_total, s->d_err,
                                s->stream);
+    else if (walk_plan(s, 0, wp))
+        msm::launch_density_walk(wp, a, list_view(s), s->tab, s->boxes[0], s->d_boxes,
+                                 multibox(s), s->d_err, s->stream);
     else if (use_lds_table(s))
         msm::launch_density_lt(eff_path(s), s->lt, a, list_view(s), s->tab, s->boxes[0],
                                s->d_boxes, multibox(s), s->d_err, s->stream);
@@ -609,12 +680,16 @@ void enqueue_force(msm_sim* s, int mode, int write_f, double h) {
     sp.mode = mode;
     sp.write_f = write_f;
     sp.track_dis = s->track_dis;
+    msm::WalkPlan wp{};
     if (use_staged(s))
         msm::launch_force_sb(s->lt, s->nbricks, s->d_brick_box, a, list_view(s), s->tab,
                              s->d_boxes, s->sb.start, s->ncell_total, sp, s->stream);
     else if (use_brick_table(s))
         msm::launch_force_bt(s->bt_lanes, s->lt, s->nbricks, s->d_brick_box, a, list_view(s),
                              s->tab, s->d_boxes, s->sb.start, s->ncell_total, sp, s->stream);
+    else if (walk_plan(s, 1, wp))
+        msm::launch_force_walk(wp, a, list_view(s), s->tab, s->boxes[0], s->d_boxes,
+                               multibox(s), sp, s->stream);
     else if (use_lds_table(s))
         msm::launch_force_lt(lt_force_lanes(s), s->lt, a, list_view(s), s->tab, s->boxes[0],
                              s->d_boxes, multibox(s), sp, s->stream);
@@ -781,6 +856,8 @@ int msm_destroy(msm_sim* s) {
     }
     for (hipEvent_t e : s->evpool) (void)hipEventDestroy(e);
     if (s->fm_ev) (void)hipEventDestroy(s->fm_ev);
+    dfree(&s->d_b1);
+    dfree(&s->d_f2);
     dfree(&s->d_b2);
     dfree(&s->d_f4);
     dfree(&s->d_e4);
@@ -842,6 +919,8 @@ int msm_set_force_table(msm_sim* s, int pot_type, int ngroup, int nkind, int nta
     };
     std::vector<double2> hb2(static_cast<size_t>(nkind) * ntab2);
     std::vector<double4> hf4(static_cast<size_t>(nkind) * ntab2), he4(hf4.size());
+    std::vector<double> hb1(hb2.size());
+    std::vector<double2> hf2(hb2.size());
     for (int k = 0; k < nkind; ++k)
         for (int i = 0; i < ntab2; ++i) {
             const size_t a = static_cast<size_t>(k) * ntab2 + i;
@@ -852,6 +931,8 @@ int msm_set_force_table(msm_sim* s, int pot_type, int ngroup, int nkind, int nta
             hf4[a] = make_double4(fr, fr1 - fr, fb, fb1 - fb);
             const double pr = knot(potr, k, i), pr1 = knot(potr, k, i + 1);
             he4[a] = make_double4(pr, pr1 - pr, pb, pb1 - pb);
+            hb1[a] = pb;
+            hf2[a] = make_double2(fr, fb);
         }
     TabDev t;
     std::memset(&t, 0, sizeof(t));  // byte-wise comparable with the current table
@@ -873,7 +954,11 @@ int msm_set_force_table(msm_sim* s, int pot_type, int ngroup, int nkind, int nta
     int rc = dreserve(s, &s->d_b2, hb2.size(), s->cap_b2);
     if (rc == MSM_OK) rc = dreserve(s, &s->d_f4, hf4.size(), s->cap_f4);
     if (rc == MSM_OK) rc = dreserve(s, &s->d_e4, he4.size(), s->cap_e4);
+    if (rc == MSM_OK) rc = dreserve(s, &s->d_b1, hb1.size(), s->cap_b1);
+    if (rc == MSM_OK) rc = dreserve(s, &s->d_f2, hf2.size(), s->cap_f2);
     if (rc != MSM_OK) return rc;
+    HIPCHK(s, hipMemcpy(s->d_b1, hb1.data(), hb1.size() * sizeof(double), hipMemcpyHostToDevice));
+    HIPCHK(s, hipMemcpy(s->d_f2, hf2.data(), hf2.size() * sizeof(double2), hipMemcpyHostToDevice));
     HIPCHK(s, hipMemcpy(s->d_b2, hb2.data(), hb2.size() * sizeof(double2), hipMemcpyHostToDevice));
     HIPCHK(s, hipMemcpy(s->d_f4, hf4.data(), hf4.size() * sizeof(double4), hipMemcpyHostToDevice));
     HIPCHK(s, hipMemcpy(s->d_e4, he4.data(), he4.size() * sizeof(double4), hipMemcpyHostToDevice));
@@ -905,6 +990,8 @@ int msm_set_force_table(msm_sim* s, int pot_type, int ngroup, int nkind, int nta
         t.nkind1 = 1;
         t.rhod = 1.0;
     }
+    t.b1 = s->d_b1;
+    t.f2 = s->d_f2;
     t.b2 = s->d_b2;
     t.f4 = s->d_f4;
     t.e4 = s->d_e4;
@@ -1005,6 +1092,10 @@ int msm_set_boxes(msm_sim* s, int nbox, const int* natoms, const double* lo, con
         if (rc != MSM_OK) return rc;
         s->sort_cap = need;
     }
+    s->half_min = HUGE_VAL;
+    for (const BoxDev& b : s->boxes)
+        for (int k = 0; k < 3; ++k)
+            if (b.ifpd[k]) s->half_min = std::min(s->half_min, 0.5 * b.len[k]);
     rc = dalloc(s, &s->d_ebox, nbox);
     if (rc != MSM_OK) return rc;
     s->has_boxes = true;
@@ -2014,18 +2105,22 @@ int msm_set_option(msm_sim* s, int option, int value) {
             if (value < 0 || value > 8 || (value > 5 && value != 8))
                 return set_err(s, MSM_ERR_ARG, "force path must be 0, 1, 2, 3, 4, 5 or 8");
             s->force_path = value;
+            s->auto_pass = 0;
             clear_graphs(s);
             return MSM_OK;
         case MSM_OPT_COMPACT_LIST:
             s->compact = value ? 1 : 0;
+            s->auto_pass = 0;
             clear_graphs(s);
             return MSM_OK;
         case MSM_OPT_CHUNK_SWEEP:
             s->lt.sweep = value ? 1 : 0;
+            s->auto_pass = 0;
             clear_graphs(s);
             return MSM_OK;
         case MSM_OPT_TABLE_LDS:
             s->table_lds = value ? 1 : 0;
+            s->auto_pass = 0;
             clear_graphs(s);
             return MSM_OK;
         case MSM_OPT_CELL_BRICK:
@@ -2049,6 +2144,7 @@ int msm_set_option(msm_sim* s, int option, int value) {
             if (value != 0 && value != 1 && value != 2 && value != 4)
                 return set_err(s, MSM_ERR_ARG, "force lanes must be 0, 1, 2 or 4");
             s->force_lanes = value;
+            s->auto_pass = 0;
             clear_graphs(s);
             return MSM_OK;
         case MSM_OPT_LT_DENSITY_BLOCK:
@@ -2056,6 +2152,7 @@ int msm_set_option(msm_sim* s, int option, int value) {
             if (value != 256 && value != 512 && value != 1024)
                 return set_err(s, MSM_ERR_ARG, "LDS-table block must be 256, 512 or 1024");
             (option == MSM_OPT_LT_DENSITY_BLOCK ? s->lt.block_d : s->lt.block_f) = value;
+            s->auto_pass = 0;
             clear_graphs(s);
             return MSM_OK;
         case MSM_OPT_LT_DENSITY_WGS:
@@ -2063,6 +2160,7 @@ int msm_set_option(msm_sim* s, int option, int value) {
             if (value < 1 || value > 16)
                 return set_err(s, MSM_ERR_ARG, "LDS-table workgroups per CU must be 1..16");
             (option == MSM_OPT_LT_DENSITY_WGS ? s->lt.wgs_d : s->lt.wgs_f) = value;
+            s->auto_pass = 0;
             clear_graphs(s);
             return MSM_OK;
         default:
@@ -2074,6 +2172,8 @@ int msm_set_option(msm_sim* s, int option, int value) {
 static int pass_kernel(const msm_sim* s) {
     if (use_staged(s)) return MSM_PASS_STAGED;
     if (use_brick_table(s)) return MSM_PASS_BRICK_TABLE;
+    msm::WalkPlan wp{};
+    if (walk_plan(s, 1, wp)) return wp.tl ? MSM_PASS_LDS_TABLE : MSM_PASS_WIDE;
     if (use_lds_table(s)) return MSM_PASS_LDS_TABLE;
     if (eff_path(s) == 3) return MSM_PASS_LANE_PAIR;
     if (eff_path(s) > 0) return MSM_PASS_LANES;
@@ -2129,9 +2229,10 @@ int msm_autotune(msm_sim* s, int reps, int* choice, double* best_ms) {
     if (reps < 1 || reps > 1000) return set_err(s, MSM_ERR_ARG, "reps must be 1..1000");
     (void)hipSetDevice(s->device);
     struct Cand {
-        int fp, lds, bd, wd, bf, wf, lanes, flanes = 0;
+        int fp, lds, bd, wd, bf, wf, lanes, flanes = 0, autop = 0;
     };
-    std::vector<Cand> cands;
+    // the choice by size first (reported as its path and shape)
+    std::vector<Cand> cands{{2, 1, 1024, 1, 1024, 1, 1, 0, 1}};
     if (msm::lt_window(s->tab, 1, 1).wf * 2 >= s->tab.ntab2) {
         for (int fp : {2, 3, 1, 4}) {
             cands.push_back({fp, 1, 1024, 1, 1024, 1, 1});
@@ -2206,6 +2307,7 @@ int msm_autotune(msm_sim* s, int reps, int* choice, double* best_ms) {
         s->lt = msm::LtShape{cands[c].bd, cands[c].wd, cands[c].bf, cands[c].wf};
         s->bt_lanes = cands[c].lanes;
         s->force_lanes = cands[c].flanes;
+        s->auto_pass = cands[c].autop;
         float ms = 0.f;
         rc = time_it([&] {
             enqueue_density(s);
@@ -2227,6 +2329,7 @@ int msm_autotune(msm_sim* s, int reps, int* choice, double* best_ms) {
     s->lt = msm::LtShape{w.bd, w.wd, w.bf, w.wf};
     s->bt_lanes = w.lanes;
     s->force_lanes = w.flanes;
+    s->auto_pass = w.autop;
     clear_graphs(s);
     // leave F' and F as the chosen kernels compute them
     enqueue_density(s);
@@ -2433,7 +2536,7 @@ int msm_set_spline_table(msm_sim* s, const double* coef, int ld, int coef_on_dev
         c = s->fm_coef;
     }
     // same buffers, sizes and grid: the table descriptor and captured segments stay valid
-    msm::launch_spline_tables(c, ld, s->tab, s->d_b2, s->d_f4, s->d_e4, s->d_m4, s->stream);
+    msm::launch_spline_tables(c, ld, s->tab, s->d_b1, s->d_f2, s->d_b2, s->d_f4, s->d_e4, s->d_m4, s->stream);
     HIPCHK(s, hipGetLastError());
     // stream-ordered before every later call on this context; msm_set_force_table, whose
     // copies are not, and the next build wait for the event.  A caller's device coefficients

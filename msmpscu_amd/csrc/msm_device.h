@@ -25,6 +25,30 @@ static __device__ __forceinline__ int atom_index() {
     return xcd_block(gridDim.x) * blockDim.x + threadIdx.x;
 }
 
+// Element of an array at a byte offset below 4 GB (scalar base + 32-bit lane offset: no 64-bit
+// address arithmetic in the lanes).
+template <typename T>
+__device__ __forceinline__ T& at(T* p, unsigned off) {
+    return *reinterpret_cast<T*>(reinterpret_cast<char*>(p) + off);
+}
+template <typename T>
+__device__ __forceinline__ const T& at(const T* p, unsigned off) {
+    return *reinterpret_cast<const T*>(reinterpret_cast<const char*>(p) + off);
+}
+
+// Atom index of the integrator's arrays: a plain index, or one whose byte offsets fit 32 bits.
+struct AtomIx {
+    unsigned i;
+};
+template <typename T>
+__device__ __forceinline__ T& el(T* p, int i) {
+    return p[i];
+}
+template <typename T>
+__device__ __forceinline__ T& el(T* p, AtomIx x) {
+    return at(p, x.i * static_cast<unsigned>(sizeof(T)));
+}
+
 static inline unsigned grid_for(int n) { return static_cast<unsigned>((n + kBlock - 1) / kBlock); }
 
 // Local id of cell (ix, iy, iz) in box b.  Cells are numbered in bricks of cbs^3 cells (x fastest
@@ -148,16 +172,17 @@ struct AtomState {
     double vx, vy, vz, dx, dy, dz;
 };
 
-__device__ __forceinline__ void load_atom_state(const AtomsDev& a, const StepParams& sp, int i,
+template <typename I>
+__device__ __forceinline__ void load_atom_state(const AtomsDev& a, const StepParams& sp, I i,
                                                 AtomState& s) {
-    s.vx = a.vx[i];
-    s.vy = a.vy[i];
-    s.vz = a.vz[i];
+    s.vx = el(a.vx, i);
+    s.vy = el(a.vy, i);
+    s.vz = el(a.vz, i);
     s.dx = s.dy = s.dz = 0.0;
     if (sp.track_dis) {
-        s.dx = a.dx[i];
-        s.dy = a.dy[i];
-        s.dz = a.dz[i];
+        s.dx = el(a.dx, i);
+        s.dy = el(a.dy, i);
+        s.dz = el(a.dz, i);
     }
 }
 
@@ -165,17 +190,17 @@ __device__ __forceinline__ void load_atom_state(const AtomsDev& a, const StepPar
 // predictor of the next step (Predictor_KERNEL0, :242-384) with the same forces, for atom i.
 // Positions of MODE 2 go to a.pos_out (the next step's buffer).  pre: the atom's velocity and
 // displacement as read by load_atom_state, or null to read them here.
-template <int MODE>
+template <int MODE, typename I>
 __device__ __forceinline__ void integrate_atom(const AtomsDev& a, const TabDev& t, const BoxDev& b,
-                                               const StepParams& sp, int i, int st, bool active,
+                                               const StepParams& sp, I i, int st, bool active,
                                                const double4& pi, int ti, double fpx, double fpy,
                                                double fpz, const AtomState* pre = nullptr) {
         if (active) {
 #pragma clang fp contract(off)
             const double cm0 = t.cm[ti];
             const double ax = fpx / cm0, ay = fpy / cm0, az = fpz / cm0;
-            double vx = pre ? pre->vx : a.vx[i], vy = pre ? pre->vy : a.vy[i],
-                   vz = pre ? pre->vz : a.vz[i];
+            double vx = pre ? pre->vx : el(a.vx, i), vy = pre ? pre->vy : el(a.vy, i),
+                   vz = pre ? pre->vz : el(a.vz, i);
             // Correction_KERNEL
             if (!(st & (STATU_FIXVELX | STATU_FIXPOSX))) vx = vx + sp.hs2 * ax;
             if (!(st & (STATU_FIXVELY | STATU_FIXPOSY))) vy = vy + sp.hs2 * ay;
@@ -209,22 +234,22 @@ __device__ __forceinline__ void integrate_atom(const AtomsDev& a, const TabDev& 
                 if (!(stat & (STATU_FIXVELY | STATU_FIXPOSY))) vy = vy + sp.hs2 * ay;
                 if (!(stat & (STATU_FIXVELZ | STATU_FIXPOSZ))) vz = vz + sp.hs2 * az;
                 if (sp.track_dis) {
-                    a.dx[i] = (pre ? pre->dx : a.dx[i]) + dx;
-                    a.dy[i] = (pre ? pre->dy : a.dy[i]) + dy;
-                    a.dz[i] = (pre ? pre->dz : a.dz[i]) + dz;
+                    el(a.dx, i) = (pre ? pre->dx : el(a.dx, i)) + dx;
+                    el(a.dy, i) = (pre ? pre->dy : el(a.dy, i)) + dy;
+                    el(a.dz, i) = (pre ? pre->dz : el(a.dz, i)) + dz;
                 }
                 if (x > b.lo[0] + b.len[0] || y > b.lo[1] + b.len[1] || z > b.lo[2] + b.len[2])
                     stat = STATU_OUTOFBOX | STATU_REFLECT;
                 else if (x < b.lo[0] || y < b.lo[1] || z < b.lo[2])
                     stat = STATU_OUTOFBOX | STATU_TRANSMIT;
-                if (stat != st) a.statu[i] = stat;
-                a.pos_out[i] = make_double4(x, y, z, 0.0);
+                if (stat != st) el(a.statu, i) = stat;
+                el(a.pos_out, i) = make_double4(x, y, z, 0.0);
             }
-            a.vx[i] = vx;
-            a.vy[i] = vy;
-            a.vz[i] = vz;
+            el(a.vx, i) = vx;
+            el(a.vy, i) = vy;
+            el(a.vz, i) = vz;
         } else if constexpr (MODE == 2) {
-            a.pos_out[i] = make_double4(pi.x, pi.y, pi.z, 0.0);
+            el(a.pos_out, i) = make_double4(pi.x, pi.y, pi.z, 0.0);
         }
     }
 

@@ -45,6 +45,8 @@ constexpr int kNlCapPass = 1536;
 constexpr int kNlMaxHalo = 216;
 
 struct TabDev {
+    const double* b1;   // density knots POTB alone (filled into LDS by the list-walk passes)
+    const double2* f2;  // force knots {FPOTR, FPOTB} alone (as b1)
     const double2* b2;  // density table {POTB, dPOTB}, nkind x (ntab+2)
     const double4* f4;  // force table {FPOTR, dFPOTR, FPOTB, dFPOTB}
     const double4* e4;  // energy table {POTR, dPOTR, POTB, dPOTB}
@@ -171,6 +173,34 @@ void launch_density_lt(int tpa, const LtShape& sh, const AtomsDev& a, const List
 void launch_force_lt(int tpa, const LtShape& sh, const AtomsDev& a, const ListDev& l,
                      const TabDev& t, const BoxDev& box0, const BoxDev* boxes, int multibox,
                      const StepParams& sp, hipStream_t s);
+// Persistent grid of kernel k (workgroups per CU capped by what fits and by the work) and the LDS
+// share of one of wgs workgroups on a CU (msm_ldstab.hip).
+unsigned lt_persistent_grid(const void* k, int block, size_t lds, int wgs, int nchunks);
+int lt_lds_budget(int wgs);
+// List-walk passes (msm_walk.hip), for fewer than kWalkMaxAtoms atoms (32-bit byte offsets).
+constexpr int kWalkMaxAtoms = 1 << 27;
+struct WalkDev {  // one launch
+    int k0, w, last;  // knot window: w knots a kind from knot k0; a pair's knot is at most k0 + last
+    int kimg;         // knot from which on a pair may need the minimum image (0: always)
+    double margin;    // atoms further than this from the periodic faces are inner
+    int units, sweep;
+};
+struct WalkPlan {  // one pass
+    int lanes;       // lanes per atom: 1, 2, 4, 8 with the knots in LDS, else 8, 16, 32
+    int tl;          // knots in LDS: a persistent grid of block threads, wgs workgroups per CU
+    int block, wgs;
+    int kimg;
+    double margin;
+    int sweep;
+};
+// Whether the LDS share of one of wgs workgroups holds the upper half of the table.
+bool walk_window_ok(const TabDev& t, int force, int wgs);
+void launch_density_walk(const WalkPlan& pl, const AtomsDev& a, const ListDev& l, const TabDev& t,
+                         const BoxDev& box0, const BoxDev* boxes, int multibox, int* err,
+                         hipStream_t s);
+void launch_force_walk(const WalkPlan& pl, const AtomsDev& a, const ListDev& l, const TabDev& t,
+                       const BoxDev& box0, const BoxDev* boxes, int multibox,
+                       const StepParams& sp, hipStream_t s);
 // LDS bricks with the table window in LDS (msm_ldstab.hip): tpa (1, 2 or 4) lanes per home
 // atom, persistent grids over the bricks of the list build (whose slot list they read); the
 // staged halo capacity (at most the list build's, l.scap) and the windows share the LDS.
@@ -230,7 +260,8 @@ void launch_adjoint(const AtomsDev& a, const ListDev& l, const TabDev& t, const 
 // box energies, dL/dF (caller order, FP(N,3)) and dL/dE for the adjoint and the loss into *loss
 // (part: fm_parts(n) doubles of scratch).  launch_spline_grad: dL/dc (3 rows of ld) from the
 // adjoint's bins of one kind.
-void launch_spline_tables(const double* coef, int ld, const TabDev& t, double2* b2, double4* f4,
+void launch_spline_tables(const double* coef, int ld, const TabDev& t, double* b1, double2* f2,
+                          double2* b2, double4* f4,
                           double4* e4, double4* m4, hipStream_t s);
 int fm_parts(int n);
 void launch_fm_loss(const double* fx, const double* fy, const double* fz, const int* gid, int n,

@@ -1164,9 +1164,11 @@ const DevLimits& dev_limits() {
     return d;
 }
 
+}  // namespace
+
 // Persistent grid: min(requested, co-resident) workgroups per CU of kernel k (cached per kernel,
 // block and LDS size) times the CU count, capped by the work.
-unsigned persistent_grid(const void* k, int block, size_t lds, int wgs, int nchunks) {
+unsigned lt_persistent_grid(const void* k, int block, size_t lds, int wgs, int nchunks) {
     static std::mutex mu;
     static std::map<std::tuple<const void*, int, size_t>, int> cache;
     int per_cu = 0;
@@ -1189,19 +1191,17 @@ unsigned persistent_grid(const void* k, int block, size_t lds, int wgs, int nchu
 }
 
 // LDS bytes one workgroup may take when wgs of them share a CU.
-int lds_budget(int wgs) {
+int lt_lds_budget(int wgs) {
     const DevLimits& d = dev_limits();
     int b = d.lds_cu / (wgs > 0 ? wgs : 1);
     if (b > d.lds_block) b = d.lds_block;
     return b & ~255;
 }
 
-}  // namespace
-
 LtWin lt_window(const TabDev& t, int wgs_d, int wgs_f) {
     LtWin w{};
     const int nk = t.ngroup > 1 ? t.nkind : 1;
-    const int bf = lds_budget(wgs_f) / (16 * nk), bd = lds_budget(wgs_d) / (8 * nk);
+    const int bf = lt_lds_budget(wgs_f) / (16 * nk), bd = lt_lds_budget(wgs_d) / (8 * nk);
     w.wf = t.ntab2 < bf ? t.ntab2 : bf;
     w.k0f = t.ntab2 - w.wf;
     w.wd = t.ntab2 < bd ? t.ntab2 : bd;
@@ -1223,7 +1223,7 @@ void launch_density_lt(int tpa, const LtShape& sh, const AtomsDev& a, const List
 #define MSM_DL(MB, E, P)                                                                     \
     do {                                                                                     \
         auto k = mt ? k_density_lt<MB, 1, E, P> : k_density_lt<MB, 0, E, P>;                 \
-        const unsigned g = persistent_grid(reinterpret_cast<const void*>(k), sh.block_d,     \
+        const unsigned g = lt_persistent_grid(reinterpret_cast<const void*>(k), sh.block_d,     \
                                            lds, sh.wgs_d, nchunks);                          \
         hipLaunchKernelGGL(k, dim3(g), dim3(sh.block_d), lds, s, a, l, t, box0, boxes, w,    \
                            nchunks, err);                                                    \
@@ -1257,7 +1257,7 @@ void launch_force_lt(int tpa, const LtShape& sh, const AtomsDev& a, const ListDe
 #define MSM_FL(MB, M, P)                                                                     \
     do {                                                                                     \
         auto k = mt ? k_force_lt<MB, 1, M, P> : k_force_lt<MB, 0, M, P>;                     \
-        const unsigned g = persistent_grid(reinterpret_cast<const void*>(k), sh.block_f,     \
+        const unsigned g = lt_persistent_grid(reinterpret_cast<const void*>(k), sh.block_f,     \
                                            lds, sh.wgs_f, nchunks);                          \
         hipLaunchKernelGGL(k, dim3(g), dim3(sh.block_f), lds, s, a, l, t, box0, boxes, sp,   \
                            w, nchunks);                                                      \
@@ -1305,9 +1305,9 @@ BtPlan bt_plan(const TabDev& t, const LtShape& sh, int scap) {
     const bool mt = t.ngroup > 1;
     const long nk = mt ? t.nkind : 1;
     const long fixed = static_cast<long>(sizeof(BrickLds)) + 1024;
-    bt_fit(lds_budget(sh.wgs_d) - fixed, bt_atom_bytes(false, mt), 8 * nk, t.ntab2, scap,
+    bt_fit(lt_lds_budget(sh.wgs_d) - fixed, bt_atom_bytes(false, mt), 8 * nk, t.ntab2, scap,
            p.cap_d, p.w.wd);
-    bt_fit(lds_budget(sh.wgs_f) - fixed, bt_atom_bytes(true, mt), 16 * nk, t.ntab2, scap,
+    bt_fit(lt_lds_budget(sh.wgs_f) - fixed, bt_atom_bytes(true, mt), 16 * nk, t.ntab2, scap,
            p.cap_f, p.w.wf);
     p.w.k0d = t.ntab2 - p.w.wd;
     p.w.k0f = t.ntab2 - p.w.wf;
@@ -1340,7 +1340,7 @@ void launch_density_bt(int tpa, const LtShape& sh, int nbricks, const int* brick
 #define MSM_DB(MT, E, P)                                                                       \
     do {                                                                                       \
         auto k = k_density_bt<MT, E, P>;                                                       \
-        const unsigned g = persistent_grid(reinterpret_cast<const void*>(k), sh.block_d, lds,  \
+        const unsigned g = lt_persistent_grid(reinterpret_cast<const void*>(k), sh.block_d, lds,  \
                                            sh.wgs_d, nbricks);                                 \
         hipLaunchKernelGGL(k, dim3(g), dim3(sh.block_d), lds, s, brick_box, nbricks, a, l, t,  \
                            boxes, start, pl.w, pl.cap_d, err);                                 \
@@ -1369,7 +1369,7 @@ void launch_force_bt(int tpa, const LtShape& sh, int nbricks, const int* brick_b
 #define MSM_FB(MT, M, P)                                                                       \
     do {                                                                                       \
         auto k = k_force_bt<MT, M, P>;                                                         \
-        const unsigned g = persistent_grid(reinterpret_cast<const void*>(k), sh.block_f, lds,  \
+        const unsigned g = lt_persistent_grid(reinterpret_cast<const void*>(k), sh.block_f, lds,  \
                                            sh.wgs_f, nbricks);                                 \
         hipLaunchKernelGGL(k, dim3(g), dim3(sh.block_f), lds, s, brick_box, nbricks, a, l, t,  \
                            boxes, start, sp, pl.w, pl.cap_f);                                  \

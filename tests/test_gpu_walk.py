@@ -1,0 +1,60 @@
+"""The list-walk density and force passes against the oracle at the sizes where their lanes per
+atom and table placement change (32, 16, 8 lanes with the global table, 8, 4, 2 with the knots in
+LDS), and on positions whose pairs leave the fast road: atoms a box length or more out, pairs
+closer than the LDS window reaches.  Bars: F' 1e-13, forces 1e-10 eV/A max-abs."""
+import numpy as np
+import pytest
+
+import msmpscu_amd.configs as cfg
+import msmpscu_amd.mdlib as md
+
+pytestmark = pytest.mark.gpu
+
+
+def _case(name):
+    kind, n = name.split("-")
+    c = {"250": (5, 5, 5), "8k": (16, 16, 16), "16k": (20, 21, 19), "39k": (27, 27, 27),
+         "130k": (40, 41, 40), "1k": (6, 6, 7), "41k": (21, 22, 22)}[n]
+    if kind == "cuni":
+        box = cfg.make_cuni_slab(c, 3.57, 900.0, 5)
+        ctrl = cfg.cuni_ctrl()
+        return box, ctrl, cfg.cuni_forcetable(box, ctrl), None
+    box = cfg.make_bcc_box(c, cfg.W_A, 0.05, 300.0, 11, n_vac=2)
+    ctrl = cfg.w_ctrl(mx=64)
+    ft = cfg.w_forcetable(box, ctrl, pot_type="EAM_TYPE" if kind == "eam" else "FS_TYPE")
+    xp = box.XP.copy()
+    if kind == "far":
+        # trial points: one box length out, several, on the far face, and two atoms 0.4 A apart
+        xp[3] += box.ZL * [1.0, 0.0, 0.0]
+        xp[40] -= box.ZL * [0.0, 3.25, 0.5]
+        xp[box.NPRT // 2] = box.BOXLOW + 0.01
+        xp[box.NPRT - 1] = xp[box.NPRT - 2] + [0.4, 0.0, 0.0]
+    return box, ctrl, ft, xp if kind == "far" else None
+
+
+@pytest.mark.parametrize("name", ["fs-250", "eam-8k", "fs-16k", "eam-39k", "fs-130k", "cuni-1k",
+                                  "cuni-41k", "far-250", "far-16k", "far-39k"])
+def test_walk_passes_vs_oracle(orc, name):
+    box, ctrl, ft, trial = _case(name)
+    fc = md.MDForceClassGPU(ForceTable=ft)
+    md.Register_ForceClass(ft.PotType, fc)
+    md.Initialize_Globle_Variables_DEV(box, ctrl, fc)
+    md.Init_Forcetable_Dev(box, ctrl, fc)
+    dev = fc.Device
+    dev.build_neighbors()
+    x = box.XP
+    if trial is not None:
+        dev.put_atoms(trial)
+        x = trial
+    dev.calc_force()
+    it = box.ITYP - 1
+    kv, ind = orc.nlist("full", box.XP, it, box.STATU, box.BOXLOW, box.ZL, ctrl.IFPD, ctrl.NB_RM,
+                        ctrl.NB_MXNBS)
+    fo, do, _ = orc.force_full(np.asfortranarray(x), it, box.STATU, kv, ind, box.ZL, ctrl.IFPD,
+                               float(np.max(ctrl.RU)) ** 2, orc.from_mdlib(ft))
+    df = np.max(np.abs(dev.get_forces() - fo))
+    dd = np.max(np.abs(dev.get_den() - do) / np.maximum(1.0, np.abs(do)))
+    print(f"{name}: n={box.NPRT} {dev.pass_kernel()} max|dF|={df:.3e} max|dF'|={dd:.3e}")
+    dev.close()
+    assert df <= 1e-10
+    assert dd <= 1e-13
