@@ -35,7 +35,7 @@ def _run(cmd, cwd=None):
     return out
 
 
-SOURCES = ("msm_api.hip", "msm_kernels.hip", "msm_bricks.hip", "msm_tpa.hip", "msm_pair.hip",
+SOURCES = ("msm_api.hip", "msm_kernels.hip", "msm_cells.hip", "msm_bricks.hip", "msm_tpa.hip", "msm_pair.hip",
            "msm_ldstab.hip", "msm_walk.hip", "msm_stage.hip", "msm_thermal.hip", "msm_adjoint.hip", "msm_host.cpp")
 
 

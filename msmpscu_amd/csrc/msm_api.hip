@@ -68,6 +68,7 @@ struct msm_sim {
     int ngroup = 0, mx = 0;
     std::vector<double> ru, nb_rm, cm;
     double* d_rnl2 = nullptr;
+    int one_radius = 1;  // one list radius for every pair of types
 
     // boxes
     bool has_boxes = false;
@@ -109,8 +110,9 @@ struct msm_sim {
     // options
     int track_dis = 1;
     int timing = 0;
-    int nlist_kind = 0;    // list build: 0 LDS bricks sized by occupancy, 1 per-atom global
-                           // scan, 2 small LDS bricks, 3 wide LDS bricks
+    int nlist_kind = 0;    // list build: 0 a wave per cell (LDS bricks sized by occupancy where
+                           // the passes read halo slots), 1 per-atom global scan, 2 small LDS
+                           // bricks, 3 wide LDS bricks
     int force_path = 2;    // 0: LDS bricks; 1, 2, 4, 8: global list with that many lanes per atom;
                            // 3: two lanes per atom with lane-pair gathers
     int table_lds = 1;     // table knots in LDS (global-list paths 1, 2, 4; brick path 0)
@@ -345,6 +347,12 @@ int read_flags(msm_sim* s) {
     return MSM_OK;
 }
 
+// Halo slots are written for the brick passes only (a list without them sends those passes to the
+// global list until the next rebuild).
+bool want_sidx(const msm_sim* s) {
+    return s->force_path == 0 || s->force_path == 5 || s->tuning;
+}
+
 // Neighbour-list rebuild on the stream (capturable: kernels only).  Reads the current set and
 // position buffer, writes the other set and buffer, then flips both.
 // keep_f: carry the forces into the new order (not needed inside msm_run, where a force pass
@@ -357,23 +365,25 @@ void enqueue_rebuild(msm_sim* s, bool keep_f = true) {
     AtomsDev a_dst = atoms_view(s, dst, p1);
     a_dst.pos = s->pos[p1];
     const int nc = s->ncell_total;
-    msm::launch_fill_int(s->sb.count, 0, nc + 2, s->stream);
-    msm::launch_cell_assign(a_src.pos, a_src.statu, a_src.boxid, s->d_boxes, s->n, nc, s->sb,
-                            s->d_err, s->stream);
-    msm::launch_scan_exclusive(s->sb.count, s->sb.start, nc + 2, s->sb.scan_tmp, s->stream);
-    msm::launch_scatter_sort(s->n, nc, s->sb, s->set[src].gid, s->stream);
-    msm::launch_gather(s->n, s->n_alloc, s->sb.perm, a_src, s->set[src].gid, a_dst,
-                       s->set[dst].gid, s->sb.key, s->set[dst].cell, keep_f ? 1 : 0, s->stream);
+    msm::launch_cell_sort(s->n, nc, s->d_boxes, a_src, s->set[src].gid, a_dst, s->set[dst].gid,
+                          s->set[dst].cell, s->sb, keep_f ? 1 : 0, s->d_err, s->stream);
     TimedScope tl(s, MSM_KCLASS_NLIST);
     if (s->nlist_kind == 1) {
         s->list_sidx = 0;
         msm::launch_nlist(s->n, s->pos[p1], s->set[dst].ityp, s->set[dst].statu,
                           s->set[dst].boxid, s->set[dst].cell, s->sb.start, s->d_boxes, s->ngroup,
                           s->d_rnl2, s->mx, s->kvois, s->indi, msm::kListRow, s->d_err, s->stream);
+    } else if (s->nlist_kind == 0 && !want_sidx(s)) {
+        s->list_sidx = 0;
+        size_t big = 0;
+        for (size_t b = 0; b < s->boxes.size(); ++b)
+            if (s->boxes[b].natoms > s->boxes[big].natoms) big = b;
+        msm::launch_nlist_cell(nc, s->n, s->occ[big], s->one_radius, s->pos[p1],
+                               s->set[dst].ityp, s->set[dst].boxid, s->sb.start, s->d_boxes,
+                               s->ngroup, s->d_rnl2, s->mx, s->kvois, s->indi, s->d_err,
+                               s->stream);
     } else {
-        // halo slots only for the brick passes (a list without them sends those passes to
-        // the global list until the next rebuild)
-        s->list_sidx = s->force_path == 0 || s->force_path == 5 || s->tuning;
+        s->list_sidx = want_sidx(s);
         msm::launch_nlist_bricks(s->nl_wide, s->nbricks, s->nl_lanes, s->nl_cap, s->list_sidx,
                                  s->d_brick_box, s->n, nc,
                                  s->pos[p1],
@@ -869,7 +879,7 @@ int msm_destroy(msm_sim* s) {
     dfree(&s->sb.slot);
     dfree(&s->sb.count);
     dfree(&s->sb.start);
-    dfree(&s->sb.perm);
+    dfree(&s->sb.arr);
     dfree(&s->sb.scan_tmp);
     dfree(&s->kvois);
     dfree(&s->indi);
@@ -1035,6 +1045,7 @@ int msm_set_ctrl(msm_sim* s, int ngroup, const double* ru, const double* nb_rm, 
         s->tab.cm[g] = cm[g];
     }
     s->tab.ru2max = ru2max;
+    s->one_radius = std::all_of(rnl2.begin(), rnl2.end(), [&](double v) { return v == rnl2[0]; });
     int rc = dalloc(s, &s->d_rnl2, rnl2.size());
     if (rc != MSM_OK) return rc;
     HIPCHK(s, hipMemcpy(s->d_rnl2, rnl2.data(), rnl2.size() * sizeof(double), hipMemcpyHostToDevice));
@@ -1091,6 +1102,8 @@ int msm_set_boxes(msm_sim* s, int nbox, const int* natoms, const double* lo, con
         if (rc == MSM_OK) rc = dalloc(s, &s->sb.scan_tmp, need / 1024 + 2);
         if (rc != MSM_OK) return rc;
         s->sort_cap = need;
+        // every rebuild leaves the counts at zero
+        HIPCHK(s, hipMemset(s->sb.count, 0, need * sizeof(int)));
     }
     s->half_min = HUGE_VAL;
     for (const BoxDev& b : s->boxes)
@@ -1135,7 +1148,7 @@ int msm_set_atoms(msm_sim* s, int n, const double* xp, const double* xp1, const 
     if (rc == MSM_OK) rc = dalloc(s, &s->epot, na);
     if (rc == MSM_OK) rc = dalloc(s, &s->sb.key, na);
     if (rc == MSM_OK) rc = dalloc(s, &s->sb.slot, na);
-    if (rc == MSM_OK) rc = dalloc(s, &s->sb.perm, na);
+    if (rc == MSM_OK) rc = dalloc(s, &s->sb.arr, na);
     if (rc == MSM_OK) rc = dalloc(s, &s->kvois, na);
     const size_t icap = static_cast<size_t>(na) * s->mx;
     if (rc == MSM_OK) rc = dalloc(s, &s->indi, icap);
@@ -2265,8 +2278,9 @@ int msm_autotune(msm_sim* s, int reps, int* choice, double* best_ms) {
     // list-build kernel (a rebuild of unchanged positions reproduces the same order and list)
     float best_nl = 0.f;
     int nl_choice = s->nlist_kind;
-    for (int g : {2, 3, 1}) {
+    for (int g : {2, 3, 1, 0}) {
         s->nlist_kind = g;
+        s->tuning = g != 0;  // 0: the wave-per-cell list, which writes no halo slots
         if ((rc = replan_bricks(s)) != MSM_OK) break;
         float ms = 0.f;
         rc = time_it([&] { enqueue_rebuild(s); }, ms);
@@ -2277,6 +2291,7 @@ int msm_autotune(msm_sim* s, int reps, int* choice, double* best_ms) {
         }
     }
     s->nlist_kind = nl_choice;
+    s->tuning = 1;
     if (rc == MSM_OK) rc = replan_bricks(s);
     if (rc == MSM_OK) enqueue_rebuild(s);
     // staged-brick passes (slot list of the brick list kernels; their workgroup shape is fixed,

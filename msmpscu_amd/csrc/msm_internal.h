@@ -107,20 +107,24 @@ struct SortBufs {
     int* slot;   // arrival slot within the cell
     int* count;  // ncell_total + 2
     int* start;  // ncell_total + 2 (exclusive scan of count)
-    int* perm;   // sorted position -> current index
+    int2* arr;   // arrival position of the counting sort -> {current index, caller index}
     int* scan_tmp;
 };
 
 // ---- launchers (msm_kernels.hip) ----
 void launch_fill_int(int* p, int v, int n, hipStream_t s);
-void launch_cell_assign(const double4* pos, const int* statu, const int* boxid,
-                        const BoxDev* boxes, int n, int ncell_total, SortBufs sb, int* err,
-                        hipStream_t s);
-void launch_scan_exclusive(const int* in, int* out, int n, int* tmp, hipStream_t s);
-void launch_scatter_sort(int n, int ncell_total, SortBufs sb, const int* gid, hipStream_t s);
-void launch_gather(int n, int n_alloc, const int* perm, const AtomsDev& src, const int* gid_src,
-                   AtomsDev& dst, int* gid_dst, const int* key, int* cell_dst, int keep_f,
-                   hipStream_t s);
+// Cell sort (msm_cells.hip): src in its current order -> dst in cell order; sb.count must hold zeros
+// (it does again afterwards).  Boxes within both limits sort in one workgroup.
+constexpr int kSortSmallAtoms = 8192, kSortSmallCells = 12288;
+void launch_cell_sort(int n, int ncell_total, const BoxDev* boxes, const AtomsDev& src,
+                      const int* gid_src, AtomsDev& dst, int* gid_dst, int* cell_dst, SortBufs sb,
+                      int keep_f, int* err, hipStream_t s);
+// List with one wave per cell (msm_cells.hip); mean: atoms per non-empty cell; one_radius: rnl2
+// holds one value for every pair of types.
+void launch_nlist_cell(int ncell_total, int n, double mean, int one_radius, const double4* pos,
+                       const int* ityp, const int* boxid, const int* start, const BoxDev* boxes,
+                       int ngroup, const double* rnl2, int mx, int* kvois, int* indi, int* err,
+                       hipStream_t s);
 void launch_nlist(int n, const double4* pos, const int* ityp, const int* statu, const int* boxid,
                   const int* cell, const int* start, const BoxDev* boxes, int ngroup,
                   const double* rnl2, int mx, int* kvois, int* indi, int stride, int* err,

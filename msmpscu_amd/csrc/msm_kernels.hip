@@ -38,220 +38,8 @@ void launch_fill_int(int* p, int v, int n, hipStream_t s) {
 }
 
 // --------------------------------------------------------------------------------------------
-// neighbour-list build: cell ids, counting sort, deterministic in-cell order, gather, list
+// neighbour list: per-atom scan (the sort and the default list are in msm_cells.hip)
 // --------------------------------------------------------------------------------------------
-
-__global__ void k_cell_assign(const double4* __restrict__ pos, const int* __restrict__ statu,
-                              const int* __restrict__ boxid, const BoxDev* __restrict__ boxes,
-                              int n, int ncell_total, int* __restrict__ key,
-                              int* __restrict__ slot, int* __restrict__ count, int* err) {
-#pragma clang fp contract(off)
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    int c = ncell_total;  // sentinel bucket: atoms outside every cell grid
-    if ((statu[i] & STATU_OUTOFBOX) != STATU_OUTOFBOX) {
-        const BoxDev& b = boxes[boxid[i]];
-        const double4 p = pos[i];
-        const double xyz[3] = {p.x, p.y, p.z};
-        int ic[3];
-        bool in = true;
-        for (int k = 0; k < 3; ++k) {
-            // (x - LB)/L * NC - eps, truncated toward zero, as MD_NeighborsList.F90:258
-            const double s = (xyz[k] - b.lo[k]) / b.len[k] * static_cast<double>(b.ncell[k]) - 1.0e-4;
-            ic[k] = static_cast<int>(s);
-            in = in && ic[k] >= 0 && ic[k] < b.ncell[k];
-        }
-        if (in)
-            c = b.cell_off + cell_local(b, ic[0], ic[1], ic[2]);
-        else
-            atomicOr(&err[kErrOutOfBox], 1);
-    }
-    key[i] = c;
-    // one atomic per distinct cell of the wave (after the first build the atoms are cell-sorted,
-    // so a wave spans a few cells): the lanes of each cell are grouped by ballots first, then
-    // the leader of every cell adds the cell's lane count, all leaders in one atomic
-    // instruction (one round trip per wave), and every lane takes base + its rank among its
-    // cell's lanes.  Slot order inside a cell is made deterministic afterwards by k_cell_order.
-    const int lane = threadIdx.x & 63;
-    unsigned long long todo = __ballot(1);
-    int lead = lane, rank = 0, cnt = 0;
-    while (todo) {
-        const int leader = __ffsll(static_cast<long long>(todo)) - 1;
-        const int lc = __shfl(c, leader, 64);
-        const unsigned long long same = __ballot(c == lc) & todo;
-        if (c == lc) {
-            lead = leader;
-            rank = __popcll(same & ((1ull << lane) - 1ull));
-            if (lane == leader) cnt = __popcll(same);
-        }
-        todo &= ~same;
-    }
-    int base = 0;
-    if (cnt > 0) base = atomicAdd(&count[c], cnt);
-    slot[i] = __shfl(base, lead, 64) + rank;
-}
-
-void launch_cell_assign(const double4* pos, const int* statu, const int* boxid,
-                        const BoxDev* boxes, int n, int ncell_total, SortBufs sb, int* err,
-                        hipStream_t s) {
-    if (n <= 0) return;
-    hipLaunchKernelGGL(k_cell_assign, dim3(grid_for(n)), dim3(kBlock), 0, s, pos, statu, boxid,
-                       boxes, n, ncell_total, sb.key, sb.slot, sb.count, err);
-}
-
-// Exclusive scan of int: block-level inclusive scans (wave64 shuffles + LDS), one-block scan of
-// the block totals, then a fix-up pass.
-constexpr int kScanBlock = 1024;
-
-__global__ void k_scan_blocks(const int* __restrict__ in, int* __restrict__ out,
-                              int* __restrict__ sums, int n) {
-    __shared__ int lds[kScanBlock / 64];
-    const int i = blockIdx.x * kScanBlock + threadIdx.x;
-    const int v = (i < n) ? in[i] : 0;
-    const int inc = block_incl_scan(v, lds);
-    if (i < n) out[i] = inc - v;  // exclusive within the block
-    if (threadIdx.x == kScanBlock - 1) sums[blockIdx.x] = inc;
-}
-
-__global__ void k_scan_sums(int* sums, int nb) {
-    __shared__ int lds[kScanBlock / 64];
-    __shared__ int carry;
-    if (threadIdx.x == 0) carry = 0;
-    __syncthreads();
-    for (int base = 0; base < nb; base += kScanBlock) {
-        const int i = base + threadIdx.x;
-        const int v = (i < nb) ? sums[i] : 0;
-        const int inc = block_incl_scan(v, lds);
-        const int c = carry;
-        if (i < nb) sums[i] = c + inc - v;
-        __syncthreads();
-        if (threadIdx.x == kScanBlock - 1) carry = c + inc;
-        __syncthreads();
-    }
-}
-
-__global__ void k_scan_add(int* out, const int* __restrict__ sums, int n) {
-    const int i = blockIdx.x * kScanBlock + threadIdx.x;
-    if (i < n) out[i] += sums[blockIdx.x];
-}
-
-void launch_scan_exclusive(const int* in, int* out, int n, int* tmp, hipStream_t s) {
-    if (n <= 0) return;
-    const int nb = (n + kScanBlock - 1) / kScanBlock;
-    hipLaunchKernelGGL(k_scan_blocks, dim3(nb), dim3(kScanBlock), 0, s, in, out, tmp, n);
-    hipLaunchKernelGGL(k_scan_sums, dim3(1), dim3(kScanBlock), 0, s, tmp, nb);
-    hipLaunchKernelGGL(k_scan_add, dim3(nb), dim3(kScanBlock), 0, s, out, tmp, n);
-}
-
-__global__ void k_scatter(int n, const int* __restrict__ key, const int* __restrict__ slot,
-                          const int* __restrict__ start, int* __restrict__ perm) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) perm[start[key[i]] + slot[i]] = i;
-}
-
-// One thread per cell: order the cell's atoms by caller index, which makes the sorted order,
-// the list order and every summation order independent of atomic arrival order.  A cell of at
-// most kCellSortReg atoms is loaded in two independent rounds (entries, then their caller
-// indices) and sorted in registers by an odd-even transposition network; a larger cell takes an
-// insertion sort in memory.
-constexpr int kCellSortReg = 16;
-
-__global__ void k_cell_order(int ncells, const int* __restrict__ start, int* __restrict__ perm,
-                             const int* __restrict__ gid) {
-    const int c = blockIdx.x * blockDim.x + threadIdx.x;
-    if (c >= ncells) return;
-    const int b = start[c], e = start[c + 1];
-    const int n = e - b;
-    if (n <= 1) return;
-    if (n <= kCellSortReg) {
-        int v[kCellSortReg], g[kCellSortReg];
-#pragma unroll
-        for (int k = 0; k < kCellSortReg; ++k) v[k] = k < n ? perm[b + k] : 0;
-#pragma unroll
-        for (int k = 0; k < kCellSortReg; ++k) g[k] = k < n ? gid[v[k]] : INT_MAX;
-        auto cswap = [&](int k) {
-            const bool sw = g[k] > g[k + 1];
-            const int g0 = sw ? g[k + 1] : g[k], g1 = sw ? g[k] : g[k + 1];
-            const int v0 = sw ? v[k + 1] : v[k], v1 = sw ? v[k] : v[k + 1];
-            g[k] = g0;
-            g[k + 1] = g1;
-            v[k] = v0;
-            v[k + 1] = v1;
-        };
-#pragma unroll
-        for (int r = 0; r < kCellSortReg / 2; ++r) {  // even phase, then odd phase
-#pragma unroll
-            for (int k = 0; k + 1 < kCellSortReg; k += 2) cswap(k);
-#pragma unroll
-            for (int k = 1; k + 1 < kCellSortReg; k += 2) cswap(k);
-        }
-#pragma unroll
-        for (int k = 0; k < kCellSortReg; ++k)
-            if (k < n) perm[b + k] = v[k];
-        return;
-    }
-    for (int a = b + 1; a < e; ++a) {
-        const int v = perm[a];
-        const int g = gid[v];
-        int q = a - 1;
-        while (q >= b && gid[perm[q]] > g) {
-            perm[q + 1] = perm[q];
-            --q;
-        }
-        perm[q + 1] = v;
-    }
-}
-
-void launch_scatter_sort(int n, int ncell_total, SortBufs sb, const int* gid, hipStream_t s) {
-    if (n <= 0) return;
-    hipLaunchKernelGGL(k_scatter, dim3(grid_for(n)), dim3(kBlock), 0, s, n, sb.key, sb.slot,
-                       sb.start, sb.perm);
-    const int nc = ncell_total + 1;
-    hipLaunchKernelGGL(k_cell_order, dim3(grid_for(nc)), dim3(kBlock), 0, s, nc, sb.start,
-                       sb.perm, gid);
-}
-
-// F = 0: forces are not carried (a force pass overwrites them before they are read).
-template <int F>
-__global__ void k_gather(int n, const int* __restrict__ perm, AtomsDev src,
-                         const int* __restrict__ gid_src, AtomsDev dst, int* __restrict__ gid_dst,
-                         const int* __restrict__ key, int* __restrict__ cell_dst) {
-    const int p = blockIdx.x * blockDim.x + threadIdx.x;
-    if (p >= n) return;
-    const int i = perm[p];
-    double4 x = src.pos[i];
-    x.w = 0.0;
-    dst.pos[p] = x;
-    dst.vx[p] = src.vx[i];
-    dst.vy[p] = src.vy[i];
-    dst.vz[p] = src.vz[i];
-    if constexpr (F) {
-        dst.fx[p] = src.fx[i];
-        dst.fy[p] = src.fy[i];
-        dst.fz[p] = src.fz[i];
-    }
-    dst.dx[p] = src.dx[i];
-    dst.dy[p] = src.dy[i];
-    dst.dz[p] = src.dz[i];
-    dst.ityp[p] = src.ityp[i];
-    dst.statu[p] = src.statu[i];
-    dst.boxid[p] = src.boxid[i];
-    gid_dst[p] = gid_src[i];
-    cell_dst[p] = key[i];
-}
-
-void launch_gather(int n, int n_alloc, const int* perm, const AtomsDev& src, const int* gid_src,
-                   AtomsDev& dst, int* gid_dst, const int* key, int* cell_dst, int keep_f,
-                   hipStream_t s) {
-    (void)n_alloc;
-    if (n <= 0) return;
-    if (keep_f)
-        hipLaunchKernelGGL(k_gather<1>, dim3(grid_for(n)), dim3(kBlock), 0, s, n, perm, src,
-                           gid_src, dst, gid_dst, key, cell_dst);
-    else
-        hipLaunchKernelGGL(k_gather<0>, dim3(grid_for(n)), dim3(kBlock), 0, s, n, perm, src,
-                           gid_src, dst, gid_dst, key, cell_dst);
-}
 
 __global__ __launch_bounds__(kBlock) void k_nlist(
     int n, const double4* __restrict__ pos, const int* __restrict__ ityp,
