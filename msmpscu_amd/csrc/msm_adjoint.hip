@@ -473,7 +473,7 @@ struct SplineTab {
 // One thread per padded knot a: the device table entries msm_set_force_table builds on the host,
 // (T(a), T(a+1) - T(a)) pairs, from the spline tables.
 __global__ void k_spline_tables(SplineTab st, double* __restrict__ b1, double2* __restrict__ f2,
-                                double2* __restrict__ b2, double4* __restrict__ f4,
+                                double2* __restrict__ e2, double2* __restrict__ b2, double4* __restrict__ f4,
                                 double4* __restrict__ e4, double4* __restrict__ m4) {
 #pragma clang fp contract(off)
     const int a = blockIdx.x * blockDim.x + threadIdx.x;
@@ -484,6 +484,7 @@ __global__ void k_spline_tables(SplineTab st, double* __restrict__ b1, double2* 
         const double pr = st.potr(a), pr1 = st.potr(a + 1);
         b1[a] = pb;
         f2[a] = make_double2(fr, fb);
+        e2[a] = make_double2(pr, pb);
         b2[a] = make_double2(pb, pb1 - pb);
         f4[a] = make_double4(fr, fr1 - fr, fb, fb1 - fb);
         e4[a] = make_double4(pr, pr1 - pr, pb, pb1 - pb);
@@ -612,13 +613,13 @@ __global__ void k_spline_grad(SplineTab st, const double* __restrict__ pairs,
 }  // namespace
 
 void launch_spline_tables(const double* coef, int ld, const TabDev& t, double* b1, double2* f2,
-                          double2* b2, double4* f4,
+                          double2* e2, double2* b2, double4* f4,
                           double4* e4, double4* m4, hipStream_t s) {
     SplineTab st{coef, coef + ld, coef + 2 * static_cast<size_t>(ld), t.ntab2 - 2,
                  t.pot_type != 0 ? t.nembd : 0, t.csi, t.csi * t.csi, t.rhod};
     const int m = std::max(t.ntab2, t.pot_type != 0 ? t.nembd2 : 0);
-    hipLaunchKernelGGL(k_spline_tables, dim3((m + 255) / 256), dim3(256), 0, s, st, b1, f2, b2, f4,
-                       e4, t.pot_type != 0 ? m4 : nullptr);
+    hipLaunchKernelGGL(k_spline_tables, dim3((m + 255) / 256), dim3(256), 0, s, st, b1, f2, e2, b2,
+                       f4, e4, t.pot_type != 0 ? m4 : nullptr);
 }
 
 int fm_parts(int n) { return std::max(1, std::min(512, (n + kAdjBlock - 1) / kAdjBlock)); }

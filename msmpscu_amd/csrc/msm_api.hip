@@ -58,9 +58,9 @@ struct msm_sim {
     bool has_table = false;
     TabDev tab{};
     double* d_b1 = nullptr;
-    double2 *d_b2 = nullptr, *d_f2 = nullptr;
+    double2 *d_b2 = nullptr, *d_f2 = nullptr, *d_e2 = nullptr;
     double4 *d_f4 = nullptr, *d_e4 = nullptr, *d_m4 = nullptr;
-    size_t cap_b1 = 0, cap_f2 = 0, cap_b2 = 0, cap_f4 = 0, cap_e4 = 0, cap_m4 = 0;  // elements allocated
+    size_t cap_b1 = 0, cap_f2 = 0, cap_e2 = 0, cap_b2 = 0, cap_f4 = 0, cap_e4 = 0, cap_m4 = 0;  // elements allocated
     int tab_ngroup = 0;
 
     // control
@@ -100,8 +100,13 @@ struct msm_sim {
 
     // flags and scratch
     int* d_err = nullptr;
-    int* h_err = nullptr;
+    int* h_err = nullptr;      // pinned: the error flags, then one double (h_word)
+    double* h_word = nullptr;
+    double* qwork = nullptr;   // per-atom scratch (quench energies)
     double* d_ebox = nullptr;
+    int nchunk = 0;               // chunks of the box sums, their boxes and partial sums (6 arrays)
+    int* d_chunk_box = nullptr;
+    double* d_part = nullptr;
     unsigned long long* d_stats = nullptr;
     double* d_boxwork = nullptr;  // per-box scratch (4 doubles a box)
     size_t boxwork_cap = 0;
@@ -231,6 +236,7 @@ void free_atoms(msm_sim* s) {
         dfree(&s->set[k].cell);
     }
     dfree(&s->epot);
+    dfree(&s->qwork);
     s->n = s->n_alloc = 0;
     s->has_atoms = false;
     s->has_list = false;
@@ -613,15 +619,8 @@ int auto_lanes(const msm_sim* s) {
     return lanes;
 }
 
-// The list-walk pass (msm_walk.hip) and its shape; false: another kernel runs.
-bool walk_plan(const msm_sim* s, int force, msm::WalkPlan& p) {
-    if (s->n >= msm::kWalkMaxAtoms || s->compact) return false;
-    const int fp = eff_path(s);
-    if (fp != 1 && fp != 2 && fp != 4) return false;
-    p.block = force ? s->lt.block_f : s->lt.block_d;
-    p.wgs = force ? s->lt.wgs_f : s->lt.wgs_d;
-    p.sweep = s->lt.sweep;
-    // inner units skip the minimum image; worth it when half a box is well beyond the list radius
+// Inner units skip the minimum image: worth it when half a box is well beyond the list radius.
+void walk_geometry(const msm_sim* s, msm::WalkPlan& p) {
     double rnl = 0.0;
     for (double r : s->nb_rm) rnl = std::max(rnl, r);
     p.margin = rnl;
@@ -630,22 +629,70 @@ bool walk_plan(const msm_sim* s, int force, msm::WalkPlan& p) {
         const double k = std::floor(std::sqrt(s->half_min * (1.0 - 1.0e-9)) * s->tab.csi);
         p.kimg = k < 1.0e9 ? static_cast<int>(k) : 1000000000;
     }
-    if (!s->auto_pass) {
-        p.tl = 1;
-        p.lanes = force ? lt_force_lanes(s) : fp;
-        return s->table_lds && walk_lds_ok(s);
-    }
+}
+
+// Lanes and table placement by size.  Filling the LDS window costs more than the global lookups it
+// saves below about 10^6 pairs: 16,000 W atoms at 8 lanes 25.6 us with it, 23.3 without; 54,000 at
+// 4 lanes 31.0, at 8 lanes from global memory 38.7; 42,600 Cu-Ni atoms at 8 lanes 93.8 with it,
+// 108.4 without.  false: a table too large for the LDS on a large box (the general passes).
+bool size_plan(const msm_sim* s, int force, msm::WalkPlan& p) {
     p.lanes = auto_lanes(s);
-    // filling the LDS window costs more than the global lookups it saves below about 10^6 pairs:
-    // 16,000 W atoms at 8 lanes 25.6 us with it, 23.3 without; 54,000 at 4 lanes 31.0, at 8 lanes
-    // from global memory 38.7; 42,600 Cu-Ni atoms at 8 lanes 93.8 with it, 108.4 without
     p.tl = p.lanes <= 8 && s->n * s->kmean >= 8.0e5 && msm::walk_window_ok(s->tab, force, p.wgs);
     if (!p.tl) {
-        // a table too large for the LDS on a large box: the two-lane global-table pass
         if (s->n * s->kmean >= 8.0e6) return false;
         p.lanes = std::max(p.lanes, 8);
     }
     return true;
+}
+
+// The list-walk pass (msm_walk.hip) and its shape; false: another kernel runs.
+bool walk_plan(const msm_sim* s, int force, msm::WalkPlan& p) {
+    if (s->n >= msm::kWalkMaxAtoms || s->compact) return false;
+    const int fp = eff_path(s);
+    if (fp != 1 && fp != 2 && fp != 4) return false;
+    walk_geometry(s, p);
+    p.block = force ? s->lt.block_f : s->lt.block_d;
+    p.wgs = force ? s->lt.wgs_f : s->lt.wgs_d;
+    p.sweep = s->lt.sweep;
+    if (s->auto_pass) return size_plan(s, force, p);
+    p.tl = 1;
+    p.lanes = force ? lt_force_lanes(s) : fp;
+    return s->table_lds && walk_lds_ok(s);
+}
+
+void enqueue_density(msm_sim* s);
+
+// The list walk of the energy and virial passes, which no option fixes; false: the general passes.
+bool aux_plan(const msm_sim* s, msm::WalkPlan& p) {
+    if (s->n >= msm::kWalkMaxAtoms) return false;
+    walk_geometry(s, p);
+    p.block = 1024;
+    p.wgs = 1;
+    p.sweep = 0;
+    return size_plan(s, 1, p);
+}
+
+// Per-atom energies; rho_out (may be null) also the densities, write_fp: F' in pos.w as the density
+// pass leaves it.
+void enqueue_epot(msm_sim* s, double* rho_out = nullptr, int write_fp = 0) {
+    AtomsDev a = atoms_view(s, s->scur, s->pcur);
+    msm::WalkPlan wp{};
+    // (a compacted force pass reads what the density pass records beside F')
+    if (!(write_fp && s->compact) && aux_plan(s, wp)) {
+        msm::launch_energy_walk(wp, a, list_view(s), s->tab, s->boxes[0], s->d_boxes,
+                                multibox(s), rho_out, write_fp, s->d_err, s->stream);
+        return;
+    }
+    if (write_fp) enqueue_density(s);
+    msm::launch_epot(a, list_view(s), s->tab, s->boxes[0], s->d_boxes, multibox(s), s->d_err,
+                     s->stream, rho_out);
+}
+
+// Box totals of ncomp per-atom arrays (stride n_stride) into out[c * nbox + box].
+void enqueue_box_sums(msm_sim* s, const double* v, size_t n_stride, int ncomp, double* out) {
+    msm::launch_box_sums(v, n_stride, ncomp, s->sb.start, s->d_boxes,
+                         static_cast<int>(s->boxes.size()), s->d_chunk_box, s->nchunk, s->d_part,
+                         out, s->stream);
 }
 
 void enqueue_density(msm_sim* s) {
@@ -840,8 +887,9 @@ int msm_create(msm_sim** out, int device) {
     int rc = dalloc(s, &s->d_err, msm::kErrSlots);
     if (rc == MSM_OK) rc = dalloc(s, &s->d_stats, 2);
     if (rc == MSM_OK && hipHostMalloc(reinterpret_cast<void**>(&s->h_err),
-                                      sizeof(int) * msm::kErrSlots) != hipSuccess)
+                                      sizeof(int) * msm::kErrSlots + sizeof(double)) != hipSuccess)
         rc = MSM_ERR_NOMEM;
+    if (rc == MSM_OK) s->h_word = reinterpret_cast<double*>(s->h_err + msm::kErrSlots);
     if (rc != MSM_OK) {
         msm_destroy(s);
         return rc;
@@ -868,6 +916,7 @@ int msm_destroy(msm_sim* s) {
     if (s->fm_ev) (void)hipEventDestroy(s->fm_ev);
     dfree(&s->d_b1);
     dfree(&s->d_f2);
+    dfree(&s->d_e2);
     dfree(&s->d_b2);
     dfree(&s->d_f4);
     dfree(&s->d_e4);
@@ -889,6 +938,8 @@ int msm_destroy(msm_sim* s) {
     dfree(&s->cmask);
     dfree(&s->d_err);
     dfree(&s->d_ebox);
+    dfree(&s->d_chunk_box);
+    dfree(&s->d_part);
     dfree(&s->d_stats);
     dfree(&s->d_boxwork);
     if (s->h_err) (void)hipHostFree(s->h_err);
@@ -930,7 +981,7 @@ int msm_set_force_table(msm_sim* s, int pot_type, int ngroup, int nkind, int nta
     std::vector<double2> hb2(static_cast<size_t>(nkind) * ntab2);
     std::vector<double4> hf4(static_cast<size_t>(nkind) * ntab2), he4(hf4.size());
     std::vector<double> hb1(hb2.size());
-    std::vector<double2> hf2(hb2.size());
+    std::vector<double2> hf2(hb2.size()), hen2(hb2.size());
     for (int k = 0; k < nkind; ++k)
         for (int i = 0; i < ntab2; ++i) {
             const size_t a = static_cast<size_t>(k) * ntab2 + i;
@@ -943,6 +994,7 @@ int msm_set_force_table(msm_sim* s, int pot_type, int ngroup, int nkind, int nta
             he4[a] = make_double4(pr, pr1 - pr, pb, pb1 - pb);
             hb1[a] = pb;
             hf2[a] = make_double2(fr, fb);
+            hen2[a] = make_double2(pr, pb);
         }
     TabDev t;
     std::memset(&t, 0, sizeof(t));  // byte-wise comparable with the current table
@@ -966,9 +1018,11 @@ int msm_set_force_table(msm_sim* s, int pot_type, int ngroup, int nkind, int nta
     if (rc == MSM_OK) rc = dreserve(s, &s->d_e4, he4.size(), s->cap_e4);
     if (rc == MSM_OK) rc = dreserve(s, &s->d_b1, hb1.size(), s->cap_b1);
     if (rc == MSM_OK) rc = dreserve(s, &s->d_f2, hf2.size(), s->cap_f2);
+    if (rc == MSM_OK) rc = dreserve(s, &s->d_e2, hen2.size(), s->cap_e2);
     if (rc != MSM_OK) return rc;
     HIPCHK(s, hipMemcpy(s->d_b1, hb1.data(), hb1.size() * sizeof(double), hipMemcpyHostToDevice));
     HIPCHK(s, hipMemcpy(s->d_f2, hf2.data(), hf2.size() * sizeof(double2), hipMemcpyHostToDevice));
+    HIPCHK(s, hipMemcpy(s->d_e2, hen2.data(), hen2.size() * sizeof(double2), hipMemcpyHostToDevice));
     HIPCHK(s, hipMemcpy(s->d_b2, hb2.data(), hb2.size() * sizeof(double2), hipMemcpyHostToDevice));
     HIPCHK(s, hipMemcpy(s->d_f4, hf4.data(), hf4.size() * sizeof(double4), hipMemcpyHostToDevice));
     HIPCHK(s, hipMemcpy(s->d_e4, he4.data(), he4.size() * sizeof(double4), hipMemcpyHostToDevice));
@@ -1002,6 +1056,7 @@ int msm_set_force_table(msm_sim* s, int pot_type, int ngroup, int nkind, int nta
     }
     t.b1 = s->d_b1;
     t.f2 = s->d_f2;
+    t.e2 = s->d_e2;
     t.b2 = s->d_b2;
     t.f4 = s->d_f4;
     t.e4 = s->d_e4;
@@ -1065,6 +1120,7 @@ int msm_set_boxes(msm_sim* s, int nbox, const int* natoms, const double* lo, con
     double rmax = 0.0;
     for (double r : s->nb_rm) rmax = std::max(rmax, r);
     std::vector<BoxDev> bx(nbox);
+    std::vector<int> chunk_box;
     long long cells = 0;
     for (int b = 0; b < nbox; ++b) {
         BoxDev& d = bx[b];
@@ -1085,6 +1141,8 @@ int msm_set_boxes(msm_sim* s, int nbox, const int* natoms, const double* lo, con
             d.ncell[k] = c;
             nc *= c;
         }
+        d.chunk_off = static_cast<int>(chunk_box.size());
+        for (int a = 0; a == 0 || a < d.natoms; a += msm::kSumChunk) chunk_box.push_back(b);
         d.cbs = s->cell_brick;
         d.cell_off = static_cast<int>(cells);
         cells += nc;
@@ -1110,7 +1168,12 @@ int msm_set_boxes(msm_sim* s, int nbox, const int* natoms, const double* lo, con
         for (int k = 0; k < 3; ++k)
             if (b.ifpd[k]) s->half_min = std::min(s->half_min, 0.5 * b.len[k]);
     rc = dalloc(s, &s->d_ebox, nbox);
+    if (rc == MSM_OK) rc = dalloc(s, &s->d_chunk_box, chunk_box.size());
+    if (rc == MSM_OK) rc = dalloc(s, &s->d_part, 6 * chunk_box.size());
     if (rc != MSM_OK) return rc;
+    s->nchunk = static_cast<int>(chunk_box.size());
+    HIPCHK(s, hipMemcpy(s->d_chunk_box, chunk_box.data(), chunk_box.size() * sizeof(int),
+                        hipMemcpyHostToDevice));
     s->has_boxes = true;
     s->has_atoms = false;
     s->has_list = false;
@@ -1146,6 +1209,7 @@ int msm_set_atoms(msm_sim* s, int n, const double* xp, const double* xp1, const 
         if (rc == MSM_OK) rc = dalloc(s, &s->set[k].cell, na);
     }
     if (rc == MSM_OK) rc = dalloc(s, &s->epot, na);
+    if (rc == MSM_OK) rc = dalloc(s, &s->qwork, na);
     if (rc == MSM_OK) rc = dalloc(s, &s->sb.key, na);
     if (rc == MSM_OK) rc = dalloc(s, &s->sb.slot, na);
     if (rc == MSM_OK) rc = dalloc(s, &s->sb.arr, na);
@@ -1342,8 +1406,7 @@ int msm_add_epot(msm_sim* s, const double* eext, int on_device) {
     int rc = add_caller_order(s, eext, on_device, dst, 1, "msm_add_epot");
     if (rc != MSM_OK || s->n == 0 || !s->has_list) return rc;
     // keep the box totals of msm_get_box_epot in step with the per-atom energies
-    msm::launch_box_sum(s->epot, s->sb.start, s->d_boxes, static_cast<int>(s->boxes.size()),
-                        s->d_ebox, s->stream);
+    enqueue_box_sums(s, s->epot, 0, 1, s->d_ebox);
     HIPCHK(s, hipStreamSynchronize(s->stream));
     return MSM_OK;
 }
@@ -1388,8 +1451,7 @@ int msm_get_box_epot(msm_sim* s, double* ebox) {
     if (!s || !ebox) return MSM_ERR_ARG;
     (void)hipSetDevice(s->device);
     if (!s->has_list) return set_err(s, MSM_ERR_STATE, "no neighbour list");
-    msm::launch_box_sum(s->epot, s->sb.start, s->d_boxes, static_cast<int>(s->boxes.size()),
-                        s->d_ebox, s->stream);
+    enqueue_box_sums(s, s->epot, 0, 1, s->d_ebox);
     HIPCHK(s, hipMemcpyAsync(ebox, s->d_ebox, s->boxes.size() * sizeof(double),
                              hipMemcpyDeviceToHost, s->stream));
     HIPCHK(s, hipStreamSynchronize(s->stream));
@@ -1457,9 +1519,7 @@ int msm_calc_epot(msm_sim* s) {
     if (rc != MSM_OK) return rc;
     (void)hipSetDevice(s->device);
     clear_flags(s);
-    AtomsDev a = atoms_view(s, s->scur, s->pcur);
-    msm::launch_epot(a, list_view(s), s->tab, s->boxes[0], s->d_boxes, multibox(s), s->d_err,
-                     s->stream);
+    enqueue_epot(s);
     return read_flags(s);
 }
 
@@ -1482,9 +1542,7 @@ int msm_calc_ptensor(msm_sim* s, double* vtensor) {
     AtomsDev a = atoms_view(s, s->scur, s->pcur);
     msm::launch_virial(a, list_view(s), s->tab, s->boxes[0], s->d_boxes, multibox(s), vir,
                        s->stream);
-    for (int c = 0; c < 6; ++c)
-        msm::launch_box_sum(vir + static_cast<size_t>(c) * s->n, s->sb.start, s->d_boxes, nbox,
-                            sums + static_cast<size_t>(c) * nbox, s->stream);
+    enqueue_box_sums(s, vir, s->n, 6, sums);
     std::vector<double> h(6 * static_cast<size_t>(nbox));
     hipError_t e = hipMemcpyAsync(h.data(), sums, h.size() * sizeof(double),
                                   hipMemcpyDeviceToHost, s->stream);
@@ -1550,8 +1608,13 @@ int msm_calc_atomic_stress(msm_sim* s, double* avp) {
     clear_flags(s);
     enqueue_density(s);
     AtomsDev a = atoms_view(s, s->scur, s->pcur);
-    msm::launch_virial(a, list_view(s), s->tab, s->boxes[0], s->d_boxes, multibox(s), vir,
-                       s->stream);
+    msm::WalkPlan wp{};
+    if (aux_plan(s, wp))
+        msm::launch_virial_walk(wp, a, list_view(s), s->tab, s->boxes[0], s->d_boxes,
+                                multibox(s), vir, s->stream);
+    else
+        msm::launch_virial(a, list_view(s), s->tab, s->boxes[0], s->d_boxes, multibox(s), vir,
+                           s->stream);
     msm::launch_unsort_stress(vir, out, s->set[s->scur].gid, n, s->stream);
     hipError_t e = hipMemcpyAsync(avp, out, 9 * static_cast<size_t>(n) * sizeof(double),
                                   hipMemcpyDeviceToHost, s->stream);
@@ -1689,44 +1752,36 @@ int msm_dyn_damp(msm_sim* s, int maxsteps, double mindele, double h, int* steps,
     if (maxsteps < 0) return set_err(s, MSM_ERR_ARG, "maxsteps must be >= 0");
     (void)hipSetDevice(s->device);
     const int n = s->n;
-    double* epot0 = nullptr;
     unsigned long long* dmax = nullptr;
-    rc = dalloc(s, &epot0, std::max(n, 1));
-    if (rc == MSM_OK) rc = dalloc(s, &dmax, 1);
-    if (rc != MSM_OK) {
-        dfree(&epot0);
-        return rc;
-    }
+    rc = dalloc(s, &dmax, 2);  // the running maximum and its block counter
+    if (rc != MSM_OK) return rc;
     clear_flags(s);
-    // UpdateEPOT_ForceClass, then copy (Do_DynDamp_Forsteps_DEV, MD_DiffScheme_GPU.F90:1809-1883)
-    msm::launch_epot(atoms_view(s, s->scur, s->pcur), list_view(s), s->tab, s->boxes[0],
-                     s->d_boxes, multibox(s), s->d_err, s->stream);
-    hipError_t e = hipMemcpyAsync(epot0, s->epot, std::max(n, 1) * sizeof(double),
+    msm::launch_fill_int(reinterpret_cast<int*>(dmax), 0, 4, s->stream);
+    // UpdateEPOT_ForceClass, then the loop of Do_DynDamp_Forsteps_DEV (MD_DiffScheme_GPU.F90:
+    // 1809-1883).  One kernel makes the corrector of an iteration, the damping and the predictor of
+    // the next; the energy pass leaves F' for the force pass; the largest energy change reaches the
+    // host through its pinned words.
+    enqueue_epot(s);
+    hipError_t e = hipMemcpyAsync(s->qwork, s->epot, std::max(n, 1) * sizeof(double),
                                   hipMemcpyDeviceToDevice, s->stream);
     int it = 1;
     double del = 0.0;
     for (; e == hipSuccess && it <= maxsteps; ++it) {
         AtomsDev a = atoms_view(s, s->scur, s->pcur);
-        msm::launch_damping(a, s->stream);
-        msm::launch_predictor(a, s->tab, s->boxes[0], s->d_boxes, multibox(s), h, s->stream);
-        enqueue_density(s);
+        msm::launch_damp_step(a, s->tab, s->boxes[0], s->d_boxes, multibox(s), h, it > 1,
+                              s->stream);
+        enqueue_epot(s, nullptr, 1);
         enqueue_force(s, 0, 1, 0.0);
-        a = atoms_view(s, s->scur, s->pcur);
-        msm::launch_epot(a, list_view(s), s->tab, s->boxes[0], s->d_boxes, multibox(s), s->d_err,
-                         s->stream);
-        unsigned long long bits = 0;
-        e = hipMemsetAsync(dmax, 0, sizeof(unsigned long long), s->stream);
+        msm::launch_epot_maxdelta_host(s->epot, s->qwork, n, dmax, s->h_word, s->stream);
+        e = hipStreamSynchronize(s->stream);
         if (e != hipSuccess) break;
-        msm::launch_epot_maxdelta(s->epot, epot0, n, dmax, s->stream);
-        e = hipMemcpyAsync(&bits, dmax, sizeof(bits), hipMemcpyDeviceToHost, s->stream);
-        if (e == hipSuccess) e = hipStreamSynchronize(s->stream);
-        if (e != hipSuccess) break;
-        std::memcpy(&del, &bits, sizeof(del));
+        del = n > 0 ? *s->h_word : 0.0;
         if (del <= mindele) break;  // converged: the reference leaves before the corrector
-        msm::launch_correction(a, s->tab, h, s->stream);
     }
-    if (e == hipSuccess) e = hipStreamSynchronize(s->stream);
-    dfree(&epot0);
+    if (e == hipSuccess && it > maxsteps && maxsteps > 0) {
+        msm::launch_correction(atoms_view(s, s->scur, s->pcur), s->tab, h, s->stream);
+        e = hipStreamSynchronize(s->stream);
+    }
     dfree(&dmax);
     if (e != hipSuccess) return set_err(s, MSM_ERR_HIP, hipGetErrorString(e));
     if (steps) *steps = it;  // maxsteps + 1 when not converged, as the reference's ITER
@@ -1793,8 +1848,7 @@ struct Quench {
     }
     // UpdateEPOT_ForceClass
     void epot() {
-        msm::launch_epot(atoms_view(s, s->scur, s->pcur), list_view(s), s->tab, s->boxes[0],
-                         s->d_boxes, multibox(s), s->d_err, s->stream);
+        enqueue_epot(s);
     }
     void copy_epot0() {
         if (ok())
@@ -2551,7 +2605,7 @@ int msm_set_spline_table(msm_sim* s, const double* coef, int ld, int coef_on_dev
         c = s->fm_coef;
     }
     // same buffers, sizes and grid: the table descriptor and captured segments stay valid
-    msm::launch_spline_tables(c, ld, s->tab, s->d_b1, s->d_f2, s->d_b2, s->d_f4, s->d_e4, s->d_m4, s->stream);
+    msm::launch_spline_tables(c, ld, s->tab, s->d_b1, s->d_f2, s->d_e2, s->d_b2, s->d_f4, s->d_e4, s->d_m4, s->stream);
     HIPCHK(s, hipGetLastError());
     // stream-ordered before every later call on this context; msm_set_force_table, whose
     // copies are not, and the next build wait for the event.  A caller's device coefficients
@@ -2606,14 +2660,14 @@ int msm_fm_loss_grad(msm_sim* s, double* loss, double* coef_grad, int ld, int gr
     hipError_t ce = hipSuccess;
     auto enqueue = [&]() {
         clear_flags(s);
-        enqueue_density(s);
+        {
+            // the energy pass is the density pass too: it leaves F' in pos.w and, with a gradient,
+            // keeps rho for the adjoint, whose own rho pass is skipped
+            TimedScope ts(s, MSM_KCLASS_DENSITY);
+            enqueue_epot(s, coef_grad ? s->adj_rho : nullptr, 1);
+        }
         enqueue_force(s, 0, 1, 0.0);
-        AtomsDev a = atoms_view(s, s->scur, s->pcur);
-        // with a gradient the energy pass also keeps rho for the adjoint, whose F' is the
-        // density pass's (in pos.w), so the adjoint's own rho pass is skipped
-        msm::launch_epot(a, list_view(s), s->tab, s->boxes[0], s->d_boxes, multibox(s), s->d_err,
-                         s->stream, coef_grad ? s->adj_rho : nullptr);
-        msm::launch_box_sum(s->epot, s->sb.start, s->d_boxes, nbox, s->d_ebox, s->stream);
+        enqueue_box_sums(s, s->epot, 0, 1, s->d_ebox);
         const AtomSet& z = s->set[s->scur];
         const size_t na = s->n_alloc;
         msm::launch_fm_loss(z.f, z.f + na, z.f + 2 * na, z.gid, n, s->fm_ft, s->d_ebox, s->fm_et,

@@ -34,6 +34,7 @@ struct BoxDev {
     int bdim[3];   // cells per brick of the LDS-staged list build
     int nbrick[3]; // bricks per direction
     int brick_off; // first global brick id of this box
+    int chunk_off; // first chunk of this box's sums (launch_box_sums)
     int cbs;       // cell ordering: bricks of cbs^3 cells are contiguous (1 = row-major)
 };
 
@@ -47,6 +48,7 @@ constexpr int kNlMaxHalo = 216;
 struct TabDev {
     const double* b1;   // density knots POTB alone (filled into LDS by the list-walk passes)
     const double2* f2;  // force knots {FPOTR, FPOTB} alone (as b1)
+    const double2* e2;  // energy knots {POTR, POTB} alone (as b1)
     const double2* b2;  // density table {POTB, dPOTB}, nkind x (ntab+2)
     const double4* f4;  // force table {FPOTR, dFPOTR, FPOTB, dFPOTB}
     const double4* e4;  // energy table {POTR, dPOTR, POTB, dPOTB}
@@ -205,6 +207,15 @@ void launch_density_walk(const WalkPlan& pl, const AtomsDev& a, const ListDev& l
 void launch_force_walk(const WalkPlan& pl, const AtomsDev& a, const ListDev& l, const TabDev& t,
                        const BoxDev& box0, const BoxDev* boxes, int multibox,
                        const StepParams& sp, hipStream_t s);
+// Energies (and, optionally, rho and F' in pos.w) and virials on the same walk
+// (msm_walk_energy.hip); vir as launch_virial.  Lanes: 2, 4, 8 with the knots in LDS (fewer taken as
+// 2), else 8, 16, 32.
+void launch_energy_walk(const WalkPlan& pl, const AtomsDev& a, const ListDev& l, const TabDev& t,
+                        const BoxDev& box0, const BoxDev* boxes, int multibox, double* rho_out,
+                        int write_fp, int* err, hipStream_t s);
+void launch_virial_walk(const WalkPlan& pl, const AtomsDev& a, const ListDev& l, const TabDev& t,
+                        const BoxDev& box0, const BoxDev* boxes, int multibox, double* vir,
+                        hipStream_t s);
 // LDS bricks with the table window in LDS (msm_ldstab.hip): tpa (1, 2 or 4) lanes per home
 // atom, persistent grids over the bricks of the list build (whose slot list they read); the
 // staged halo capacity (at most the list build's, l.scap) and the windows share the LDS.
@@ -265,7 +276,7 @@ void launch_adjoint(const AtomsDev& a, const ListDev& l, const TabDev& t, const 
 // (part: fm_parts(n) doubles of scratch).  launch_spline_grad: dL/dc (3 rows of ld) from the
 // adjoint's bins of one kind.
 void launch_spline_tables(const double* coef, int ld, const TabDev& t, double* b1, double2* f2,
-                          double2* b2, double4* f4,
+                          double2* e2, double2* b2, double4* f4,
                           double4* e4, double4* m4, hipStream_t s);
 int fm_parts(int n);
 void launch_fm_loss(const double* fx, const double* fy, const double* fz, const int* gid, int n,
@@ -291,6 +302,13 @@ void launch_epot(const AtomsDev& a, const ListDev& l, const TabDev& t, const Box
 void launch_predictor(const AtomsDev& a, const TabDev& t, const BoxDev& box0,
                       const BoxDev* boxes, int multibox, double h, hipStream_t s);
 void launch_correction(const AtomsDev& a, const TabDev& t, double h, hipStream_t s);
+// One step of the damped quench up to the predictor: [corrector of the step before,] damping,
+// predictor.
+void launch_damp_step(const AtomsDev& a, const TabDev& t, const BoxDev& box0, const BoxDev* boxes,
+                      int multibox, double h, int correct, hipStream_t s);
+// max |epot - epot0| into *host (pinned), then epot0 = epot; work: two words, zero before and after.
+void launch_epot_maxdelta_host(const double* epot, double* epot0, int n, unsigned long long* work,
+                               double* host, hipStream_t s);
 void launch_unsort_d(const double* src, double* dst, const int* gid, int n, hipStream_t s);
 void launch_sort_pos(const double* src, double4* dst, const int* gid, int n, hipStream_t s);
 void launch_sort_d(const double* src, double* dst, const int* gid, int n, hipStream_t s);
@@ -350,8 +368,13 @@ void launch_move3(const AtomsDev& a, P3 dx, const BoxDev& box0, const BoxDev* bo
                   hipStream_t s);
 // AVP(N, 9) in caller order (column-major) from launch_virial's per-atom halves.
 void launch_unsort_stress(const double* vir, double* avp, const int* gid, int n, hipStream_t s);
-void launch_box_sum(const double* epot, const int* start, const BoxDev* boxes, int nbox,
-                    double* out, hipStream_t s);
+// Sums of ncomp per-atom arrays (stride n_stride) over the atoms of every box, in a fixed order:
+// blocks of kSumChunk atoms (chunk_box: the box of each of nchunk chunks; BoxDev::chunk_off the
+// box's first), then the chunks of a box.  part: ncomp x nchunk doubles; out[c * nbox + box].
+constexpr int kSumChunk = 2048;
+void launch_box_sums(const double* v, size_t n_stride, int ncomp, const int* start,
+                     const BoxDev* boxes, int nbox, const int* chunk_box, int nchunk,
+                     double* part, double* out, hipStream_t s);
 void launch_list_stats(const int* kvois, int n, unsigned long long* total, int* maxk,
                        hipStream_t s);
 

@@ -306,20 +306,42 @@ void launch_epot(const AtomsDev& a, const ListDev& l, const TabDev& t, const Box
 // stand-alone integrator kernels (Predictor_DEV / Correction_DEV)
 // --------------------------------------------------------------------------------------------
 
-template <int MB>
+// DAMP: the damping of the quench in front of the predictor; CORR: in front of that, the corrector
+// of the step before with the same forces (k_correction, k_damping and k_predictor in one).
+template <int MB, int DAMP, int CORR>
 __global__ __launch_bounds__(kBlock) void k_predictor(AtomsDev a, TabDev t, BoxDev box0,
                                                       const BoxDev* __restrict__ boxes, double h) {
 #pragma clang fp contract(off)
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= a.n) return;
     int stat = a.statu[i];
-    if ((stat & STATU_ACTIVE) != STATU_ACTIVE) return;
+    const bool active = (stat & STATU_ACTIVE) == STATU_ACTIVE;
+    if (!active && !DAMP) return;
     const int st0 = stat;
     const BoxDev& b = box_of<MB>(box0, boxes, a.boxid, i);
     const double hs2 = h * 0.5, h2s2 = h * hs2;
     const double cm0 = t.cm[a.ityp[i]];
-    const double ax = a.fx[i] / cm0, ay = a.fy[i] / cm0, az = a.fz[i] / cm0;
+    const double fx = a.fx[i], fy = a.fy[i], fz = a.fz[i];
+    const double ax = fx / cm0, ay = fy / cm0, az = fz / cm0;
     double vx = a.vx[i], vy = a.vy[i], vz = a.vz[i];
+    if constexpr (CORR) {
+        if (active) {
+            if (!(stat & (STATU_FIXVELX | STATU_FIXPOSX))) vx = vx + hs2 * ax;
+            if (!(stat & (STATU_FIXVELY | STATU_FIXPOSY))) vy = vy + hs2 * ay;
+            if (!(stat & (STATU_FIXVELZ | STATU_FIXPOSZ))) vz = vz + hs2 * az;
+        }
+    }
+    if constexpr (DAMP) {
+        if (vx * fx < 0.0 || (stat & STATU_FIXPOSX)) vx = 0.0;
+        if (vy * fy < 0.0 || (stat & STATU_FIXPOSY)) vy = 0.0;
+        if (vz * fz < 0.0 || (stat & STATU_FIXPOSZ)) vz = 0.0;
+        if (!active) {
+            a.vx[i] = vx;
+            a.vy[i] = vy;
+            a.vz[i] = vz;
+            return;
+        }
+    }
     const double4 p = a.pos[i];
     double x = p.x, y = p.y, z = p.z;
     double dx = h * vx + h2s2 * ax;
@@ -364,11 +386,24 @@ void launch_predictor(const AtomsDev& a, const TabDev& t, const BoxDev& box0,
                       const BoxDev* boxes, int multibox, double h, hipStream_t s) {
     if (a.n <= 0) return;
     if (multibox)
-        hipLaunchKernelGGL(k_predictor<1>, dim3(grid_for(a.n)), dim3(kBlock), 0, s, a, t, box0,
+        hipLaunchKernelGGL((k_predictor<1, 0, 0>), dim3(grid_for(a.n)), dim3(kBlock), 0, s, a, t, box0,
                            boxes, h);
     else
-        hipLaunchKernelGGL(k_predictor<0>, dim3(grid_for(a.n)), dim3(kBlock), 0, s, a, t, box0,
+        hipLaunchKernelGGL((k_predictor<0, 0, 0>), dim3(grid_for(a.n)), dim3(kBlock), 0, s, a, t, box0,
                            boxes, h);
+}
+
+void launch_damp_step(const AtomsDev& a, const TabDev& t, const BoxDev& box0, const BoxDev* boxes,
+                      int multibox, double h, int correct, hipStream_t s) {
+    if (a.n <= 0) return;
+    const dim3 g(grid_for(a.n)), b(kBlock);
+    if (multibox) {
+        if (correct) hipLaunchKernelGGL((k_predictor<1, 1, 1>), g, b, 0, s, a, t, box0, boxes, h);
+        else         hipLaunchKernelGGL((k_predictor<1, 1, 0>), g, b, 0, s, a, t, box0, boxes, h);
+    } else {
+        if (correct) hipLaunchKernelGGL((k_predictor<0, 1, 1>), g, b, 0, s, a, t, box0, boxes, h);
+        else         hipLaunchKernelGGL((k_predictor<0, 1, 0>), g, b, 0, s, a, t, box0, boxes, h);
+    }
 }
 
 __global__ __launch_bounds__(kBlock) void k_correction(AtomsDev a, TabDev t, double h) {
@@ -540,6 +575,41 @@ void launch_epot_maxdelta(const double* epot, double* epot0, int n, unsigned lon
     if (n > 0)
         hipLaunchKernelGGL(k_epot_maxdelta, dim3(grid_for(n)), dim3(kBlock), 0, s, epot, epot0, n,
                            out);
+}
+
+// The same, written to pinned host memory by the last workgroup, which leaves the maximum and the
+// workgroup counter at zero for the next call (one launch in place of a clear, the reduction and a
+// copy).
+__global__ __launch_bounds__(kBlock) void k_epot_maxdelta_host(const double* __restrict__ epot,
+                                                               double* __restrict__ epot0, int n,
+                                                               unsigned long long* work,
+                                                               double* __restrict__ host) {
+    __shared__ double lds[kBlock / 64];
+    double d = 0.0;
+    for (int i = blockIdx.x * kBlock + threadIdx.x; i < n; i += gridDim.x * kBlock) {
+        const double v = epot[i];
+        d = fmax(d, fabs(v - epot0[i]));
+        epot0[i] = v;
+    }
+    for (int o = 32; o > 0; o >>= 1) d = fmax(d, __shfl_xor(d, o, 64));
+    if ((threadIdx.x & 63) == 0) lds[threadIdx.x >> 6] = d;
+    __syncthreads();
+    if (threadIdx.x != 0) return;
+    for (int k = 1; k < kBlock / 64; ++k) d = fmax(d, lds[k]);
+    if (d > 0.0) atomicMax(&work[0], static_cast<unsigned long long>(__double_as_longlong(d)));
+    __threadfence();
+    if (atomicAdd(&work[1], 1ull) + 1ull == gridDim.x) {
+        __threadfence();
+        *host = __longlong_as_double(static_cast<long long>(atomicExch(&work[0], 0ull)));
+        atomicExch(&work[1], 0ull);
+    }
+}
+
+void launch_epot_maxdelta_host(const double* epot, double* epot0, int n, unsigned long long* work,
+                               double* host, hipStream_t s) {
+    if (n > 0)
+        hipLaunchKernelGGL(k_epot_maxdelta_host, dim3(std::min(grid_for(n), 256u)), dim3(kBlock), 0,
+                           s, epot, epot0, n, work, host);
 }
 
 // --------------------------------------------------------------------------------------------
@@ -965,31 +1035,73 @@ void launch_virial(const AtomsDev& a, const ListDev& l, const TabDev& t, const B
     }
 }
 
-// One workgroup per box: fixed-order strided partial sums then a fixed-shape tree, so the total
-// is the same on every run.
-__global__ __launch_bounds__(kBlock) void k_box_sum(const double* __restrict__ epot,
-                                                    const int* __restrict__ start,
-                                                    const BoxDev* __restrict__ boxes,
-                                                    double* __restrict__ out) {
-    __shared__ double lds[kBlock];
-    const BoxDev b = boxes[blockIdx.x];
-    const int c0 = b.cell_off, c1 = b.cell_off + b.ncell[0] * b.ncell[1] * b.ncell[2];
-    const int a0 = start[c0], a1 = start[c1];
-    double s = 0.0;
-    for (int i = a0 + threadIdx.x; i < a1; i += kBlock) s += epot[i];
+// Box sums of per-atom arrays, the same on every run: a workgroup adds kSumChunk atoms (eight loads a
+// thread in flight, then a fixed-shape tree), a second launch the chunks of a box.  One workgroup
+// per box walking all its atoms took 51 us for 54,000 atoms, six times over for a virial.
+__device__ __forceinline__ double block_sum(double s, double* lds) {
     lds[threadIdx.x] = s;
     __syncthreads();
     for (int w = kBlock / 2; w > 0; w >>= 1) {
         if ((int)threadIdx.x < w) lds[threadIdx.x] += lds[threadIdx.x + w];
         __syncthreads();
     }
-    if (threadIdx.x == 0) out[blockIdx.x] = lds[0];
+    return lds[0];
 }
 
-void launch_box_sum(const double* epot, const int* start, const BoxDev* boxes, int nbox,
-                    double* out, hipStream_t s) {
-    if (nbox > 0)
-        hipLaunchKernelGGL(k_box_sum, dim3(nbox), dim3(kBlock), 0, s, epot, start, boxes, out);
+__global__ __launch_bounds__(kBlock) void k_sum_chunks(const double* __restrict__ v,
+                                                       size_t n_stride,
+                                                       const int* __restrict__ start,
+                                                       const BoxDev* __restrict__ boxes,
+                                                       const int* __restrict__ chunk_box,
+                                                       int nbox, double* __restrict__ part,
+                                                       double* __restrict__ out) {
+    __shared__ double lds[kBlock];
+    constexpr int kPer = kSumChunk / kBlock;
+    const int bi = chunk_box[blockIdx.x], c = blockIdx.y;
+    const BoxDev& b = boxes[bi];
+    const int c0 = b.cell_off, c1 = b.cell_off + b.ncell[0] * b.ncell[1] * b.ncell[2];
+    const int a0 = start[c0] + (static_cast<int>(blockIdx.x) - b.chunk_off) * kSumChunk,
+              a1 = start[c1];
+    double x[kPer];
+#pragma unroll
+    for (int k = 0; k < kPer; ++k) {
+        const int i = a0 + k * kBlock + threadIdx.x;
+        x[k] = i < a1 ? v[c * n_stride + i] : 0.0;
+    }
+    double s = 0.0;
+#pragma unroll
+    for (int k = 0; k < kPer; ++k) s += x[k];
+    s = block_sum(s, lds);
+    if (threadIdx.x == 0) {
+        part[static_cast<size_t>(c) * gridDim.x + blockIdx.x] = s;
+        if (b.natoms <= kSumChunk) out[c * nbox + bi] = s;  // the box's only chunk
+    }
+}
+
+__global__ __launch_bounds__(kBlock) void k_sum_boxes(const BoxDev* __restrict__ boxes, int nbox,
+                                                      int nchunk, const double* __restrict__ part,
+                                                      double* __restrict__ out) {
+    __shared__ double lds[kBlock];
+    const int bi = blockIdx.x, c = blockIdx.y;
+    const BoxDev& b = boxes[bi];
+    if (b.natoms <= kSumChunk) return;
+    const int k1 = b.chunk_off + (b.natoms + kSumChunk - 1) / kSumChunk;
+    double s = 0.0;
+    for (int k = b.chunk_off + threadIdx.x; k < k1; k += kBlock)
+        s += part[static_cast<size_t>(c) * nchunk + k];
+    s = block_sum(s, lds);
+    if (threadIdx.x == 0) out[c * nbox + bi] = s;
+}
+
+void launch_box_sums(const double* v, size_t n_stride, int ncomp, const int* start,
+                     const BoxDev* boxes, int nbox, const int* chunk_box, int nchunk,
+                     double* part, double* out, hipStream_t s) {
+    if (nbox <= 0) return;
+    hipLaunchKernelGGL(k_sum_chunks, dim3(nchunk, ncomp), dim3(kBlock), 0, s, v, n_stride, start,
+                       boxes, chunk_box, nbox, part, out);
+    if (nchunk > nbox)
+        hipLaunchKernelGGL(k_sum_boxes, dim3(nbox, ncomp), dim3(kBlock), 0, s, boxes, nbox,
+                           nchunk, part, out);
 }
 
 // Sum and maximum of KVOIS: grid-stride partial results, reduced per wave and then per

@@ -1,0 +1,320 @@
+// msm_walk.h -- what the list-walk kernels share (msm_walk.hip, msm_walk_energy.hip): units and
+// lanes, knot access, the side road of odd pairs, the force of a group of slots, launch shapes.
+#pragma once
+
+#include <algorithm>
+#include <type_traits>
+
+#include "msm_device.h"
+
+namespace msm {
+
+namespace {
+
+template <int CTRL>
+__device__ __forceinline__ double dpp(double v) {
+    const unsigned long long a = static_cast<unsigned long long>(__double_as_longlong(v));
+    const unsigned lo = static_cast<unsigned>(__builtin_amdgcn_mov_dpp(
+        static_cast<int>(static_cast<unsigned>(a)), CTRL, 0xF, 0xF, true));
+    const unsigned hi = static_cast<unsigned>(__builtin_amdgcn_mov_dpp(
+        static_cast<int>(static_cast<unsigned>(a >> 32)), CTRL, 0xF, 0xF, true));
+    return __longlong_as_double(
+        static_cast<long long>((static_cast<unsigned long long>(hi) << 32) | lo));
+}
+
+// Sum over the L consecutive lanes of an atom, in every lane (all lanes of the wave active):
+// quad permutes, half-row and row mirrors, then a swizzle across the two rows of 16.
+template <int L>
+__device__ __forceinline__ double atom_sum(double v) {
+    if constexpr (L >= 2) v = v + dpp<0xB1>(v);
+    if constexpr (L >= 4) v = v + dpp<0x4E>(v);
+    if constexpr (L >= 8) v = v + dpp<0x141>(v);
+    if constexpr (L >= 16) v = v + dpp<0x140>(v);
+    if constexpr (L >= 32) {
+        const unsigned long long a = static_cast<unsigned long long>(__double_as_longlong(v));
+        const unsigned lo = static_cast<unsigned>(
+            __builtin_amdgcn_ds_swizzle(static_cast<int>(static_cast<unsigned>(a)), 0x401F));
+        const unsigned hi = static_cast<unsigned>(
+            __builtin_amdgcn_ds_swizzle(static_cast<int>(static_cast<unsigned>(a >> 32)), 0x401F));
+        v = v + __longlong_as_double(
+                    static_cast<long long>((static_cast<unsigned long long>(hi) << 32) | lo));
+    }
+    return v;
+}
+
+// A pointer that is the same in every lane, in scalar registers.
+__device__ __forceinline__ const int* uniform(const int* p) {
+    const unsigned long long a = reinterpret_cast<unsigned long long>(p);
+    const unsigned lo = __builtin_amdgcn_readfirstlane(static_cast<unsigned>(a));
+    const unsigned hi = __builtin_amdgcn_readfirstlane(static_cast<unsigned>(a >> 32));
+    return reinterpret_cast<const int*>((static_cast<unsigned long long>(hi) << 32) | lo);
+}
+
+constexpr int ilog2(int v) { return v <= 1 ? 0 : 1 + ilog2(v / 2); }
+
+// Slots per group: the gathers of a group are in flight together.
+constexpr int group_d(int L) { return L <= 4 ? 6 : L == 8 ? 4 : 3; }
+constexpr int group_f(int) { return 3; }
+
+// What a lane needs of its unit.
+struct Lane {
+    const int* blk;   // list block of the unit's atoms (uniform)
+    unsigned lo;      // byte offset of the lane's first slot in it
+    unsigned ib;      // atom index
+    int kv;           // list length (0: inactive)
+    int sub;          // lane within the atom
+    int last;         // the lane's last slot
+    int ti;           // type
+};
+
+// Units of this wave: u = first, first + step, ... < end.  sweep = 0: each workgroup takes an
+// equal contiguous range of its XCD's units, its waves in turn; sweep = 1: the workgroups of an
+// XCD take that XCD's range in turn.
+__device__ __forceinline__ void unit_iter(int units, int sweep, int& first, int& step, int& end) {
+    const int nb = gridDim.x, nw = blockDim.x >> 6;
+    const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    if (!sweep || nb < 8) {
+        const int b = xcd_block(nb);
+        first = static_cast<int>(static_cast<long long>(b) * units / nb) + wv;
+        end = static_cast<int>(static_cast<long long>(b + 1) * units / nb);
+        step = nw;
+    } else {
+        const int x = blockIdx.x & 7, k = blockIdx.x >> 3;
+        first = static_cast<int>(static_cast<long long>(x) * units / 8) + k * nw + wv;
+        end = static_cast<int>(static_cast<long long>(x + 1) * units / 8);
+        step = ((nb - x + 7) >> 3) * nw;
+    }
+}
+
+// Whether an atom at (x, y, z) lies further than m from every periodic face of its box.
+__device__ __forceinline__ bool inner(const BoxDev& b, double m, double x, double y, double z) {
+    const double dx = x - b.lo[0], dy = y - b.lo[1], dz = z - b.lo[2];
+    return (!b.ifpd[0] || (dx > m && b.len[0] - dx > m)) &&
+           (!b.ifpd[1] || (dy > m && b.len[1] - dy > m)) &&
+           (!b.ifpd[2] || (dz > m && b.len[2] - dz > m));
+}
+
+__device__ __forceinline__ int slot_index(const Lane& q, int s, int shift) {
+    return at(q.blk, q.lo + (static_cast<unsigned>(s) << shift));
+}
+
+// Knots: from the LDS window (TL = 1: rows of w.w knots from knot w.k0) or from global memory.
+template <int TL>
+struct Knots;
+template <>
+struct Knots<1> {
+    const double* d;    // POTB
+    const double2* f;   // {FPOTR, FPOTB}
+    __device__ __forceinline__ void den(int q, double& v, double& dv) const {
+        const double p0 = d[q], p1 = d[q + 1];
+        v = p0;
+        dv = p1 - p0;
+    }
+    __device__ __forceinline__ void frc(int q, double& r, double& dr, double& b, double& db) const {
+        const double2 t0 = f[q], t1 = f[q + 1];
+        r = t0.x;
+        dr = t1.x - t0.x;
+        b = t0.y;
+        db = t1.y - t0.y;
+    }
+    __device__ __forceinline__ void frb(int q, double& b, double& db) const {
+        b = f[q].y;
+        db = f[q + 1].y - b;
+    }
+};
+template <>
+struct Knots<0> {
+    const double2* d;
+    const double4* f;
+    __device__ __forceinline__ void den(int q, double& v, double& dv) const {
+        const double2 e = at(d, static_cast<unsigned>(q) * 16u);
+        v = e.x;
+        dv = e.y;
+    }
+    __device__ __forceinline__ void frc(int q, double& r, double& dr, double& b, double& db) const {
+        const double4 e = at(f, static_cast<unsigned>(q) * 32u);
+        r = e.x;
+        dr = e.y;
+        b = e.z;
+        db = e.w;
+    }
+    __device__ __forceinline__ void frb(int q, double& b, double& db) const {
+        const double4 e = at(f, static_cast<unsigned>(q) * 32u);
+        b = e.z;
+        db = e.w;
+    }
+};
+
+// A pair's place in the table.  ok: inside the cutoff with its knots in the window (q is in
+// bounds either way); odd: the pair goes the side road.
+struct Place {
+    double sk, inv_r, dk;
+    int kk, q;
+    bool ok, odd;
+};
+
+template <int IMG>
+__device__ __forceinline__ Place place(const TabDev& t, const WalkDev& w, double r2) {
+    Place p;
+    p.sk = table_coord(r2, t.csi, p.inv_r);
+    p.kk = static_cast<int>(p.sk);
+    p.dk = p.sk - p.kk;
+    const unsigned kd = static_cast<unsigned>(p.kk - w.k0);
+    const bool reg = kd <= static_cast<unsigned>(w.last), in = r2 <= t.ru2max;
+    const bool far = IMG == 0 && p.kk >= w.kimg;
+    p.q = static_cast<int>(min(kd, static_cast<unsigned>(w.last)));
+    p.ok = reg && in && !far;
+    p.odd = (in && !reg) || far;
+    return p;
+}
+
+// Whether a lane's slot s is in the list.
+template <int L>
+__device__ __forceinline__ bool listed(const Lane& q, int s) {
+    return s * L + q.sub < q.kv;
+}
+
+__device__ __forceinline__ void add_virial(double h, double sx, double sy, double sz,
+                                           double (&v)[6]) {
+    v[0] = v[0] + sx * sx * h;
+    v[1] = v[1] + sy * sy * h;
+    v[2] = v[2] + sz * sz * h;
+    v[3] = v[3] + sx * sy * h;
+    v[4] = v[4] + sx * sz * h;
+    v[5] = v[5] + sy * sz * h;
+}
+
+// V = 1: the half virial of every pair as well (components xx, yy, zz, xy, xz, yz).
+template <int MT, int IMG, int LG, int V>
+__device__ __forceinline__ void force_odd(const AtomsDev& a, const TabDev& t, const WalkDev& w,
+                                          const BoxDev& b, const Lane& q, int s, int cnt,
+                                          const double4& pi, double& fx, double& fy, double& fz,
+                                          double (&vir)[6]) {
+#pragma unroll 1
+    for (int u = 0; u < cnt; ++u) {
+        if (s + u > q.last) break;
+        const int j = slot_index(q, s + u, 8 + LG);
+        const double4 pj = a.pos[j];
+        double sx = pi.x - pj.x, sy = pi.y - pj.y, sz = pi.z - pj.z;
+        if constexpr (IMG == 0) {
+            if (!place<0>(t, w, sx * sx + sy * sy + sz * sz).odd) continue;
+        }
+        sx = min_image(sx, b.len[0], b.ilen[0]);
+        sy = min_image(sy, b.len[1], b.ilen[1]);
+        sz = min_image(sz, b.len[2], b.ilen[2]);
+        const double r2 = sx * sx + sy * sy + sz * sz;
+        if (!(r2 <= t.ru2max) || (IMG == 1 && !place<1>(t, w, r2).odd)) continue;
+        int kind = t.kpair[0], kind1 = t.kpair[0];
+        if constexpr (MT) {
+            const int tj = a.ityp[j];
+            kind = t.kpair[q.ti * t.ngroup + tj];
+            kind1 = t.kpair[tj * t.ngroup + q.ti];
+        }
+        double inv_r;
+        const double sk = table_coord(r2, t.csi, inv_r);
+        const int kk = min(static_cast<int>(sk), t.ntab2 - 2);
+        const double dk = sk - kk;
+        const double4 f = t.f4[static_cast<size_t>(kind) * t.ntab2 + kk];
+        const double4 f1 = t.f4[static_cast<size_t>(kind1) * t.ntab2 + kk];
+        const double ft = (f.x + dk * f.y) * (inv_r * inv_r) +
+                          ((f.z + dk * f.w) * pi.w + (f1.z + dk * f1.w) * pj.w) * inv_r;
+        fx = fx + ft * sx;
+        fy = fy + ft * sy;
+        fz = fz + ft * sz;
+        if constexpr (V) add_virial(0.5 * ft, sx, sy, sz, vir);
+    }
+}
+
+// As density_slots, for the force.
+template <int G, int FULL, int MT, int IMG, int L, int TL, int V>
+__device__ __forceinline__ void force_slots(const AtomsDev& a, const TabDev& t, const WalkDev& w,
+                                            const BoxDev& b, const Lane& q, const Knots<TL>& kn,
+                                            const int* s_row, int s, const double4& pi, double& fx,
+                                            double& fy, double& fz, double (&vir)[6], int (&js)[G]) {
+    constexpr int LG = ilog2(L);
+    double4 pj[G];
+    int tj[G];
+#pragma unroll
+    for (int u = 0; u < G; ++u) {
+        if (!FULL && u > 0 && (s + u) * L >= q.kv) break;
+        pj[u] = at(a.pos, static_cast<unsigned>(js[u]) << 5);
+        tj[u] = MT ? at(a.ityp, static_cast<unsigned>(js[u]) << 2) : 0;
+    }
+    if constexpr (FULL) {
+#pragma unroll
+        for (int u = 0; u < G; ++u) js[u] = slot_index(q, min(s + G + u, q.last), 8 + LG);
+    }
+    unsigned long long odd = 0;
+#pragma unroll
+    for (int u = 0; u < G; ++u) {
+        if (!FULL && u > 0 && (s + u) * L >= q.kv) break;
+        double sx = pi.x - pj[u].x, sy = pi.y - pj[u].y, sz = pi.z - pj[u].z;
+        if constexpr (IMG == 1) {
+            sx = min_image(sx, b.len[0], b.ilen[0]);
+            sy = min_image(sy, b.len[1], b.ilen[1]);
+            sz = min_image(sz, b.len[2], b.ilen[2]);
+        }
+        const Place p = place<IMG>(t, w, sx * sx + sy * sy + sz * sz);
+        const bool valid = FULL || listed<L>(q, s + u);
+        double fr, dfr, fb, dfb;
+        kn.frc(p.q + (MT ? s_row[q.ti * t.ngroup + tj[u]] : 0), fr, dfr, fb, dfb);
+        fb = fb + p.dk * dfb;
+        double fb1 = fb;
+        if constexpr (MT) {
+            double g, dg;
+            kn.frb(p.q + s_row[tj[u] * t.ngroup + q.ti], g, dg);
+            fb1 = g + p.dk * dg;
+        }
+        // FPOTR/r^2 + (FPOTB(KTAB) F'_i + FPOTB(KTAB1) F'_j)/r  (CALFORCE_KERNEL)
+        double ft = (fr + p.dk * dfr) * (p.inv_r * p.inv_r) + (fb * pi.w + fb1 * pj[u].w) * p.inv_r;
+        ft = (p.ok && valid) ? ft : 0.0;
+        fx = fx + ft * sx;
+        fy = fy + ft * sy;
+        fz = fz + ft * sz;
+        if constexpr (V) add_virial(0.5 * ft, sx, sy, sz, vir);
+        odd |= __ballot(p.odd && valid);
+    }
+    if (odd) force_odd<MT, IMG, LG, V>(a, t, w, b, q, s, G, pi, fx, fy, fz, vir);
+}
+
+// Window of the upper part of the table for an LDS share: knots from k0 on.
+inline void window(const TabDev& t, long budget, int bytes, WalkDev& w) {
+    const int nk = t.ngroup > 1 ? t.nkind : 1;
+    const int fit = static_cast<int>(std::max(0L, budget / (static_cast<long>(bytes) * nk)));
+    const int want = t.ntab2 - 3 * (t.ntab2 / 8);
+    w.w = std::min(want, fit);
+    w.k0 = t.ntab2 - w.w;
+    w.last = t.ntab2 - 2 - w.k0;
+}
+
+inline long walk_budget(const TabDev& t, int wgs) {
+    return lt_lds_budget(wgs) - (t.ngroup > 1 ? 4 * kMaxGroup * kMaxGroup : 0);
+}
+
+// Launch parameters common to the passes; returns the workgroups.
+template <typename K>
+unsigned walk_launch(K k, const WalkPlan& pl, int bytes, int n, const TabDev& t, WalkDev& w,
+                     int& threads, size_t& lds) {
+    w.kimg = pl.kimg;
+    w.margin = pl.margin;
+    w.sweep = pl.sweep;
+    w.units = (n + 64 / pl.lanes - 1) / (64 / pl.lanes);
+    if (pl.tl) {
+        threads = pl.block;
+        window(t, walk_budget(t, pl.wgs), bytes, w);
+        lds = static_cast<size_t>(w.w) * (t.ngroup > 1 ? t.nkind : 1) * bytes;
+        const int nwv = threads / 64;
+        return lt_persistent_grid(reinterpret_cast<const void*>(k), threads, lds, pl.wgs,
+                                  (w.units + nwv - 1) / nwv);
+    }
+    threads = kBlock;
+    lds = 0;
+    w.k0 = 0;
+    w.w = t.ntab2;
+    w.last = t.ntab2 - 2;
+    return static_cast<unsigned>((w.units + kBlock / 64 - 1) / (kBlock / 64));
+}
+
+}  // namespace
+
+}  // namespace msm

@@ -1,7 +1,9 @@
-"""The list-walk density and force passes against the oracle at the sizes where their lanes per
+"""The list-walk density, force, energy and stress passes against the oracle at the sizes where their lanes per
 atom and table placement change (32, 16, 8 lanes with the global table, 8, 4, 2 with the knots in
 LDS), and on positions whose pairs leave the fast road: atoms a box length or more out, pairs
-closer than the LDS window reaches.  Bars: F' 1e-13, forces 1e-10 eV/A max-abs."""
+closer than the LDS window reaches.  Bars: F' 1e-13, forces 1e-10 eV/A max-abs, total
+energy 1e-12 relative, each atom's energy and stress 1e-13 of their largest absolute value (sums of
+at most a hundred terms)."""
 import numpy as np
 import pytest
 
@@ -50,11 +52,21 @@ def test_walk_passes_vs_oracle(orc, name):
     it = box.ITYP - 1
     kv, ind = orc.nlist("full", box.XP, it, box.STATU, box.BOXLOW, box.ZL, ctrl.IFPD, ctrl.NB_RM,
                         ctrl.NB_MXNBS)
-    fo, do, _ = orc.force_full(np.asfortranarray(x), it, box.STATU, kv, ind, box.ZL, ctrl.IFPD,
-                               float(np.max(ctrl.RU)) ** 2, orc.from_mdlib(ft))
+    ru2, t = float(np.max(ctrl.RU)) ** 2, orc.from_mdlib(ft)
+    fo, do, eo = orc.force_full(np.asfortranarray(x), it, box.STATU, kv, ind, box.ZL, ctrl.IFPD,
+                                ru2, t)
+    ao, aabs = orc.atomic_stress_full(np.asfortranarray(x), it, box.STATU, kv, ind, box.ZL,
+                                      ctrl.IFPD, ru2, t, do, with_abs=True)
     df = np.max(np.abs(dev.get_forces() - fo))
     dd = np.max(np.abs(dev.get_den() - do) / np.maximum(1.0, np.abs(do)))
-    print(f"{name}: n={box.NPRT} {dev.pass_kernel()} max|dF|={df:.3e} max|dF'|={dd:.3e}")
+    dev.calc_epot()
+    de = np.max(np.abs(dev.get_epot() - eo)) / np.max(np.abs(eo))
+    et = abs(dev.get_box_epot()[0] - eo.sum()) / abs(eo.sum())
+    da = np.max(np.abs(dev.calc_atomic_stress() - ao)) / np.max(aabs)
+    print(f"{name}: n={box.NPRT} {dev.pass_kernel()} max|dF|={df:.3e} max|dF'|={dd:.3e} "
+          f"dE {de:.3e} total {et:.3e} stress {da:.3e}")
     dev.close()
     assert df <= 1e-10
     assert dd <= 1e-13
+    assert de <= 1e-13 and et <= 1e-12
+    assert da <= 1e-13
