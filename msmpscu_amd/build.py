@@ -37,7 +37,7 @@ def _run(cmd, cwd=None):
 
 SOURCES = ("msm_api.hip", "msm_kernels.hip", "msm_cells.hip", "msm_bricks.hip", "msm_tpa.hip", "msm_pair.hip",
            "msm_ldstab.hip", "msm_walk.hip", "msm_walk_energy.hip",
-           "msm_stage.hip", "msm_thermal.hip", "msm_adjoint.hip", "msm_host.cpp")
+           "msm_stage.hip", "msm_thermal.hip", "msm_adjoint.hip", "msm_copy.cpp", "msm_host.cpp")
 
 
 def build_library(jobs: int = 8) -> str:

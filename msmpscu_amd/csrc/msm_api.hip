@@ -13,6 +13,7 @@
 #include <tuple>
 #include <vector>
 
+#include "msm_copy.h"
 #include "msm_hip.h"
 #include "msm_internal.h"
 
@@ -48,6 +49,9 @@ struct GraphKey {
 };
 
 }  // namespace
+
+// The context's pinned words: flags and one double ahead, then room for small copies.
+constexpr size_t kPinnedHead = 64, kSmallCopy = size_t(64) << 10;
 
 struct msm_sim {
     int device = 0;
@@ -99,9 +103,13 @@ struct msm_sim {
     bool has_list = false;
 
     // flags and scratch
-    int* d_err = nullptr;
-    int* h_err = nullptr;      // pinned: the error flags, then one double (h_word)
+    int* d_err = nullptr;      // device address of h_err
+    int* h_err = nullptr;      // pinned: the error flags, one double (h_word), small copies
     double* h_word = nullptr;
+    char *h_small = nullptr, *d_small = nullptr;  // kSmallCopy bytes: host and device address
+    bool has_ring = false;     // counted among the users of the GPU's pinned copy ring
+    double* d_stage = nullptr; // copies to and from the host in the caller's order
+    size_t cap_stage = 0;
     double* qwork = nullptr;   // per-atom scratch (quench energies)
     double* d_ebox = nullptr;
     int nchunk = 0;               // chunks of the box sums, their boxes and partial sums (6 arrays)
@@ -237,6 +245,8 @@ void free_atoms(msm_sim* s) {
     }
     dfree(&s->epot);
     dfree(&s->qwork);
+    dfree(&s->d_stage);
+    s->cap_stage = 0;
     s->n = s->n_alloc = 0;
     s->has_atoms = false;
     s->has_list = false;
@@ -335,12 +345,38 @@ void resolve_timing(msm_sim* s) {
     s->pending.clear();
 }
 
-// Device error flags: cleared with a fill kernel so the clear can sit inside captured graphs.
-void clear_flags(msm_sim* s) { msm::launch_fill_int(s->d_err, 0, msm::kErrSlots, s->stream); }
+// Error flags (pinned host memory): cleared before the launches of a call, whose synchronisation at
+// its end leaves none of its kernels running.
+void clear_flags(msm_sim* s) {
+    for (int k = 0; k < msm::kErrSlots; ++k) s->h_err[k] = 0;
+}
+
+// A device block (its parts in order, without gaps; total a multiple of 4) to the caller's arrays.
+// Up to 64 KB a kernel writes it into the context's pinned words, which spares the copy engine's
+// start-up; beyond, the ring of msm_copy.h.  Returns with the stream idle and the data in place.
+hipError_t pull(msm_sim* s, const void* base, size_t total, const msm::CopyPart* parts,
+                int nparts) {
+    if (total > kSmallCopy)
+        return msm::copy_to_host(s->device, base, total, parts, nparts, s->stream);
+    msm::launch_copy_words(base, s->d_small, total, s->stream);
+    const hipError_t e = hipStreamSynchronize(s->stream);
+    if (e != hipSuccess) return e;
+    for (int k = 0; k < nparts; ++k)
+        std::memcpy(parts[k].host, s->h_small + parts[k].offset, parts[k].bytes);
+    return hipSuccess;
+}
+
+// The caller's array to a device block, the other way; with the block still to be read by work on
+// the stream, the caller synchronises before the next push.
+hipError_t push(msm_sim* s, void* dst, const void* host, size_t total) {
+    if (total > kSmallCopy)
+        return msm::copy_to_device(s->device, dst, host, total, s->stream);
+    std::memcpy(s->h_small, host, total);
+    msm::launch_copy_words(s->d_small, dst, total, s->stream);
+    return hipSuccess;
+}
 
 int read_flags(msm_sim* s) {
-    HIPCHK(s, hipMemcpyAsync(s->h_err, s->d_err, sizeof(int) * msm::kErrSlots,
-                             hipMemcpyDeviceToHost, s->stream));
     HIPCHK(s, hipStreamSynchronize(s->stream));
     resolve_timing(s);
     if (s->h_err[msm::kErrOutOfBox])
@@ -884,12 +920,21 @@ int msm_create(msm_sim** out, int device) {
         delete s;
         return MSM_ERR_HIP;
     }
-    int rc = dalloc(s, &s->d_err, msm::kErrSlots);
-    if (rc == MSM_OK) rc = dalloc(s, &s->d_stats, 2);
+    int rc = dalloc(s, &s->d_stats, 2);
     if (rc == MSM_OK && hipHostMalloc(reinterpret_cast<void**>(&s->h_err),
-                                      sizeof(int) * msm::kErrSlots + sizeof(double)) != hipSuccess)
+                                      kPinnedHead + kSmallCopy) != hipSuccess)
         rc = MSM_ERR_NOMEM;
-    if (rc == MSM_OK) s->h_word = reinterpret_cast<double*>(s->h_err + msm::kErrSlots);
+    if (rc == MSM_OK && hipHostGetDevicePointer(reinterpret_cast<void**>(&s->d_err), s->h_err, 0) !=
+                            hipSuccess)
+        rc = MSM_ERR_HIP;
+    if (rc == MSM_OK) {
+        s->h_word = reinterpret_cast<double*>(s->h_err + msm::kErrSlots);
+        s->h_small = reinterpret_cast<char*>(s->h_err) + kPinnedHead;
+        s->d_small = reinterpret_cast<char*>(s->d_err) + kPinnedHead;
+        clear_flags(s);
+        s->has_ring = msm::copy_ring_acquire(device) == hipSuccess;
+        if (!s->has_ring) rc = set_err(s, MSM_ERR_NOMEM, "pinned copy buffers");
+    }
     if (rc != MSM_OK) {
         msm_destroy(s);
         return rc;
@@ -936,13 +981,13 @@ int msm_destroy(msm_sim* s) {
     dfree(&s->cidx);
     dfree(&s->ckv);
     dfree(&s->cmask);
-    dfree(&s->d_err);
     dfree(&s->d_ebox);
     dfree(&s->d_chunk_box);
     dfree(&s->d_part);
     dfree(&s->d_stats);
     dfree(&s->d_boxwork);
     if (s->h_err) (void)hipHostFree(s->h_err);
+    if (s->has_ring) msm::copy_ring_release(s->device);
     if (s->fm_host) (void)hipHostFree(s->fm_host);
     if (s->stream) (void)hipStreamDestroy(s->stream);
     delete s;
@@ -1270,60 +1315,46 @@ int msm_get_atoms(msm_sim* s, double* xp, double* xp1, double* fp, int* statu, d
     (void)hipSetDevice(s->device);
     if (!s->has_atoms) return set_err(s, MSM_ERR_STATE, "no atoms");
     const int n = s->n;
-    const size_t na = s->n_alloc;
-    AtomSet& z = s->set[s->scur];
-    double* tmp = nullptr;
-    int* itmp = nullptr;
-    int rc = dalloc(s, &tmp, 3 * na);
-    if (rc == MSM_OK) rc = dalloc(s, &itmp, na);
-    if (rc != MSM_OK) {
-        dfree(&tmp);
-        return rc;
+    if (n == 0) return MSM_OK;
+    const size_t m = n;
+    const AtomsDev a = atoms_view(s, s->scur, s->pcur);
+    const int* gid = s->set[s->scur].gid;
+    void* const host[5] = {xp, xp1, fp, dis, statu};
+    // everything through one device block, or array by array where that would be large
+    const bool whole = m <= (size_t(1) << 22);
+    msm::CopyPart parts[5];
+    int np = 0, what = 0;
+    size_t total = 0;
+    for (int k = 0; k < 5; ++k) {
+        if (host[k]) {
+            const size_t bytes = k < 4 ? 3 * m * sizeof(double) : m * sizeof(int);
+            parts[np++] = {total, bytes, host[k]};
+            what |= 1 << k;
+            total += bytes;
+        }
+        if (!what || (whole && k < 4)) continue;
+        const int rc = dreserve(s, &s->d_stage, (total + 7) / 8, s->cap_stage);
+        if (rc != MSM_OK) return rc;
+        msm::launch_copy_out(a, gid, what, s->d_stage, s->stream);
+        HIPCHK(s, pull(s, s->d_stage, total, parts, np));
+        np = what = 0;
+        total = 0;
     }
-    auto pull3 = [&](const double* src3, double* host) -> int {
-        for (int k = 0; k < 3; ++k)
-            msm::launch_unsort_d(src3 + k * na, tmp + k * static_cast<size_t>(n), z.gid, n, s->stream);
-        HIPCHK(s, hipMemcpyAsync(host, tmp, 3 * static_cast<size_t>(n) * sizeof(double),
-                                 hipMemcpyDeviceToHost, s->stream));
-        HIPCHK(s, hipStreamSynchronize(s->stream));
-        return MSM_OK;
-    };
-    if (xp && n > 0) {
-        for (int k = 0; k < 3; ++k)
-            msm::launch_unsort_pos(s->pos[s->pcur], tmp + k * static_cast<size_t>(n), z.gid, n, k, s->stream);
-        HIPCHK(s, hipMemcpyAsync(xp, tmp, 3 * static_cast<size_t>(n) * sizeof(double),
-                                 hipMemcpyDeviceToHost, s->stream));
-        HIPCHK(s, hipStreamSynchronize(s->stream));
-    }
-    if (rc == MSM_OK && xp1 && n > 0) rc = pull3(z.v, xp1);
-    if (rc == MSM_OK && fp && n > 0) rc = pull3(z.f, fp);
-    if (rc == MSM_OK && dis && n > 0) rc = pull3(z.dis, dis);
-    if (rc == MSM_OK && statu && n > 0) {
-        msm::launch_unsort_i(z.statu, itmp, z.gid, n, s->stream);
-        hipError_t e = hipMemcpyAsync(statu, itmp, n * sizeof(int), hipMemcpyDeviceToHost, s->stream);
-        if (e == hipSuccess) e = hipStreamSynchronize(s->stream);
-        if (e != hipSuccess) rc = set_err(s, MSM_ERR_HIP, hipGetErrorString(e));
-    }
-    dfree(&tmp);
-    dfree(&itmp);
-    return rc;
+    return MSM_OK;
 }
 
 static int pull_sorted_d(msm_sim* s, const double* src, int comp_pos, double* host) {
     const int n = s->n;
     if (n == 0) return MSM_OK;
-    double* tmp = nullptr;
-    int rc = dalloc(s, &tmp, n);
+    const int rc = dreserve(s, &s->d_stage, n, s->cap_stage);
     if (rc != MSM_OK) return rc;
     AtomSet& z = s->set[s->scur];
     if (comp_pos >= 0)
-        msm::launch_unsort_pos(s->pos[s->pcur], tmp, z.gid, n, comp_pos, s->stream);
+        msm::launch_unsort_pos(s->pos[s->pcur], s->d_stage, z.gid, n, comp_pos, s->stream);
     else
-        msm::launch_unsort_d(src, tmp, z.gid, n, s->stream);
-    hipError_t e = hipMemcpyAsync(host, tmp, n * sizeof(double), hipMemcpyDeviceToHost, s->stream);
-    if (e == hipSuccess) e = hipStreamSynchronize(s->stream);
-    dfree(&tmp);
-    if (e != hipSuccess) return set_err(s, MSM_ERR_HIP, hipGetErrorString(e));
+        msm::launch_unsort_d(src, s->d_stage, z.gid, n, s->stream);
+    const msm::CopyPart part{0, n * sizeof(double), host};
+    HIPCHK(s, pull(s, s->d_stage, part.bytes, &part, 1));
     return MSM_OK;
 }
 
@@ -1333,29 +1364,22 @@ int msm_put_atoms(msm_sim* s, const double* xp, const double* xp1) {
     if (!s->has_atoms) return set_err(s, MSM_ERR_STATE, "no atoms");
     const int n = s->n;
     if (n == 0 || (!xp && !xp1)) return MSM_OK;
-    const size_t na = s->n_alloc;
+    const size_t na = s->n_alloc, n3 = 3 * static_cast<size_t>(n);
     AtomSet& z = s->set[s->scur];
-    double* tmp = nullptr;
-    int rc = dalloc(s, &tmp, 3 * static_cast<size_t>(n));
+    const int rc = dreserve(s, &s->d_stage, n3, s->cap_stage);
     if (rc != MSM_OK) return rc;
-    hipError_t e = hipSuccess;
     if (xp) {
-        e = hipMemcpyAsync(tmp, xp, 3 * static_cast<size_t>(n) * sizeof(double),
-                           hipMemcpyHostToDevice, s->stream);
-        if (e == hipSuccess) msm::launch_sort_pos(tmp, s->pos[s->pcur], z.gid, n, s->stream);
+        HIPCHK(s, push(s, s->d_stage, xp, n3 * sizeof(double)));
+        msm::launch_sort_pos(s->d_stage, s->pos[s->pcur], z.gid, n, s->stream);
     }
-    if (e == hipSuccess && xp1) {
-        if (xp) e = hipStreamSynchronize(s->stream);  // tmp is reused
-        if (e == hipSuccess)
-            e = hipMemcpyAsync(tmp, xp1, 3 * static_cast<size_t>(n) * sizeof(double),
-                               hipMemcpyHostToDevice, s->stream);
-        for (int k = 0; e == hipSuccess && k < 3; ++k)
-            msm::launch_sort_d(tmp + k * static_cast<size_t>(n), z.v + k * na, z.gid, n,
+    if (xp1) {
+        if (xp) HIPCHK(s, hipStreamSynchronize(s->stream));  // the block is reused
+        HIPCHK(s, push(s, s->d_stage, xp1, n3 * sizeof(double)));
+        for (int k = 0; k < 3; ++k)
+            msm::launch_sort_d(s->d_stage + k * static_cast<size_t>(n), z.v + k * na, z.gid, n,
                                s->stream);
     }
-    if (e == hipSuccess) e = hipStreamSynchronize(s->stream);
-    dfree(&tmp);
-    if (e != hipSuccess) return set_err(s, MSM_ERR_HIP, hipGetErrorString(e));
+    HIPCHK(s, hipStreamSynchronize(s->stream));
     return MSM_OK;
 }
 
@@ -1420,16 +1444,14 @@ int msm_put_dis(msm_sim* s, const double* dis) {
     if (n == 0) return MSM_OK;
     const size_t na = s->n_alloc;
     AtomSet& z = s->set[s->scur];
-    double* tmp = nullptr;
-    int rc = dalloc(s, &tmp, 3 * static_cast<size_t>(n));
+    const size_t n3 = 3 * static_cast<size_t>(n);
+    const int rc = dreserve(s, &s->d_stage, n3, s->cap_stage);
     if (rc != MSM_OK) return rc;
-    hipError_t e = hipMemcpyAsync(tmp, dis, 3 * static_cast<size_t>(n) * sizeof(double),
-                                  hipMemcpyHostToDevice, s->stream);
-    for (int k = 0; e == hipSuccess && k < 3; ++k)
-        msm::launch_sort_d(tmp + k * static_cast<size_t>(n), z.dis + k * na, z.gid, n, s->stream);
-    if (e == hipSuccess) e = hipStreamSynchronize(s->stream);
-    dfree(&tmp);
-    if (e != hipSuccess) return set_err(s, MSM_ERR_HIP, hipGetErrorString(e));
+    HIPCHK(s, push(s, s->d_stage, dis, n3 * sizeof(double)));
+    for (int k = 0; k < 3; ++k)
+        msm::launch_sort_d(s->d_stage + k * static_cast<size_t>(n), z.dis + k * na, z.gid, n,
+                           s->stream);
+    HIPCHK(s, hipStreamSynchronize(s->stream));
     return MSM_OK;
 }
 
@@ -1451,10 +1473,15 @@ int msm_get_box_epot(msm_sim* s, double* ebox) {
     if (!s || !ebox) return MSM_ERR_ARG;
     (void)hipSetDevice(s->device);
     if (!s->has_list) return set_err(s, MSM_ERR_STATE, "no neighbour list");
+    const msm::CopyPart part{0, s->boxes.size() * sizeof(double), ebox};
+    if (part.bytes <= kSmallCopy) {  // the sums go straight to the pinned words
+        enqueue_box_sums(s, s->epot, 0, 1, reinterpret_cast<double*>(s->d_small));
+        HIPCHK(s, hipStreamSynchronize(s->stream));
+        std::memcpy(ebox, s->h_small, part.bytes);
+        return MSM_OK;
+    }
     enqueue_box_sums(s, s->epot, 0, 1, s->d_ebox);
-    HIPCHK(s, hipMemcpyAsync(ebox, s->d_ebox, s->boxes.size() * sizeof(double),
-                             hipMemcpyDeviceToHost, s->stream));
-    HIPCHK(s, hipStreamSynchronize(s->stream));
+    HIPCHK(s, pull(s, s->d_ebox, part.bytes, &part, 1));
     return MSM_OK;
 }
 
@@ -1475,22 +1502,17 @@ int msm_get_neighbors(msm_sim* s, int* kvois, int* indi, int ld) {
     const int n = s->n;
     if (ld < n) return set_err(s, MSM_ERR_ARG, "ld smaller than the atom count");
     if (n == 0) return MSM_OK;
-    int *kv = nullptr, *ix = nullptr;
-    int rc = dalloc(s, &kv, n);
-    if (rc == MSM_OK) rc = dalloc(s, &ix, static_cast<size_t>(ld) * s->mx);
-    if (rc != MSM_OK) {
-        dfree(&kv);
-        return rc;
-    }
+    int* kv = nullptr;
+    const size_t ni = static_cast<size_t>(ld) * s->mx;
+    int rc = dalloc(s, &kv, n + ni);
+    if (rc != MSM_OK) return rc;
+    int* ix = kv + n;
     msm::launch_unsort_list(s->kvois, s->indi, msm::kListRow, s->set[s->scur].gid, n, s->mx, kv, ix,
                             ld, s->stream);
-    hipError_t e = hipMemcpyAsync(kvois, kv, n * sizeof(int), hipMemcpyDeviceToHost, s->stream);
-    if (e == hipSuccess)
-        e = hipMemcpyAsync(indi, ix, static_cast<size_t>(ld) * s->mx * sizeof(int),
-                           hipMemcpyDeviceToHost, s->stream);
-    if (e == hipSuccess) e = hipStreamSynchronize(s->stream);
+    const msm::CopyPart part[2] = {{0, n * sizeof(int), kvois},
+                                   {n * sizeof(int), ni * sizeof(int), indi}};
+    const hipError_t e = pull(s, kv, (n + ni) * sizeof(int), part, 2);
     dfree(&kv);
-    dfree(&ix);
     if (e != hipSuccess) return set_err(s, MSM_ERR_HIP, hipGetErrorString(e));
     return MSM_OK;
 }
@@ -1529,27 +1551,20 @@ int msm_calc_ptensor(msm_sim* s, double* vtensor) {
     if (!vtensor) return set_err(s, MSM_ERR_ARG, "null argument");
     (void)hipSetDevice(s->device);
     const int nbox = static_cast<int>(s->boxes.size());
-    double* vir = nullptr;
-    double* sums = nullptr;
-    rc = dalloc(s, &vir, 6 * static_cast<size_t>(std::max(s->n, 1)));
-    if (rc == MSM_OK) rc = dalloc(s, &sums, 6 * static_cast<size_t>(nbox));
-    if (rc != MSM_OK) {
-        dfree(&vir);
-        return rc;
-    }
+    const size_t n6 = 6 * static_cast<size_t>(std::max(s->n, 1)), nsum = 6 * static_cast<size_t>(nbox);
+    rc = dreserve(s, &s->d_stage, n6 + nsum, s->cap_stage);
+    if (rc != MSM_OK) return rc;
+    double* vir = s->d_stage;
+    double* sums = s->d_stage + n6;
     clear_flags(s);
     enqueue_density(s);
     AtomsDev a = atoms_view(s, s->scur, s->pcur);
     msm::launch_virial(a, list_view(s), s->tab, s->boxes[0], s->d_boxes, multibox(s), vir,
                        s->stream);
     enqueue_box_sums(s, vir, s->n, 6, sums);
-    std::vector<double> h(6 * static_cast<size_t>(nbox));
-    hipError_t e = hipMemcpyAsync(h.data(), sums, h.size() * sizeof(double),
-                                  hipMemcpyDeviceToHost, s->stream);
-    if (e == hipSuccess) e = hipStreamSynchronize(s->stream);
-    dfree(&vir);
-    dfree(&sums);
-    if (e != hipSuccess) return set_err(s, MSM_ERR_HIP, hipGetErrorString(e));
+    std::vector<double> h(nsum);
+    const msm::CopyPart part{0, nsum * sizeof(double), h.data()};
+    HIPCHK(s, pull(s, sums, part.bytes, &part, 1));
     static const int row[6] = {0, 1, 2, 0, 0, 1}, col[6] = {0, 1, 2, 1, 2, 2};
     for (int b = 0; b < nbox; ++b)
         for (int c = 0; c < 6; ++c) {
@@ -1597,14 +1612,10 @@ int msm_calc_atomic_stress(msm_sim* s, double* avp) {
     (void)hipSetDevice(s->device);
     const int n = s->n;
     if (n == 0) return MSM_OK;
-    double* vir = nullptr;
-    double* out = nullptr;
-    rc = dalloc(s, &vir, 6 * static_cast<size_t>(n));
-    if (rc == MSM_OK) rc = dalloc(s, &out, 9 * static_cast<size_t>(n));
-    if (rc != MSM_OK) {
-        dfree(&vir);
-        return rc;
-    }
+    rc = dreserve(s, &s->d_stage, 15 * static_cast<size_t>(n), s->cap_stage);
+    if (rc != MSM_OK) return rc;
+    double* vir = s->d_stage;
+    double* out = vir + 6 * static_cast<size_t>(n);
     clear_flags(s);
     enqueue_density(s);
     AtomsDev a = atoms_view(s, s->scur, s->pcur);
@@ -1616,12 +1627,8 @@ int msm_calc_atomic_stress(msm_sim* s, double* avp) {
         msm::launch_virial(a, list_view(s), s->tab, s->boxes[0], s->d_boxes, multibox(s), vir,
                            s->stream);
     msm::launch_unsort_stress(vir, out, s->set[s->scur].gid, n, s->stream);
-    hipError_t e = hipMemcpyAsync(avp, out, 9 * static_cast<size_t>(n) * sizeof(double),
-                                  hipMemcpyDeviceToHost, s->stream);
-    if (e == hipSuccess) e = hipStreamSynchronize(s->stream);
-    dfree(&vir);
-    dfree(&out);
-    if (e != hipSuccess) return set_err(s, MSM_ERR_HIP, hipGetErrorString(e));
+    const msm::CopyPart part{0, 9 * static_cast<size_t>(n) * sizeof(double), avp};
+    HIPCHK(s, pull(s, out, part.bytes, &part, 1));
     return read_flags(s);
 }
 
@@ -1662,11 +1669,9 @@ int msm_check_timestep(msm_sim* s, double th, double mxd2, int* exceeded) {
         return set_err(s, MSM_ERR_ARG, "th > 0, mxd2 >= 0 and an output flag are required");
     (void)hipSetDevice(s->device);
     // the context's flag slot (no allocation per call: the step search calls this repeatedly)
-    int* flag = s->d_err + msm::kErrDt;
-    msm::launch_fill_int(flag, 0, 1, s->stream);
-    msm::launch_check_dt(atoms_view(s, s->scur, s->pcur), s->tab, th, mxd2, flag, s->stream);
-    HIPCHK(s, hipMemcpyAsync(s->h_err + msm::kErrDt, flag, sizeof(int), hipMemcpyDeviceToHost,
-                             s->stream));
+    s->h_err[msm::kErrDt] = 0;
+    msm::launch_check_dt(atoms_view(s, s->scur, s->pcur), s->tab, th, mxd2,
+                         s->d_err + msm::kErrDt, s->stream);
     HIPCHK(s, hipStreamSynchronize(s->stream));
     *exceeded = s->h_err[msm::kErrDt] ? 1 : 0;
     return MSM_OK;
@@ -2658,8 +2663,8 @@ int msm_fm_loss_grad(msm_sim* s, double* loss, double* coef_grad, int ld, int gr
     // everything up to the flags as one graph on repeated calls (one launch instead of about
     // twenty); the key holds what the captured kernels and copies bake in
     hipError_t ce = hipSuccess;
+    clear_flags(s);
     auto enqueue = [&]() {
-        clear_flags(s);
         {
             // the energy pass is the density pass too: it leaves F' in pos.w and, with a gradient,
             // keeps rho for the adjoint, whose own rho pass is skipped

@@ -141,7 +141,7 @@ __global__ __launch_bounds__(kNlSmallBlock) void k_nlist_small(
             scan(std::false_type{}, h + c_nix[s] + g.H[0] * (c_niy[s] + g.H[1] * c_niz[s]));
         int c = static_cast<int>((w - li) / kListRow);
         if (c > mx) {
-            atomicOr(&err[kErrOverflow], 1);
+            err[kErrOverflow] = 1;
             c = mx;
         }
         kvois[p] = c;
@@ -272,7 +272,7 @@ __global__ __launch_bounds__(kNlBlock, MT ? 4 : 8) void k_nlist_bricks(
             scan(std::false_type{}, h + c_nix[s] + g.H[0] * (c_niy[s] + g.H[1] * c_niz[s]));
         if (sub == 0) {
             if (c > mx) {
-                atomicOr(&err[kErrOverflow], 1);
+                err[kErrOverflow] = 1;
                 c = mx;
             }
             kvois[p] = c;
@@ -428,7 +428,7 @@ __global__ __launch_bounds__(kBlock) void k_density_bricks(const int* __restrict
                     const double sk = den0 / t.rhod + 1.0;
                     int kk = static_cast<int>(sk + 0.000001);
                     if (kk > t.nembd) {
-                        atomicOr(&err[kErrEmbd], 1);
+                        err[kErrEmbd] = 1;
                         kk = t.nembd;
                     }
                     const double4 m = t.m4[t.kembd[ti] * t.nembd2 + kk];

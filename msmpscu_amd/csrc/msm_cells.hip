@@ -45,7 +45,7 @@ __device__ __forceinline__ int cell_of(const double4* __restrict__ pos,
         in = in && ic[k] >= 0 && ic[k] < b.ncell[k];
     }
     if (in) return b.cell_off + cell_local(b, ic[0], ic[1], ic[2]);
-    atomicOr(&err[kErrOutOfBox], 1);
+    err[kErrOutOfBox] = 1;
     return ncell_total;
 }
 
@@ -400,7 +400,7 @@ __global__ __launch_bounds__(64 * kCellWaves, R > 6 ? 3 : R > 4 ? 5 : 8) void k_
         }
         if (lane < hn && (lane & ((1 << lgs) - 1)) == part) {
             if (kv > mx) {
-                atomicOr(&err[kErrOverflow], 1);
+                err[kErrOverflow] = 1;
                 kv = mx;
             }
             kvois[s0 + h0 + lane] = kv;

@@ -1,0 +1,162 @@
+// msm_copy.cpp -- pinned-ring copies (msm_copy.h).
+#include "msm_copy.h"
+
+#include <algorithm>
+#include <atomic>
+#include <cstring>
+#include <mutex>
+#include <thread>
+
+namespace msm {
+
+namespace {
+
+struct Ring {
+    std::mutex life;          // users, base, ev
+    std::mutex use;           // one transfer at a time
+    int users = 0;
+    char* base = nullptr;
+    hipEvent_t ev[kCopySlots] = {};
+};
+
+constexpr int kMaxDevices = 64;
+
+Ring* ring_of(int device) {
+    static Ring rings[kMaxDevices];
+    return device >= 0 && device < kMaxDevices ? &rings[device] : nullptr;
+}
+
+void drop(Ring& r) {
+    for (hipEvent_t& e : r.ev) {
+        if (e) (void)hipEventDestroy(e);
+        e = nullptr;
+    }
+    if (r.base) (void)hipHostFree(r.base);
+    r.base = nullptr;
+}
+
+// Runs work(slot) on the calling thread (slot 0) and up to extra others; a thread that cannot be
+// had is one fewer.
+template <typename F>
+void on_threads(int extra, F&& work) {
+    std::thread th[kCopySlots];
+    int n = 0;
+    for (; n < extra; ++n) {
+        try {
+            th[n] = std::thread(work, n + 1);
+        } catch (...) {
+            break;
+        }
+    }
+    work(0);
+    for (int k = 0; k < n; ++k) th[k].join();
+}
+
+// Chunk size and extra threads: a thread for every half megabyte.
+void shape(size_t total, size_t& chunk, int& extra) {
+    const size_t want = (total + (kCopySlotBytes / 2) - 1) / (kCopySlotBytes / 2);
+    const int threads = static_cast<int>(std::min<size_t>(std::max<size_t>(want, 1), kCopySlots));
+    extra = threads - 1;
+    chunk = std::min(kCopySlotBytes, (((total + threads - 1) / threads) + 4095) & ~size_t(4095));
+}
+
+}  // namespace
+
+hipError_t copy_ring_acquire(int device) {
+    Ring* r = ring_of(device);
+    if (!r) return hipErrorInvalidDevice;
+    std::lock_guard<std::mutex> g(r->life);
+    if (r->users == 0) {
+        hipError_t e = hipHostMalloc(reinterpret_cast<void**>(&r->base),
+                                     kCopySlots * kCopySlotBytes);
+        for (int k = 0; k < kCopySlots && e == hipSuccess; ++k)
+            e = hipEventCreateWithFlags(&r->ev[k], hipEventDisableTiming);
+        if (e != hipSuccess) {
+            drop(*r);
+            return e;
+        }
+    }
+    ++r->users;
+    return hipSuccess;
+}
+
+void copy_ring_release(int device) {
+    Ring* r = ring_of(device);
+    if (!r) return;
+    std::lock_guard<std::mutex> g(r->life);
+    if (r->users > 0 && --r->users == 0) drop(*r);
+}
+
+hipError_t copy_to_host(int device, const void* base, size_t total, const CopyPart* parts,
+                        int nparts, hipStream_t stream) {
+    Ring* r = ring_of(device);
+    if (!r || total == 0) return r ? hipStreamSynchronize(stream) : hipErrorInvalidDevice;
+    // the stream's earlier work ends before the ring is taken, for other streams to use it meanwhile
+    const hipError_t idle = hipStreamSynchronize(stream);
+    if (idle != hipSuccess) return idle;
+    std::lock_guard<std::mutex> g(r->use);
+    size_t chunk;
+    int extra;
+    shape(total, chunk, extra);
+    std::atomic<size_t> next{0};
+    std::atomic<int> err{hipSuccess};
+    on_threads(extra, [&](int slot) {
+        if (slot > 0 && hipSetDevice(device) != hipSuccess) return;
+        char* pin = r->base + slot * kCopySlotBytes;
+        for (;;) {
+            const size_t a = next.fetch_add(chunk);
+            if (a >= total || err.load() != hipSuccess) return;
+            const size_t b = std::min(a + chunk, total);
+            hipError_t e = hipMemcpyAsync(pin, static_cast<const char*>(base) + a, b - a,
+                                          hipMemcpyDeviceToHost, stream);
+            if (e == hipSuccess) e = hipEventRecord(r->ev[slot], stream);
+            if (e == hipSuccess) e = hipEventSynchronize(r->ev[slot]);
+            if (e != hipSuccess) {
+                err.store(e);
+                return;
+            }
+            for (int k = 0; k < nparts; ++k) {
+                const size_t lo = std::max(a, parts[k].offset),
+                             hi = std::min(b, parts[k].offset + parts[k].bytes);
+                if (lo < hi)
+                    std::memcpy(static_cast<char*>(parts[k].host) + (lo - parts[k].offset),
+                                pin + (lo - a), hi - lo);
+            }
+        }
+    });
+    return static_cast<hipError_t>(err.load());
+}
+
+hipError_t copy_to_device(int device, void* dst, const void* host, size_t total,
+                          hipStream_t stream) {
+    Ring* r = ring_of(device);
+    if (!r) return hipErrorInvalidDevice;
+    if (total == 0) return hipSuccess;
+    std::lock_guard<std::mutex> g(r->use);
+    size_t chunk;
+    int extra;
+    shape(total, chunk, extra);
+    std::atomic<size_t> next{0};
+    std::atomic<int> err{hipSuccess};
+    on_threads(extra, [&](int slot) {
+        if (slot > 0 && hipSetDevice(device) != hipSuccess) return;
+        char* pin = r->base + slot * kCopySlotBytes;
+        for (;;) {
+            const size_t a = next.fetch_add(chunk);
+            if (a >= total || err.load() != hipSuccess) return;
+            const size_t b = std::min(a + chunk, total);
+            std::memcpy(pin, static_cast<const char*>(host) + a, b - a);
+            hipError_t e = hipMemcpyAsync(static_cast<char*>(dst) + a, pin, b - a,
+                                          hipMemcpyHostToDevice, stream);
+            if (e == hipSuccess) e = hipEventRecord(r->ev[slot], stream);
+            if (e == hipSuccess) e = hipEventSynchronize(r->ev[slot]);
+            if (e != hipSuccess) {
+                err.store(e);
+                return;
+            }
+        }
+    });
+    return static_cast<hipError_t>(err.load());
+}
+
+}  // namespace msm

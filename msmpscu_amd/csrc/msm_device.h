@@ -299,7 +299,7 @@ static __device__ void nlist_atom_global(int p, int lc, const BoxDev& b, const d
         }
     }
     if (cnt > mx) {
-        atomicOr(&err[kErrOverflow], 1);
+        err[kErrOverflow] = 1;
         cnt = mx;
     }
     kvois[p] = cnt;

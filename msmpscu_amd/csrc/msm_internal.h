@@ -21,6 +21,8 @@ namespace msm {
 constexpr int kMaxGroup = 16;
 constexpr int kBlock = 256;
 
+// The flags live in pinned host memory: a kernel that finds an error stores 1 there, the host clears
+// them before a call's launches and reads them after its synchronisation (no clear kernel, no copy).
 // kErrDt: flag of the time-step check (not an error; read by msm_check_timestep alone)
 enum ErrSlot { kErrOverflow = 0, kErrOutOfBox = 1, kErrEmbd = 2, kErrDt = 3, kErrSlots = 4 };
 
@@ -309,12 +311,17 @@ void launch_damp_step(const AtomsDev& a, const TabDev& t, const BoxDev& box0, co
 // max |epot - epot0| into *host (pinned), then epot0 = epot; work: two words, zero before and after.
 void launch_epot_maxdelta_host(const double* epot, double* epot0, int n, unsigned long long* work,
                                double* host, hipStream_t s);
+// The caller's-order arrays that the flags ask for, one after another in out: positions (3 n),
+// velocities (3 n), forces (3 n), displacements (3 n), status (n ints).
+constexpr int kOutX = 1, kOutV = 2, kOutF = 4, kOutD = 8, kOutS = 16;
+void launch_copy_out(const AtomsDev& a, const int* gid, int what, void* out, hipStream_t s);
+// bytes (a multiple of 4) from src to dst, either of them pinned host memory
+void launch_copy_words(const void* src, void* dst, size_t bytes, hipStream_t s);
 void launch_unsort_d(const double* src, double* dst, const int* gid, int n, hipStream_t s);
 void launch_sort_pos(const double* src, double4* dst, const int* gid, int n, hipStream_t s);
 void launch_sort_d(const double* src, double* dst, const int* gid, int n, hipStream_t s);
 // dst[p] += src[gid[p]] (a caller-order array added into the sorted order)
 void launch_add_sorted(const double* src, double* dst, const int* gid, int n, hipStream_t s);
-void launch_unsort_i(const int* src, int* dst, const int* gid, int n, hipStream_t s);
 void launch_unsort_pos(const double4* src, double* dst, const int* gid, int n, int comp,
                        hipStream_t s);
 void launch_unsort_list(const int* kvois, const int* indi, int stride, const int* gid, int n,

@@ -110,7 +110,7 @@ __global__ __launch_bounds__(kBlock) void k_density(AtomsDev a, ListDev l, TabDe
                 const double sk = den0 / t.rhod + 1.0;
                 int kk = static_cast<int>(sk + 0.000001);
                 if (kk > t.nembd) {
-                    atomicOr(&err[kErrEmbd], 1);
+                    err[kErrEmbd] = 1;
                     kk = t.nembd;
                 }
                 const double4 m = t.m4[t.kembd[ti] * t.nembd2 + kk];
@@ -278,7 +278,7 @@ __global__ __launch_bounds__(kBlock) void k_epot(AtomsDev a, ListDev l, TabDev t
             int kk = static_cast<int>(sk + 0.000001);
             if (kk < 0) kk = 0;
             if (kk > t.nembd) {
-                atomicOr(&err[kErrEmbd], 1);
+                err[kErrEmbd] = 1;
                 kk = t.nembd;
             }
             const double4 m = t.m4[t.kembd[a.ityp[i]] * t.nembd2 + kk];
@@ -469,7 +469,7 @@ __global__ void k_check_dt(AtomsDev a, TabDev t, double th, double h2s2, double 
         }
     }
     const unsigned long long b = __ballot(over);
-    if (b != 0ull && static_cast<int>(threadIdx.x & 63) == __ffsll(b) - 1) atomicOr(flag, 1);
+    if (b != 0ull && static_cast<int>(threadIdx.x & 63) == __ffsll(b) - 1) *flag = 1;
 }
 
 void launch_check_dt(const AtomsDev& a, const TabDev& t, double th, double mxd2, int* flag,
@@ -763,12 +763,53 @@ void launch_move3(const AtomsDev& a, P3 dx, const BoxDev& box0, const BoxDev* bo
 // copy-out helpers (sorted -> caller order), box totals, list statistics
 // --------------------------------------------------------------------------------------------
 
-__global__ void k_unsort_d(const double* __restrict__ src, double* __restrict__ dst,
-                           const int* __restrict__ gid, int n) {
+// The per-atom arrays of a copy-out in the caller's order, in one launch.
+__global__ void k_copy_out(AtomsDev a, const int* __restrict__ gid, int what,
+                           double* __restrict__ out) {
     const int p = blockIdx.x * blockDim.x + threadIdx.x;
-    if (p < n) dst[gid[p]] = src[p];
+    if (p >= a.n) return;
+    const size_t n = a.n;
+    double* o = out + gid[p];
+    if (what & kOutX) {
+        const double4 x = a.pos[p];
+        o[0] = x.x;
+        o[n] = x.y;
+        o[2 * n] = x.z;
+        o += 3 * n;
+    }
+    auto put3 = [&](const double* x, const double* y, const double* z) {
+        o[0] = x[p];
+        o[n] = y[p];
+        o[2 * n] = z[p];
+        o += 3 * n;
+    };
+    if (what & kOutV) put3(a.vx, a.vy, a.vz);
+    if (what & kOutF) put3(a.fx, a.fy, a.fz);
+    if (what & kOutD) put3(a.dx, a.dy, a.dz);
+    if (what & kOutS) {
+        const size_t off = o - out - gid[p];
+        reinterpret_cast<int*>(out + off)[gid[p]] = a.statu[p];
+    }
 }
-__global__ void k_unsort_i(const int* __restrict__ src, int* __restrict__ dst,
+
+__global__ void k_copy_words(const int* __restrict__ src, int* __restrict__ dst, int n) {
+    const int k = blockIdx.x * blockDim.x + threadIdx.x;
+    if (k < n) dst[k] = src[k];
+}
+
+void launch_copy_words(const void* src, void* dst, size_t bytes, hipStream_t s) {
+    const int n = static_cast<int>(bytes / 4);
+    hipLaunchKernelGGL(k_copy_words, dim3(grid_for(n)), dim3(kBlock), 0, s,
+                       static_cast<const int*>(src), static_cast<int*>(dst), n);
+}
+
+void launch_copy_out(const AtomsDev& a, const int* gid, int what, void* out, hipStream_t s) {
+    if (a.n > 0)
+        hipLaunchKernelGGL(k_copy_out, dim3(grid_for(a.n)), dim3(kBlock), 0, s, a, gid, what,
+                           static_cast<double*>(out));
+}
+
+__global__ void k_unsort_d(const double* __restrict__ src, double* __restrict__ dst,
                            const int* __restrict__ gid, int n) {
     const int p = blockIdx.x * blockDim.x + threadIdx.x;
     if (p < n) dst[gid[p]] = src[p];
@@ -836,9 +877,6 @@ void launch_unsort_stress(const double* vir, double* avp, const int* gid, int n,
 
 void launch_unsort_d(const double* src, double* dst, const int* gid, int n, hipStream_t s) {
     if (n > 0) hipLaunchKernelGGL(k_unsort_d, dim3(grid_for(n)), dim3(kBlock), 0, s, src, dst, gid, n);
-}
-void launch_unsort_i(const int* src, int* dst, const int* gid, int n, hipStream_t s) {
-    if (n > 0) hipLaunchKernelGGL(k_unsort_i, dim3(grid_for(n)), dim3(kBlock), 0, s, src, dst, gid, n);
 }
 void launch_unsort_pos(const double4* src, double* dst, const int* gid, int n, int comp,
                        hipStream_t s) {

@@ -96,7 +96,7 @@ __global__ __launch_bounds__(kBlock) void k_density_pair(AtomsDev a, ListDev l, 
                 const double sk = den0 / t.rhod + 1.0;
                 int kk = static_cast<int>(sk + 0.000001);
                 if (kk > t.nembd) {
-                    atomicOr(&err[kErrEmbd], 1);
+                    err[kErrEmbd] = 1;
                     kk = t.nembd;
                 }
                 const double4 m = t.m4[t.kembd[ti] * t.nembd2 + kk];

@@ -269,7 +269,7 @@ __device__ __forceinline__ void sb_density_round(int base, int nat, bool staged,
                 const double sk = den / t.rhod + 1.0;
                 int kk = static_cast<int>(sk + 0.000001);
                 if (kk > t.nembd) {
-                    atomicOr(&err[kErrEmbd], 1);
+                    err[kErrEmbd] = 1;
                     kk = t.nembd;
                 }
                 const double4 m = t.m4[t.kembd[ti] * t.nembd2 + kk];

@@ -193,7 +193,7 @@ __global__ __launch_bounds__(TL ? kLtMaxBlock : kBlock) void k_density_w(
                 const double sk = den / t.rhod + 1.0;
                 int kk = static_cast<int>(sk + 0.000001);
                 if (kk > t.nembd) {
-                    atomicOr(&err[kErrEmbd], 1);
+                    err[kErrEmbd] = 1;
                     kk = t.nembd;
                 }
                 const double4 m = t.m4[t.kembd[q.ti] * t.nembd2 + kk];

@@ -471,9 +471,9 @@ class DeviceMD:
     def calc_atomic_stress(self) -> np.ndarray:
         """Per-atom stress AVP(N, 9) in caller order (msm_calc_atomic_stress): components P11,
         P12, P13, P21, ..., P33 of sum_j s_a s_b FORTOT; Fortran-ordered (N, 9) array."""
-        v = np.zeros(9 * self.n)
-        check(lib().msm_calc_atomic_stress(self.h, dptr(v)), "msm_calc_atomic_stress", self.h)
-        return v.reshape(9, self.n).T.copy(order="F")
+        v = np.empty((self.n, 9), order="F")
+        check(lib().msm_calc_atomic_stress(self.h, dptr(v.T)), "msm_calc_atomic_stress", self.h)
+        return v
 
     def damping(self):
         check(lib().msm_damping(self.h), "msm_damping", self.h)
@@ -622,36 +622,31 @@ class DeviceMD:
     # ---- copy-out ----
     def get_atoms(self):
         n = self.n
-        xp = np.zeros(3 * n)
-        xp1 = np.zeros(3 * n)
-        fp = np.zeros(3 * n)
-        dis = np.zeros(3 * n)
-        st = np.zeros(n, dtype=np.int32)
-        check(lib().msm_get_atoms(self.h, dptr(xp), dptr(xp1), dptr(fp), iptr(st), dptr(dis)),
-              "msm_get_atoms", self.h)
-        f = lambda a: a.reshape(3, n).T.copy(order="F")  # noqa: E731
-        return f(xp), f(xp1), f(fp), st, f(dis)
+        xp, xp1, fp, dis = (np.empty((n, 3), order="F") for _ in range(4))
+        st = np.empty(n, dtype=np.int32)
+        check(lib().msm_get_atoms(self.h, dptr(xp.T), dptr(xp1.T), dptr(fp.T), iptr(st),
+                                  dptr(dis.T)), "msm_get_atoms", self.h)
+        return xp, xp1, fp, st, dis
 
     def get_forces(self) -> np.ndarray:
         """FP (N, 3) in the caller's order alone (msm_get_atoms with the other outputs NULL)."""
-        n = self.n
-        fp = np.zeros(3 * n)
-        check(lib().msm_get_atoms(self.h, None, None, dptr(fp), None, None), "msm_get_atoms",
+        fp = np.empty((self.n, 3), order="F")
+        check(lib().msm_get_atoms(self.h, None, None, dptr(fp.T), None, None), "msm_get_atoms",
               self.h)
-        return fp.reshape(3, n).T.copy(order="F")
+        return fp
 
     def get_den(self) -> np.ndarray:
-        d = np.zeros(self.n)
+        d = np.empty(self.n)
         check(lib().msm_get_den(self.h, dptr(d)), "msm_get_den", self.h)
         return d
 
     def get_epot(self) -> np.ndarray:
-        d = np.zeros(self.n)
+        d = np.empty(self.n)
         check(lib().msm_get_epot(self.h, dptr(d)), "msm_get_epot", self.h)
         return d
 
     def get_box_epot(self) -> np.ndarray:
-        d = np.zeros(self.nbox)
+        d = np.empty(self.nbox)
         check(lib().msm_get_box_epot(self.h, dptr(d)), "msm_get_box_epot", self.h)
         return d
 
