@@ -42,12 +42,21 @@ __device__ __forceinline__ double atom_sum(double v) {
     return v;
 }
 
-// A pointer that is the same in every lane, in scalar registers.
-__device__ __forceinline__ const int* uniform(const int* p) {
+// A pointer to global memory that is the same in every lane, in scalar registers.  The address
+// space is spelled out: from a pointer put together of integers the compiler would make flat loads,
+// which count as LDS accesses too, and the next use of a knot would wait for the indices in flight.
+using GlobalInts = const __attribute__((address_space(1))) int*;
+
+__device__ __forceinline__ GlobalInts uniform(const int* p) {
     const unsigned long long a = reinterpret_cast<unsigned long long>(p);
     const unsigned lo = __builtin_amdgcn_readfirstlane(static_cast<unsigned>(a));
     const unsigned hi = __builtin_amdgcn_readfirstlane(static_cast<unsigned>(a >> 32));
-    return reinterpret_cast<const int*>((static_cast<unsigned long long>(hi) << 32) | lo);
+    return reinterpret_cast<GlobalInts>((static_cast<unsigned long long>(hi) << 32) | lo);
+}
+
+__device__ __forceinline__ int slot_at(GlobalInts p, unsigned off) {
+    return *reinterpret_cast<GlobalInts>(
+        reinterpret_cast<const __attribute__((address_space(1))) char*>(p) + off);
 }
 
 constexpr int ilog2(int v) { return v <= 1 ? 0 : 1 + ilog2(v / 2); }
@@ -58,7 +67,7 @@ constexpr int group_f(int) { return 3; }
 
 // What a lane needs of its unit.
 struct Lane {
-    const int* blk;   // list block of the unit's atoms (uniform)
+    GlobalInts blk;   // list block of the unit's atoms (uniform)
     unsigned lo;      // byte offset of the lane's first slot in it
     unsigned ib;      // atom index
     int kv;           // list length (0: inactive)
@@ -95,7 +104,7 @@ __device__ __forceinline__ bool inner(const BoxDev& b, double m, double x, doubl
 }
 
 __device__ __forceinline__ int slot_index(const Lane& q, int s, int shift) {
-    return at(q.blk, q.lo + (static_cast<unsigned>(s) << shift));
+    return slot_at(q.blk, q.lo + (static_cast<unsigned>(s) << shift));
 }
 
 // Knots: from the LDS window (TL = 1: rows of w.w knots from knot w.k0) or from global memory.

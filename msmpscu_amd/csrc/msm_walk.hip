@@ -158,7 +158,7 @@ __global__ __launch_bounds__(TL ? kLtMaxBlock : kBlock) void k_density_w(
         q.ti = MT ? at(a.ityp, q.ib * 4u) : 0;
 #pragma unroll
         for (int k = 0; k < G; ++k)
-            js[k] = at(q.blk, row + static_cast<unsigned>(min(sub + k * L, l.mx - 1)) * 256u);
+            js[k] = slot_at(q.blk, row + static_cast<unsigned>(min(sub + k * L, l.mx - 1)) * 256u);
         const BoxDev& b = box_of<MB>(box0, boxes, a.boxid, static_cast<int>(q.ib));
         const bool active = have && (st & STATU_ACTIVE) == STATU_ACTIVE;
         q.kv = active ? kv : 0;
@@ -253,7 +253,7 @@ __global__ __launch_bounds__(TL ? kLtMaxBlock : kBlock) void k_force_w(
         q.ti = MT ? at(a.ityp, q.ib * 4u) : 0;
 #pragma unroll
         for (int k = 0; k < G; ++k)
-            js[k] = at(q.blk, row + static_cast<unsigned>(min(sub + k * L, l.mx - 1)) * 256u);
+            js[k] = slot_at(q.blk, row + static_cast<unsigned>(min(sub + k * L, l.mx - 1)) * 256u);
         AtomState as;
         if constexpr (MODE >= 1)
             if (sub == 0) load_atom_state(a, sp, AtomIx{q.ib}, as);

@@ -135,7 +135,7 @@ __global__ __launch_bounds__(TL ? kLtMaxBlock : kBlock) void k_energy_w(
         q.ti = MT ? at(a.ityp, q.ib * 4u) : 0;
 #pragma unroll
         for (int k = 0; k < G; ++k)
-            js[k] = at(q.blk, row + static_cast<unsigned>(min(sub + k * L, l.mx - 1)) * 256u);
+            js[k] = slot_at(q.blk, row + static_cast<unsigned>(min(sub + k * L, l.mx - 1)) * 256u);
         const BoxDev& b = box_of<MB>(box0, boxes, a.boxid, static_cast<int>(q.ib));
         const bool active = have && (st & STATU_ACTIVE) == STATU_ACTIVE;
         q.kv = active ? kv : 0;
@@ -231,7 +231,7 @@ __global__ __launch_bounds__(TL ? kLtMaxBlock : kBlock) void k_virial_w(
         q.ti = MT ? at(a.ityp, q.ib * 4u) : 0;
 #pragma unroll
         for (int k = 0; k < G; ++k)
-            js[k] = at(q.blk, row + static_cast<unsigned>(min(sub + k * L, l.mx - 1)) * 256u);
+            js[k] = slot_at(q.blk, row + static_cast<unsigned>(min(sub + k * L, l.mx - 1)) * 256u);
         const BoxDev& b = box_of<MB>(box0, boxes, a.boxid, static_cast<int>(q.ib));
         const bool active = have && (st & STATU_ACTIVE) == STATU_ACTIVE;
         q.kv = active ? kv : 0;
