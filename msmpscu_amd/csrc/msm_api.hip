@@ -1260,7 +1260,7 @@ int msm_set_atoms(msm_sim* s, int n, const double* xp, const double* xp1, const 
     if (rc == MSM_OK) rc = dalloc(s, &s->sb.arr, na);
     if (rc == MSM_OK) rc = dalloc(s, &s->kvois, na);
     const size_t icap = static_cast<size_t>(na) * s->mx;
-    if (rc == MSM_OK) rc = dalloc(s, &s->indi, icap);
+    if (rc == MSM_OK) rc = dalloc(s, &s->indi, icap + msm::kWalkSlack);
     // the staged passes issue a full chunk of slot loads past an atom's last slot
     if (rc == MSM_OK) rc = dalloc(s, &s->sidx, icap + msm::kSbSlack);
     if (rc == MSM_OK) rc = dalloc(s, &s->cidx, icap);

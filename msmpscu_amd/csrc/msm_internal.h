@@ -187,9 +187,11 @@ unsigned lt_persistent_grid(const void* k, int block, size_t lds, int wgs, int n
 int lt_lds_budget(int wgs);
 // List-walk passes (msm_walk.hip), for fewer than kWalkMaxAtoms atoms (32-bit byte offsets).
 constexpr int kWalkMaxAtoms = 1 << 27;
+constexpr size_t kWalkSlack = 2 * 64 * 96;  // ints after the list's last row
 struct WalkDev {  // one launch
     int k0, w, last;  // knot window: w knots a kind from knot k0; a pair's knot is at most k0 + last
     int kimg;         // knot from which on a pair may need the minimum image (0: always)
+    unsigned odd0, odd1;  // first odd knot of the window without / with the minimum image
     double margin;    // atoms further than this from the periodic faces are inner
     int units, sweep;
 };

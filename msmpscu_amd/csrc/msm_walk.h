@@ -3,6 +3,7 @@
 #pragma once
 
 #include <algorithm>
+#include <cmath>
 #include <type_traits>
 
 #include "msm_device.h"
@@ -155,32 +156,52 @@ struct Knots<0> {
 };
 
 // A pair's place in the table.  ok: inside the cutoff with its knots in the window (q is in
-// bounds either way); odd: the pair goes the side road.
+// bounds either way); odd: the pair goes the side road, which looks at it once more: those below
+// the window, those that may need the minimum image (IMG = 0) and, where the cutoff does not lie
+// within the table, those above it (one unsigned comparison for all three).
 struct Place {
-    double sk, inv_r, dk;
-    int kk, q;
+    double inv_r, dk;
+    int q;
     bool ok, odd;
 };
 
 template <int IMG>
 __device__ __forceinline__ Place place(const TabDev& t, const WalkDev& w, double r2) {
     Place p;
-    p.sk = table_coord(r2, t.csi, p.inv_r);
-    p.kk = static_cast<int>(p.sk);
-    p.dk = p.sk - p.kk;
-    const unsigned kd = static_cast<unsigned>(p.kk - w.k0);
-    const bool reg = kd <= static_cast<unsigned>(w.last), in = r2 <= t.ru2max;
-    const bool far = IMG == 0 && p.kk >= w.kimg;
+    const double sk = table_coord(r2, t.csi, p.inv_r);
+    const int kk = static_cast<int>(sk);
+    p.dk = sk - kk;  // contracts with sk's last product: the fraction without its rounding
+    const unsigned kd = static_cast<unsigned>(kk - w.k0);
     p.q = static_cast<int>(min(kd, static_cast<unsigned>(w.last)));
-    p.ok = reg && in && !far;
-    p.odd = (in && !reg) || far;
+    p.odd = kd >= (IMG ? w.odd1 : w.odd0);
+    p.ok = r2 <= t.ru2max && !p.odd;
     return p;
+}
+
+// The lanes in which p holds.
+__device__ __forceinline__ unsigned long long lanes_of(bool p) {
+    return __builtin_amdgcn_ballot_w64(p);
 }
 
 // Whether a lane's slot s is in the list.
 template <int L>
 __device__ __forceinline__ bool listed(const Lane& q, int s) {
     return s * L + q.sub < q.kv;
+}
+
+// The indices of a lane's slots s + G .. s + 2 G - 1.  Beyond the end of the list they are whatever
+// the memory holds (the list is allocated with kWalkSlack ints after its last row): slot_atom
+// replaces them where they would be used.
+template <int G, int LG>
+__device__ __forceinline__ void next_slots(const Lane& q, int s, int (&js)[G]) {
+    const unsigned o = q.lo + (static_cast<unsigned>(s + G) << (8 + LG));
+#pragma unroll
+    for (int u = 0; u < G; ++u) js[u] = slot_at(q.blk, o + (static_cast<unsigned>(u) << (8 + LG)));
+}
+
+template <int FULL, int L>
+__device__ __forceinline__ unsigned slot_atom(const Lane& q, int s, int j) {
+    return FULL || listed<L>(q, s) ? static_cast<unsigned>(j) : q.ib;
 }
 
 __device__ __forceinline__ void add_virial(double h, double sx, double sy, double sz,
@@ -246,13 +267,11 @@ __device__ __forceinline__ void force_slots(const AtomsDev& a, const TabDev& t, 
 #pragma unroll
     for (int u = 0; u < G; ++u) {
         if (!FULL && u > 0 && (s + u) * L >= q.kv) break;
-        pj[u] = at(a.pos, static_cast<unsigned>(js[u]) << 5);
-        tj[u] = MT ? at(a.ityp, static_cast<unsigned>(js[u]) << 2) : 0;
+        const unsigned j = slot_atom<FULL, L>(q, s + u, js[u]);
+        pj[u] = at(a.pos, j << 5);
+        tj[u] = MT ? at(a.ityp, j << 2) : 0;
     }
-    if constexpr (FULL) {
-#pragma unroll
-        for (int u = 0; u < G; ++u) js[u] = slot_index(q, min(s + G + u, q.last), 8 + LG);
-    }
+    if constexpr (FULL) next_slots<G, LG>(q, s, js);
     unsigned long long odd = 0;
 #pragma unroll
     for (int u = 0; u < G; ++u) {
@@ -281,7 +300,7 @@ __device__ __forceinline__ void force_slots(const AtomsDev& a, const TabDev& t, 
         fy = fy + ft * sy;
         fz = fz + ft * sz;
         if constexpr (V) add_virial(0.5 * ft, sx, sy, sz, vir);
-        odd |= __ballot(p.odd && valid);
+        odd |= lanes_of(p.odd && valid);
     }
     if (odd) force_odd<MT, IMG, LG, V>(a, t, w, b, q, s, G, pi, fx, fy, fz, vir);
 }
@@ -296,6 +315,15 @@ inline void window(const TabDev& t, long budget, int bytes, WalkDev& w) {
     w.last = t.ntab2 - 2 - w.k0;
 }
 
+// From which knot of the window on a pair is odd (place).  Within the table: every pair inside the
+// cutoff has its knots there.
+inline void odd_knots(const TabDev& t, WalkDev& w) {
+    const bool within = t.csi * std::sqrt(std::sqrt(t.ru2max)) < t.ntab2 - 1 - 1.0e-6;
+    const unsigned top = within ? 0x80000000u : static_cast<unsigned>(w.last) + 1u;
+    w.odd1 = top;
+    w.odd0 = std::min(top, static_cast<unsigned>(std::max(w.kimg - w.k0, 0)));
+}
+
 inline long walk_budget(const TabDev& t, int wgs) {
     return lt_lds_budget(wgs) - (t.ngroup > 1 ? 4 * kMaxGroup * kMaxGroup : 0);
 }
@@ -307,10 +335,12 @@ unsigned walk_launch(K k, const WalkPlan& pl, int bytes, int n, const TabDev& t,
     w.kimg = pl.kimg;
     w.margin = pl.margin;
     w.sweep = pl.sweep;
+    static_assert(kWalkSlack >= 2 * 64 * 96, "slots that a group may read past the list");
     w.units = (n + 64 / pl.lanes - 1) / (64 / pl.lanes);
     if (pl.tl) {
         threads = pl.block;
         window(t, walk_budget(t, pl.wgs), bytes, w);
+        odd_knots(t, w);
         lds = static_cast<size_t>(w.w) * (t.ngroup > 1 ? t.nkind : 1) * bytes;
         const int nwv = threads / 64;
         return lt_persistent_grid(reinterpret_cast<const void*>(k), threads, lds, pl.wgs,
@@ -321,6 +351,7 @@ unsigned walk_launch(K k, const WalkPlan& pl, int bytes, int n, const TabDev& t,
     w.k0 = 0;
     w.w = t.ntab2;
     w.last = t.ntab2 - 2;
+    odd_knots(t, w);
     return static_cast<unsigned>((w.units + kBlock / 64 - 1) / (kBlock / 64));
 }
 

@@ -7,8 +7,8 @@
 // n < kWalkMaxAtoms, whose records lie below 4 GB).
 //
 // Below about 10^5 atoms a pass is the length of one wave's chain of loads (state, indices, records,
-// knots) after about 4 us of launch; above, the issue of the pair loop and the rate of the L1's
-// line accesses (75 % and 67 % busy on a million W atoms) bound it together.  So
+// knots) after about 4 us of launch; above, the vector memory pipe (a record per pair: 1.1 line
+// accesses a clock and CU, the data return 97 % busy on a million W atoms, the VALU 55 %).  So
 //  - a unit whose atoms all lie further than the list radius from the periodic faces of their box
 //    ("inner": four fifths of a million-atom box) evaluates its pairs without the minimum image.
 //    The knot index tells a pair that might need it after all (its distance reaches half the
@@ -81,15 +81,12 @@ __device__ __forceinline__ double density_slots(const AtomsDev& a, const TabDev&
     for (int u = 0; u < G; ++u) {
         if (!FULL && u > 0 && (s + u) * L >= q.kv) break;
         // x, y, z only: another wave may be writing the neighbour's w
-        const unsigned o = static_cast<unsigned>(js[u]) << 5;
+        const unsigned j = slot_atom<FULL, L>(q, s + u, js[u]), o = j << 5;
         qxy[u] = *reinterpret_cast<const double2*>(&at(a.pos, o));
         qz[u] = at(a.pos, o).z;
-        tj[u] = MT ? at(a.ityp, static_cast<unsigned>(js[u]) << 2) : 0;
+        tj[u] = MT ? at(a.ityp, j << 2) : 0;
     }
-    if constexpr (FULL) {
-#pragma unroll
-        for (int u = 0; u < G; ++u) js[u] = slot_index(q, min(s + G + u, q.last), 8 + LG);
-    }
+    if constexpr (FULL) next_slots<G, LG>(q, s, js);
     unsigned long long odd = 0;
 #pragma unroll
     for (int u = 0; u < G; ++u) {
@@ -106,7 +103,7 @@ __device__ __forceinline__ double density_slots(const AtomsDev& a, const TabDev&
         kn.den(p.q + (MT ? s_row[q.ti * t.ngroup + tj[u]] : 0), v, dv);
         v = v + p.dk * dv;
         den = den + ((p.ok && valid) ? v : 0.0);
-        odd |= __ballot(p.odd && valid);
+        odd |= lanes_of(p.odd && valid);
     }
     if (odd) den = density_odd<MT, IMG, LG>(a, t, w, b, q, s, G, px, py, pz, den);
     return den;
@@ -149,8 +146,8 @@ __global__ __launch_bounds__(TL ? kLtMaxBlock : kBlock) void k_density_w(
         q.blk = uniform(l.indi + static_cast<size_t>(p0 >> 6) * l.mx * kListRow);
         const unsigned row = static_cast<unsigned>((p0 & 63) + pl) * 4u;
         q.lo = row + static_cast<unsigned>(sub) * 256u;
-        // the atom's loads in one batch, with the first group's slot indices (slots clamped below
-        // mx, masked by the list length once it is known)
+        // the atom's loads in one batch, with the first group's slot indices (masked by
+        // the list length once it is known)
         int js[G];
         const int st = at(a.statu, q.ib * 4u), kv = at(l.kvois, q.ib * 4u);
         const double2 pxy = *reinterpret_cast<const double2*>(&at(a.pos, q.ib * 32u));
@@ -158,7 +155,7 @@ __global__ __launch_bounds__(TL ? kLtMaxBlock : kBlock) void k_density_w(
         q.ti = MT ? at(a.ityp, q.ib * 4u) : 0;
 #pragma unroll
         for (int k = 0; k < G; ++k)
-            js[k] = slot_at(q.blk, row + static_cast<unsigned>(min(sub + k * L, l.mx - 1)) * 256u);
+            js[k] = slot_at(q.blk, row + static_cast<unsigned>(sub + k * L) * 256u);
         const BoxDev& b = box_of<MB>(box0, boxes, a.boxid, static_cast<int>(q.ib));
         const bool active = have && (st & STATU_ACTIVE) == STATU_ACTIVE;
         q.kv = active ? kv : 0;
@@ -167,8 +164,6 @@ __global__ __launch_bounds__(TL ? kLtMaxBlock : kBlock) void k_density_w(
         const bool fast = w.kimg > 0 && !__any(active && !inner(b, w.margin, pxy.x, pxy.y, pz));
         double den = 0.0;
         if (q.kv > 0) {
-#pragma unroll
-            for (int k = 0; k < G; ++k) js[k] = k <= q.last ? js[k] : static_cast<int>(q.ib);
             auto slots = [&](auto img) {
                 constexpr int IMG = decltype(img)::value;
                 int s = 0;
@@ -253,7 +248,7 @@ __global__ __launch_bounds__(TL ? kLtMaxBlock : kBlock) void k_force_w(
         q.ti = MT ? at(a.ityp, q.ib * 4u) : 0;
 #pragma unroll
         for (int k = 0; k < G; ++k)
-            js[k] = slot_at(q.blk, row + static_cast<unsigned>(min(sub + k * L, l.mx - 1)) * 256u);
+            js[k] = slot_at(q.blk, row + static_cast<unsigned>(sub + k * L) * 256u);
         AtomState as;
         if constexpr (MODE >= 1)
             if (sub == 0) load_atom_state(a, sp, AtomIx{q.ib}, as);
@@ -265,8 +260,6 @@ __global__ __launch_bounds__(TL ? kLtMaxBlock : kBlock) void k_force_w(
         const bool fast = w.kimg > 0 && !__any(active && !inner(b, w.margin, pi.x, pi.y, pi.z));
         double fx = 0.0, fy = 0.0, fz = 0.0, vir[6];
         if (q.kv > 0) {
-#pragma unroll
-            for (int k = 0; k < G; ++k) js[k] = k <= q.last ? js[k] : static_cast<int>(q.ib);
             auto slots = [&](auto img) {
                 constexpr int IMG = decltype(img)::value;
                 int s = 0;

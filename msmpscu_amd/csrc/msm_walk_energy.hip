@@ -57,15 +57,12 @@ __device__ __forceinline__ void energy_slots(const AtomsDev& a, const TabDev& t,
     for (int u = 0; u < G; ++u) {
         if (!FULL && u > 0 && (s + u) * L >= q.kv) break;
         // x, y, z only: another wave may be writing the neighbour's w
-        const unsigned o = static_cast<unsigned>(js[u]) << 5;
+        const unsigned j = slot_atom<FULL, L>(q, s + u, js[u]), o = j << 5;
         qxy[u] = *reinterpret_cast<const double2*>(&at(a.pos, o));
         qz[u] = at(a.pos, o).z;
-        tj[u] = MT ? at(a.ityp, static_cast<unsigned>(js[u]) << 2) : 0;
+        tj[u] = MT ? at(a.ityp, j << 2) : 0;
     }
-    if constexpr (FULL) {
-#pragma unroll
-        for (int u = 0; u < G; ++u) js[u] = slot_index(q, min(s + G + u, q.last), 8 + LG);
-    }
+    if constexpr (FULL) next_slots<G, LG>(q, s, js);
     unsigned long long odd = 0;
 #pragma unroll
     for (int u = 0; u < G; ++u) {
@@ -84,7 +81,7 @@ __device__ __forceinline__ void energy_slots(const AtomsDev& a, const TabDev& t,
         d = d + p.dk * dd;
         er = er + (use ? v : 0.0);
         den = den + (use ? d : 0.0);
-        odd |= __ballot(p.odd && (FULL || listed<L>(q, s + u)));
+        odd |= lanes_of(p.odd && (FULL || listed<L>(q, s + u)));
     }
     if (odd) energy_odd<MT, IMG, LG>(a, t, w, b, q, s, G, px, py, pz, er, den);
 }
@@ -135,7 +132,7 @@ __global__ __launch_bounds__(TL ? kLtMaxBlock : kBlock) void k_energy_w(
         q.ti = MT ? at(a.ityp, q.ib * 4u) : 0;
 #pragma unroll
         for (int k = 0; k < G; ++k)
-            js[k] = slot_at(q.blk, row + static_cast<unsigned>(min(sub + k * L, l.mx - 1)) * 256u);
+            js[k] = slot_at(q.blk, row + static_cast<unsigned>(sub + k * L) * 256u);
         const BoxDev& b = box_of<MB>(box0, boxes, a.boxid, static_cast<int>(q.ib));
         const bool active = have && (st & STATU_ACTIVE) == STATU_ACTIVE;
         q.kv = active ? kv : 0;
@@ -144,8 +141,6 @@ __global__ __launch_bounds__(TL ? kLtMaxBlock : kBlock) void k_energy_w(
         const bool fast = w.kimg > 0 && !__any(active && !inner(b, w.margin, pxy.x, pxy.y, pz));
         double er = 0.0, den = 0.0;
         if (q.kv > 0) {
-#pragma unroll
-            for (int k = 0; k < G; ++k) js[k] = k <= q.last ? js[k] : static_cast<int>(q.ib);
             auto slots = [&](auto img) {
                 constexpr int IMG = decltype(img)::value;
                 int s = 0;
@@ -231,7 +226,7 @@ __global__ __launch_bounds__(TL ? kLtMaxBlock : kBlock) void k_virial_w(
         q.ti = MT ? at(a.ityp, q.ib * 4u) : 0;
 #pragma unroll
         for (int k = 0; k < G; ++k)
-            js[k] = slot_at(q.blk, row + static_cast<unsigned>(min(sub + k * L, l.mx - 1)) * 256u);
+            js[k] = slot_at(q.blk, row + static_cast<unsigned>(sub + k * L) * 256u);
         const BoxDev& b = box_of<MB>(box0, boxes, a.boxid, static_cast<int>(q.ib));
         const bool active = have && (st & STATU_ACTIVE) == STATU_ACTIVE;
         q.kv = active ? kv : 0;
@@ -240,8 +235,6 @@ __global__ __launch_bounds__(TL ? kLtMaxBlock : kBlock) void k_virial_w(
         const bool fast = w.kimg > 0 && !__any(active && !inner(b, w.margin, pi.x, pi.y, pi.z));
         double fx = 0.0, fy = 0.0, fz = 0.0, p[6] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
         if (q.kv > 0) {
-#pragma unroll
-            for (int k = 0; k < G; ++k) js[k] = k <= q.last ? js[k] : static_cast<int>(q.ib);
             auto slots = [&](auto img) {
                 constexpr int IMG = decltype(img)::value;
                 int s = 0;
