@@ -309,10 +309,16 @@ void launch_correction(const AtomsDev& a, const TabDev& t, double h, hipStream_t
 // One step of the damped quench up to the predictor: [corrector of the step before,] damping,
 // predictor.
 void launch_damp_step(const AtomsDev& a, const TabDev& t, const BoxDev& box0, const BoxDev* boxes,
-                      int multibox, double h, int correct, hipStream_t s);
-// max |epot - epot0| into *host (pinned), then epot0 = epot; work: two words, zero before and after.
-void launch_epot_maxdelta_host(const double* epot, double* epot0, int n, unsigned long long* work,
-                               double* host, hipStream_t s);
+                      int multibox, double h, int correct, const unsigned long long* work,
+                      hipStream_t s);
+// The end of a step: max |epot - epot0| and whether it is mindele or less, to the host; then
+// epot0 = epot.  work: four words, zero before the first step.
+struct DampNote {  // pinned
+    double del;
+    int converged, steps;
+};
+void launch_damp_check(const double* epot, double* epot0, int n, double mindele,
+                       unsigned long long* work, DampNote* host, hipStream_t s);
 // The caller's-order arrays that the flags ask for, one after another in out: positions (3 n),
 // velocities (3 n), forces (3 n), displacements (3 n), status (n ints).
 constexpr int kOutX = 1, kOutV = 2, kOutF = 4, kOutD = 8, kOutS = 16;

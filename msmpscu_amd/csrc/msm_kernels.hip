@@ -307,13 +307,16 @@ void launch_epot(const AtomsDev& a, const ListDev& l, const TabDev& t, const Box
 // --------------------------------------------------------------------------------------------
 
 // DAMP: the damping of the quench in front of the predictor; CORR: in front of that, the corrector
-// of the step before with the same forces (k_correction, k_damping and k_predictor in one).
+// of the step before with the same forces (k_correction, k_damping and k_predictor in one), and
+// nothing at all once *stop is set (the quench has converged).
 template <int MB, int DAMP, int CORR>
 __global__ __launch_bounds__(kBlock) void k_predictor(AtomsDev a, TabDev t, BoxDev box0,
-                                                      const BoxDev* __restrict__ boxes, double h) {
+                                                      const BoxDev* __restrict__ boxes, double h,
+                                                      const unsigned long long* stop) {
 #pragma clang fp contract(off)
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= a.n) return;
+    if (DAMP && *stop) return;
     int stat = a.statu[i];
     const bool active = (stat & STATU_ACTIVE) == STATU_ACTIVE;
     if (!active && !DAMP) return;
@@ -387,22 +390,24 @@ void launch_predictor(const AtomsDev& a, const TabDev& t, const BoxDev& box0,
     if (a.n <= 0) return;
     if (multibox)
         hipLaunchKernelGGL((k_predictor<1, 0, 0>), dim3(grid_for(a.n)), dim3(kBlock), 0, s, a, t, box0,
-                           boxes, h);
+                           boxes, h, nullptr);
     else
         hipLaunchKernelGGL((k_predictor<0, 0, 0>), dim3(grid_for(a.n)), dim3(kBlock), 0, s, a, t, box0,
-                           boxes, h);
+                           boxes, h, nullptr);
 }
 
 void launch_damp_step(const AtomsDev& a, const TabDev& t, const BoxDev& box0, const BoxDev* boxes,
-                      int multibox, double h, int correct, hipStream_t s) {
+                      int multibox, double h, int correct, const unsigned long long* work,
+                      hipStream_t s) {
+    const unsigned long long* stop = work + 2;
     if (a.n <= 0) return;
     const dim3 g(grid_for(a.n)), b(kBlock);
     if (multibox) {
-        if (correct) hipLaunchKernelGGL((k_predictor<1, 1, 1>), g, b, 0, s, a, t, box0, boxes, h);
-        else         hipLaunchKernelGGL((k_predictor<1, 1, 0>), g, b, 0, s, a, t, box0, boxes, h);
+        if (correct) hipLaunchKernelGGL((k_predictor<1, 1, 1>), g, b, 0, s, a, t, box0, boxes, h, stop);
+        else         hipLaunchKernelGGL((k_predictor<1, 1, 0>), g, b, 0, s, a, t, box0, boxes, h, stop);
     } else {
-        if (correct) hipLaunchKernelGGL((k_predictor<0, 1, 1>), g, b, 0, s, a, t, box0, boxes, h);
-        else         hipLaunchKernelGGL((k_predictor<0, 1, 0>), g, b, 0, s, a, t, box0, boxes, h);
+        if (correct) hipLaunchKernelGGL((k_predictor<0, 1, 1>), g, b, 0, s, a, t, box0, boxes, h, stop);
+        else         hipLaunchKernelGGL((k_predictor<0, 1, 0>), g, b, 0, s, a, t, box0, boxes, h, stop);
     }
 }
 
@@ -577,14 +582,15 @@ void launch_epot_maxdelta(const double* epot, double* epot0, int n, unsigned lon
                            out);
 }
 
-// The same, written to pinned host memory by the last workgroup, which leaves the maximum and the
-// workgroup counter at zero for the next call (one launch in place of a clear, the reduction and a
-// copy).
-__global__ __launch_bounds__(kBlock) void k_epot_maxdelta_host(const double* __restrict__ epot,
-                                                               double* __restrict__ epot0, int n,
-                                                               unsigned long long* work,
-                                                               double* __restrict__ host) {
+// The same for a step of the quench, in work: {running maximum, workgroups done, converged, steps
+// done}.  The last workgroup tells the host, in pinned memory, and sets the converged word, on which
+// the steps queued behind do nothing.
+__global__ __launch_bounds__(kBlock) void k_damp_check(const double* __restrict__ epot,
+                                                       double* __restrict__ epot0, int n,
+                                                       double mindele, unsigned long long* work,
+                                                       DampNote* __restrict__ host) {
     __shared__ double lds[kBlock / 64];
+    if (work[2]) return;
     double d = 0.0;
     for (int i = blockIdx.x * kBlock + threadIdx.x; i < n; i += gridDim.x * kBlock) {
         const double v = epot[i];
@@ -600,16 +606,22 @@ __global__ __launch_bounds__(kBlock) void k_epot_maxdelta_host(const double* __r
     __threadfence();
     if (atomicAdd(&work[1], 1ull) + 1ull == gridDim.x) {
         __threadfence();
-        *host = __longlong_as_double(static_cast<long long>(atomicExch(&work[0], 0ull)));
+        const double del = __longlong_as_double(static_cast<long long>(atomicExch(&work[0], 0ull)));
+        const int done = static_cast<int>(++work[3]), conv = del <= mindele;
         atomicExch(&work[1], 0ull);
+        host->del = del;
+        host->converged = conv;
+        __threadfence_system();
+        __hip_atomic_store(&host->steps, done, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+        if (conv) atomicExch(&work[2], 1ull);  // (every workgroup has read it)
     }
 }
 
-void launch_epot_maxdelta_host(const double* epot, double* epot0, int n, unsigned long long* work,
-                               double* host, hipStream_t s) {
+void launch_damp_check(const double* epot, double* epot0, int n, double mindele,
+                       unsigned long long* work, DampNote* host, hipStream_t s) {
     if (n > 0)
-        hipLaunchKernelGGL(k_epot_maxdelta_host, dim3(std::min(grid_for(n), 256u)), dim3(kBlock), 0,
-                           s, epot, epot0, n, work, host);
+        hipLaunchKernelGGL(k_damp_check, dim3(std::min(grid_for(n), 256u)), dim3(kBlock), 0, s,
+                           epot, epot0, n, mindele, work, host);
 }
 
 // --------------------------------------------------------------------------------------------
