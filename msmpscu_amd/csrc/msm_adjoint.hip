@@ -67,7 +67,13 @@ __device__ __forceinline__ void adj_flush(const double* bins, const AdjDev& d, i
     }
 }
 
-__device__ __forceinline__ double pair_sum2(double v) { return v + __shfl_xor(v, 1, 64); }
+// Sum over the LN lanes of an atom.
+template <int LN>
+__device__ __forceinline__ double lane_sum(double v) {
+#pragma unroll
+    for (int m = 1; m < LN; m <<= 1) v = v + __shfl_xor(v, m, 64);
+    return v;
+}
 
 }  // namespace
 
@@ -87,6 +93,19 @@ __global__ void k_adj_gather(const double* __restrict__ dldf, const int* __restr
 template <int EAM>
 __device__ __forceinline__ void fprime(const TabDev& t, int ke, double rho, double& fp,
                                        double& dfp);
+
+// The list of an atom shared by LN lanes, kAdjGroup slots of a lane at a time: the records of a
+// group are in flight together, and the indices of the next with them.  LN is 2, or up to 8 where
+// two lanes an atom would leave compute units without a workgroup (adjoint_lanes).
+constexpr int kAdjGroup = 4;
+
+template <int LN>
+__device__ __forceinline__ void adj_slots(const ListDev& l, size_t base, int iw, int kv,
+                                          int (&js)[kAdjGroup]) {
+#pragma unroll
+    for (int u = 0; u < kAdjGroup; ++u)
+        js[u] = l.indi[base + static_cast<size_t>(min(iw + LN * u, kv - 1)) * l.stride];
+}
 
 // rho_k and F'_k (same arithmetic as the density pass; F' goes to pos.w as there).
 template <int MB, int EAM, int MT>
@@ -148,7 +167,7 @@ __device__ __forceinline__ void fprime(const TabDev& t, int ke, double rho, doub
 
 // Pair pass: FPOTR / FPOTB / POTR knot terms and lambda_k.  Bins: [FPOTR | FPOTB | POTR], each
 // nkind x ntab2, kind-major.
-template <int MB, int EAM, bool LDSB, int MT>
+template <int MB, int EAM, bool LDSB, int MT, int LN>
 __global__ __launch_bounds__(kAdjBlock) void k_adj_pairs(AtomsDev a, ListDev l, TabDev t,
                                                          BoxDev box0,
                                                          const BoxDev* __restrict__ boxes,
@@ -164,7 +183,7 @@ __global__ __launch_bounds__(kAdjBlock) void k_adj_pairs(AtomsDev a, ListDev l, 
     const double4* __restrict__ g4 = reinterpret_cast<const double4*>(d.g);
     for (int c = c0; c < c1; ++c) {
         const int gt = c * blockDim.x + threadIdx.x;
-        const int k = gt >> 1, sub = gt & 1;
+        const int k = gt / LN, sub = gt % LN;
         const bool have = k < a.n;
         const bool active = have && (a.statu[k] & STATU_ACTIVE) == STATU_ACTIVE;
         double lam = 0.0;
@@ -176,42 +195,51 @@ __global__ __launch_bounds__(kAdjBlock) void k_adj_pairs(AtomsDev a, ListDev l, 
             const double gb = d.gbox[MB ? a.boxid[k] : 0];
             const int kv = l.kvois[k];
             const int tk = MT ? a.ityp[k] : 0;
-            for (int iw = sub; iw < kv; iw += 2) {
-                const int j = l.indi[list_base(k, l.mx) + static_cast<size_t>(iw) * l.stride];
-                const double4 pj = a.pos[j];
-                const double sx = min_image(pk.x - pj.x, b.len[0], b.ilen[0]);
-                const double sy = min_image(pk.y - pj.y, b.len[1], b.ilen[1]);
-                const double sz = min_image(pk.z - pj.z, b.len[2], b.ilen[2]);
-                const double r2 = sx * sx + sy * sy + sz * sz;
-                if (!(r2 <= t.ru2max)) continue;
-                int kind = t.kpair[0], kind1 = t.kpair[0];
-                if constexpr (MT) {
-                    const int tj = a.ityp[j];
-                    kind = t.kpair[tk * t.ngroup + tj];
-                    kind1 = t.kpair[tj * t.ngroup + tk];
+            constexpr int G = kAdjGroup;
+            const size_t lb = list_base(k, l.mx);
+            int js[G];
+            if (sub < kv) adj_slots<LN>(l, lb, sub, kv, js);
+            for (int iw = sub; iw < kv; iw += LN * G) {
+                double4 pj[G], gj[G];
+                int tj[G];
+#pragma unroll
+                for (int u = 0; u < G; ++u) {
+                    pj[u] = a.pos[js[u]];
+                    gj[u] = g4[js[u]];
+                    tj[u] = MT ? a.ityp[js[u]] : 0;
                 }
-                double inv_r;
-                const double sk = table_coord(r2, t.csi, inv_r);
-                const int kk = min(static_cast<int>(sk), t.ntab2 - 2);
-                const double dk = sk - kk;
-                const double4 f = t.f4[kind * nt + kk];
-                const double bp = f.z + dk * f.w;
-                const double ak = gkx * sx + gky * sy + gkz * sz;
-                const double4 gj = g4[j];
-                const double aj = gj.x * sx + gj.y * sy + gj.z * sz;
-                const int row = MT ? kind * nt : 0;
-                bin_add(b_fr + row, kk, dk, ak * inv_r * inv_r);
-                if constexpr (MT) {
-                    bin_add(b_fb + row, kk, dk, ak * pk.w * inv_r);
-                    bin_add(b_fb + kind1 * nt, kk, dk, ak * pj.w * inv_r);
-                } else {
-                    bin_add(b_fb, kk, dk, ak * (pk.w + pj.w) * inv_r);
+                adj_slots<LN>(l, lb, iw + LN * G, kv, js);
+#pragma unroll
+                for (int u = 0; u < G; ++u) {
+                    const double sx = min_image(pk.x - pj[u].x, b.len[0], b.ilen[0]);
+                    const double sy = min_image(pk.y - pj[u].y, b.len[1], b.ilen[1]);
+                    const double sz = min_image(pk.z - pj[u].z, b.len[2], b.ilen[2]);
+                    const double r2 = sx * sx + sy * sy + sz * sz;
+                    if (iw + LN * u >= kv || !(r2 <= t.ru2max)) continue;
+                    const int kind = t.kpair[MT ? tk * t.ngroup + tj[u] : 0];
+                    const int kind1 = t.kpair[MT ? tj[u] * t.ngroup + tk : 0];
+                    double inv_r;
+                    const double sk = table_coord(r2, t.csi, inv_r);
+                    const int kk = min(static_cast<int>(sk), t.ntab2 - 2);
+                    const double dk = sk - kk;
+                    const double4 f = t.f4[kind * nt + kk];
+                    const double bp = f.z + dk * f.w;
+                    const double ak = gkx * sx + gky * sy + gkz * sz;
+                    const double aj = gj[u].x * sx + gj[u].y * sy + gj[u].z * sz;
+                    const int row = MT ? kind * nt : 0;
+                    bin_add(b_fr + row, kk, dk, ak * inv_r * inv_r);
+                    if constexpr (MT) {
+                        bin_add(b_fb + row, kk, dk, ak * pk.w * inv_r);
+                        bin_add(b_fb + kind1 * nt, kk, dk, ak * pj[u].w * inv_r);
+                    } else {
+                        bin_add(b_fb, kk, dk, ak * (pk.w + pj[u].w) * inv_r);
+                    }
+                    bin_add(b_pr + row, kk, dk, gb * inv_r);
+                    lam = lam + (ak - aj) * bp * inv_r;
                 }
-                bin_add(b_pr + row, kk, dk, gb * inv_r);
-                lam = lam + (ak - aj) * bp * inv_r;
             }
         }
-        lam = pair_sum2(lam);
+        lam = lane_sum<LN>(lam);
         if (have && sub == 0) d.lam[k] = active ? lam : 0.0;
     }
     adj_flush<LDSB>(bins, d, 3 * nkt);
@@ -219,7 +247,7 @@ __global__ __launch_bounds__(kAdjBlock) void k_adj_pairs(AtomsDev a, ListDev l, 
 
 // Density pass: mu_k, POTB knot terms and the embedding knot terms.  Bins: [POTB | FEMBD |
 // DFEMBD] (nkind x ntab2, then nkind1 x nembd2 twice; the embedding parts only for EAM).
-template <int MB, int EAM, bool LDSB, int MT>
+template <int MB, int EAM, bool LDSB, int MT, int LN>
 __global__ __launch_bounds__(kAdjBlock) void k_adj_density(AtomsDev a, ListDev l, TabDev t,
                                                            BoxDev box0,
                                                            const BoxDev* __restrict__ boxes,
@@ -235,7 +263,7 @@ __global__ __launch_bounds__(kAdjBlock) void k_adj_density(AtomsDev a, ListDev l
     adj_range(nchunks, c0, c1);
     for (int c = c0; c < c1; ++c) {
         const int gt = c * blockDim.x + threadIdx.x;
-        const int k = gt >> 1, sub = gt & 1;
+        const int k = gt / LN, sub = gt % LN;
         const bool have = k < a.n;
         const bool active = have && (a.statu[k] & STATU_ACTIVE) == STATU_ACTIVE;
         if (!active) continue;
@@ -267,19 +295,32 @@ __global__ __launch_bounds__(kAdjBlock) void k_adj_density(AtomsDev a, ListDev l
         const BoxDev& b = box_of<MB>(box0, boxes, a.boxid, k);
         const double4 pk = a.pos[k];
         const int kv = l.kvois[k];
-        for (int iw = sub; iw < kv; iw += 2) {
-            const int j = l.indi[list_base(k, l.mx) + static_cast<size_t>(iw) * l.stride];
-            const double4 pj = a.pos[j];
-            const double sx = min_image(pk.x - pj.x, b.len[0], b.ilen[0]);
-            const double sy = min_image(pk.y - pj.y, b.len[1], b.ilen[1]);
-            const double sz = min_image(pk.z - pj.z, b.len[2], b.ilen[2]);
-            const double r2 = sx * sx + sy * sy + sz * sz;
-            if (!(r2 <= t.ru2max)) continue;
-            const int row = MT ? t.kpair[tk * t.ngroup + a.ityp[j]] * nt : 0;
-            double inv_r;
-            const double sk = table_coord(r2, t.csi, inv_r);
-            const int kk = min(static_cast<int>(sk), t.ntab2 - 2);
-            bin_add(b_pb + row, kk, sk - kk, mu);
+        constexpr int G = kAdjGroup;
+        const size_t lb = list_base(k, l.mx);
+        int js[G];
+        if (sub < kv) adj_slots<LN>(l, lb, sub, kv, js);
+        for (int iw = sub; iw < kv; iw += LN * G) {
+            double4 pj[G];
+            int tj[G];
+#pragma unroll
+            for (int u = 0; u < G; ++u) {
+                pj[u] = a.pos[js[u]];
+                tj[u] = MT ? a.ityp[js[u]] : 0;
+            }
+            adj_slots<LN>(l, lb, iw + LN * G, kv, js);
+#pragma unroll
+            for (int u = 0; u < G; ++u) {
+                const double sx = min_image(pk.x - pj[u].x, b.len[0], b.ilen[0]);
+                const double sy = min_image(pk.y - pj[u].y, b.len[1], b.ilen[1]);
+                const double sz = min_image(pk.z - pj[u].z, b.len[2], b.ilen[2]);
+                const double r2 = sx * sx + sy * sy + sz * sz;
+                if (iw + LN * u >= kv || !(r2 <= t.ru2max)) continue;
+                const int row = MT ? t.kpair[tk * t.ngroup + tj[u]] * nt : 0;
+                double inv_r;
+                const double sk = table_coord(r2, t.csi, inv_r);
+                const int kk = min(static_cast<int>(sk), t.ntab2 - 2);
+                bin_add(b_pb + row, kk, sk - kk, mu);
+            }
         }
     }
     adj_flush<LDSB>(bins, d, nkt + 2 * nke);
@@ -289,7 +330,7 @@ __global__ __launch_bounds__(kAdjBlock) void k_adj_density(AtomsDev a, ListDev l
 // workgroup takes kRedBins consecutive bins; its kRedSplit thread rows each sum the partials of
 // every kRedSplit-th workgroup (eight loads in flight per thread), and the rows' sums meet in a
 // fixed-shape tree in LDS.
-constexpr int kRedBins = 64, kRedSplit = 4;
+constexpr int kRedBins = 64, kRedSplit = 16;
 
 __global__ __launch_bounds__(kRedBins * kRedSplit) void k_adj_reduce(
     const double* __restrict__ part, int nwg, size_t stride, int nbin, double* __restrict__ out) {
@@ -339,8 +380,19 @@ int adj_cus() {
 
 }  // namespace
 
+// Lanes per atom: enough for a workgroup of 1024 on every compute unit, 2 to 8.  65,536 W atoms with
+// 2 lanes (128 workgroups) / 4 lanes (256): pair pass 30.1 / 20.6 us,
+// density pass 21.6 / 15.9.
+static int adjoint_lanes(int n) {
+    int ln = 2;
+    while (ln < 8 && static_cast<long long>(n) * ln < static_cast<long long>(adj_cus()) * kAdjBlock)
+        ln *= 2;
+    return ln;
+}
+
 int adjoint_workgroups(int n) {
-    const int nchunks = static_cast<int>((2LL * n + kAdjBlock - 1) / kAdjBlock);
+    const int nchunks =
+        static_cast<int>((static_cast<long long>(adjoint_lanes(n)) * n + kAdjBlock - 1) / kAdjBlock);
     const int cus = adj_cus();
     return nchunks < cus ? (nchunks > 0 ? nchunks : 1) : cus;
 }
@@ -356,7 +408,7 @@ void adjoint_bins(const TabDev& t, int& nb1, int& nb2) {
 
 void launch_adjoint(const AtomsDev& a, const ListDev& l, const TabDev& t, const BoxDev& box0,
                     const BoxDev* boxes, int multibox, const double* dldf, const int* gid,
-                    AdjDev d, double* out_pairs, double* out_dens, hipStream_t s,
+                    AdjDev d, double* out, hipStream_t s,
                     bool rho_ready) {
     if (a.n <= 0) return;
     const bool eam = t.pot_type != 0, mt = t.ngroup > 1;
@@ -372,7 +424,9 @@ void launch_adjoint(const AtomsDev& a, const ListDev& l, const TabDev& t, const 
     }
 #undef MSM_ARM
 #undef MSM_AR
-    const int nchunks = static_cast<int>((2LL * a.n + kAdjBlock - 1) / kAdjBlock);
+    const int ln = adjoint_lanes(a.n);
+    const int nchunks =
+        static_cast<int>((static_cast<long long>(ln) * a.n + kAdjBlock - 1) / kAdjBlock);
     const int nwg = adjoint_workgroups(a.n);
     const int lim = adj_lds_limit();
     int nb1, nb2;
@@ -381,8 +435,13 @@ void launch_adjoint(const AtomsDev& a, const ListDev& l, const TabDev& t, const 
     const bool l2 = static_cast<size_t>(nb2) * sizeof(double) <= static_cast<size_t>(lim);
     const size_t s1 = l1 ? nb1 * sizeof(double) : 0, s2 = l2 ? nb2 * sizeof(double) : 0;
 #define MSM_AP(MB, E, LB, M)                                                               \
-    hipLaunchKernelGGL((k_adj_pairs<MB, E, LB, M>), dim3(nwg), dim3(kAdjBlock), s1, s, a, l, \
-                       t, box0, boxes, d, nchunks)
+    do {                                                                                   \
+        auto k = ln == 2   ? k_adj_pairs<MB, E, LB, M, 2>                                  \
+                 : ln == 4 ? k_adj_pairs<MB, E, LB, M, 4>                                  \
+                           : k_adj_pairs<MB, E, LB, M, 8>;                                 \
+        hipLaunchKernelGGL(k, dim3(nwg), dim3(kAdjBlock), s1, s, a, l, t, box0, boxes, d,  \
+                           nchunks);                                                       \
+    } while (0)
 #define MSM_APL(MB, E)                                                              \
     do {                                                                            \
         if (mt) { if (l1) MSM_AP(MB, E, true, 1); else MSM_AP(MB, E, false, 1); }   \
@@ -392,12 +451,16 @@ void launch_adjoint(const AtomsDev& a, const ListDev& l, const TabDev& t, const 
     else          { if (eam) MSM_APL(0, 1); else MSM_APL(0, 0); }
 #undef MSM_APL
 #undef MSM_AP
-    const unsigned gr1 = static_cast<unsigned>((nb1 + kRedBins - 1) / kRedBins);
-    hipLaunchKernelGGL(k_adj_reduce, dim3(gr1), dim3(kRedBins * kRedSplit), 0, s, d.part, nwg,
-                       d.part_stride, nb1, out_pairs);
-#define MSM_AD(MB, E, LB, M)                                                                 \
-    hipLaunchKernelGGL((k_adj_density<MB, E, LB, M>), dim3(nwg), dim3(kAdjBlock), s2, s, a, l, \
-                       t, box0, boxes, d, nchunks)
+    double* const part = d.part;
+    d.part = part + nb1;  // the density pass's bins behind the pair pass's, for one reduction
+#define MSM_AD(MB, E, LB, M)                                                               \
+    do {                                                                                   \
+        auto k = ln == 2   ? k_adj_density<MB, E, LB, M, 2>                                \
+                 : ln == 4 ? k_adj_density<MB, E, LB, M, 4>                                \
+                           : k_adj_density<MB, E, LB, M, 8>;                               \
+        hipLaunchKernelGGL(k, dim3(nwg), dim3(kAdjBlock), s2, s, a, l, t, box0, boxes, d,  \
+                           nchunks);                                                       \
+    } while (0)
 #define MSM_ADL(MB, E)                                                              \
     do {                                                                            \
         if (mt) { if (l2) MSM_AD(MB, E, true, 1); else MSM_AD(MB, E, false, 1); }   \
@@ -407,9 +470,9 @@ void launch_adjoint(const AtomsDev& a, const ListDev& l, const TabDev& t, const 
     else          { if (eam) MSM_ADL(0, 1); else MSM_ADL(0, 0); }
 #undef MSM_ADL
 #undef MSM_AD
-    const unsigned gr2 = static_cast<unsigned>((nb2 + kRedBins - 1) / kRedBins);
-    hipLaunchKernelGGL(k_adj_reduce, dim3(gr2), dim3(kRedBins * kRedSplit), 0, s, d.part, nwg,
-                       d.part_stride, nb2, out_dens);
+    const unsigned gr = static_cast<unsigned>((nb1 + nb2 + kRedBins - 1) / kRedBins);
+    hipLaunchKernelGGL(k_adj_reduce, dim3(gr), dim3(kRedBins * kRedSplit), 0, s, part, nwg,
+                       d.part_stride, nb1 + nb2, out);
 }
 
 // --------------------------------------------------------------------------------------------

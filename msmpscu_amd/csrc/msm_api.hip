@@ -2447,7 +2447,7 @@ static int adj_reserve(msm_sim* s, size_t& nb1, size_t& nb2, size_t& stride) {
     msm::adjoint_bins(s->tab, nbin1, nbin2);
     nb1 = static_cast<size_t>(nbin1);
     nb2 = static_cast<size_t>(nbin2);
-    stride = std::max(nb1, nb2);
+    stride = nb1 + nb2;
     const size_t npart = stride * msm::adjoint_workgroups(n);
     if (s->adj_cap_n < static_cast<size_t>(s->n_alloc)) {
         dfree(&s->adj_dldf);
@@ -2485,7 +2485,7 @@ static int adj_reserve(msm_sim* s, size_t& nb1, size_t& nb2, size_t& stride) {
 
 // The adjoint passes on dL/dF (s->adj_dldf, caller order) and dL/dE (s->adj_gbox) into the bins
 // s->adj_out (pairs) and s->adj_out + nb1 (density).
-static void adj_launch(msm_sim* s, size_t nb1, size_t stride, bool rho_ready = false) {
+static void adj_launch(msm_sim* s, size_t stride, bool rho_ready = false) {
     msm::AdjDev d{};
     d.g = s->adj_g;
     d.gbox = s->adj_gbox;
@@ -2496,8 +2496,7 @@ static void adj_launch(msm_sim* s, size_t nb1, size_t stride, bool rho_ready = f
     AtomsDev a = atoms_view(s, s->scur, s->pcur);
     TimedScope ts(s, MSM_KCLASS_ADJOINT);
     msm::launch_adjoint(a, list_view(s), s->tab, s->boxes[0], s->d_boxes, multibox(s),
-                        s->adj_dldf, s->set[s->scur].gid, d, s->adj_out, s->adj_out + nb1,
-                        s->stream, rho_ready);
+                        s->adj_dldf, s->set[s->scur].gid, d, s->adj_out, s->stream, rho_ready);
 }
 
 int msm_adjoint(msm_sim* s, const double* dldf, const double* dlde, double* g_potr,
@@ -2519,7 +2518,7 @@ int msm_adjoint(msm_sim* s, const double* dldf, const double* dlde, double* g_po
                              hipMemcpyHostToDevice, s->stream));
     HIPCHK(s, hipMemcpyAsync(s->adj_gbox, dlde, nbox * sizeof(double), hipMemcpyHostToDevice,
                              s->stream));
-    adj_launch(s, nb1, stride);
+    adj_launch(s, stride);
     std::vector<double> h(nb1 + nb2);
     HIPCHK(s, hipMemcpyAsync(h.data(), s->adj_out, h.size() * sizeof(double),
                              hipMemcpyDeviceToHost, s->stream));
@@ -2677,7 +2676,9 @@ int msm_fm_loss_grad(msm_sim* s, double* loss, double* coef_grad, int ld, int gr
     if ((rc = fm_reserve(s, &s->fm_part, msm::fm_parts(n), s->fm_cap_part)) != MSM_OK) return rc;
     if ((rc = fm_reserve(s, &s->fm_loss, 1, s->fm_cap_loss)) != MSM_OK) return rc;
     const size_t m = coef_grad && !grad_on_device ? 3 * static_cast<size_t>(ld) : 0;
-    if (m && (rc = fm_reserve(s, &s->fm_grad, m, s->fm_cap_grad)) != MSM_OK) return rc;
+    // the loss in front of the gradient, so that one copy takes both
+    if (m && (rc = fm_reserve(s, &s->fm_grad, m + 1, s->fm_cap_grad)) != MSM_OK) return rc;
+    double* const dloss = m ? s->fm_grad : s->fm_loss;
     if ((rc = fm_reserve_host(s, m + 1)) != MSM_OK) return rc;
     // everything up to the flags as one graph on repeated calls (one launch instead of about
     // twenty); the key holds what the captured kernels and copies bake in
@@ -2696,18 +2697,15 @@ int msm_fm_loss_grad(msm_sim* s, double* loss, double* coef_grad, int ld, int gr
         const size_t na = s->n_alloc;
         msm::launch_fm_loss(z.f, z.f + na, z.f + 2 * na, z.gid, n, s->fm_ft, s->d_ebox, s->fm_et,
                             s->d_boxes, nbox, s->fm_w_e, s->adj_dldf, s->adj_gbox, s->fm_part,
-                            s->fm_loss, s->stream);
+                            dloss, s->stream);
         if (coef_grad) {
-            adj_launch(s, nb1, stride, true);
-            double* g = grad_on_device ? coef_grad : s->fm_grad;
+            adj_launch(s, stride, true);
+            double* g = grad_on_device ? coef_grad : s->fm_grad + 1;
             msm::launch_spline_grad(s->adj_out, s->adj_out + nb1, s->tab, ld, g, s->stream);
-            if (m && ce == hipSuccess)
-                ce = hipMemcpyAsync(s->fm_host + 1, g, m * sizeof(double), hipMemcpyDeviceToHost,
-                                    s->stream);
         }
         if (ce == hipSuccess)
-            ce = hipMemcpyAsync(s->fm_host, s->fm_loss, sizeof(double), hipMemcpyDeviceToHost,
-                                s->stream);
+            ce = hipMemcpyAsync(s->fm_host, dloss, (m + 1) * sizeof(double),
+                                hipMemcpyDeviceToHost, s->stream);
     };
     if (s->timing) {  // direct launches, each bracketed by events
         enqueue();

@@ -265,13 +265,13 @@ struct AdjDev {
 int adjoint_workgroups(int n);
 // Bin counts of the two adjoint passes (doubles): pairs nb1, density nb2.
 void adjoint_bins(const TabDev& t, int& nb1, int& nb2);
-// out_pairs: 3 x nkind x ntab2 knot gradients [FPOTR | FPOTB | POTR], each kind-major; out_dens:
+// out: 3 x nkind x ntab2 knot gradients [FPOTR | FPOTB | POTR], each kind-major, then
 // nkind x ntab2 + 2 x nkind1 x nembd2 [POTB | FEMBD | DFEMBD] (embedding parts for EAM only).
 // rho_ready: d.rho and pos.w (F') already hold the current values (the energy pass's rho_out and
 // the density pass), so the rho pass is skipped.
 void launch_adjoint(const AtomsDev& a, const ListDev& l, const TabDev& t, const BoxDev& box0,
                     const BoxDev* boxes, int multibox, const double* dldf, const int* gid,
-                    AdjDev d, double* out_pairs, double* out_dens, hipStream_t s,
+                    AdjDev d, double* out, hipStream_t s,
                     bool rho_ready = false);
 // Device-resident force matching (msm_adjoint.hip).  launch_spline_tables: the knot tables b2,
 // f4, e4 (and m4 for EAM) of one kind from the cubic B-spline coefficients coef (rows pair,
