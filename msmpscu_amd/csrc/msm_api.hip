@@ -690,7 +690,16 @@ bool walk_plan(const msm_sim* s, int force, msm::WalkPlan& p) {
     p.block = force ? s->lt.block_f : s->lt.block_d;
     p.wgs = force ? s->lt.wgs_f : s->lt.wgs_d;
     p.sweep = s->lt.sweep;
-    if (s->auto_pass) return size_plan(s, force, p);
+    if (s->auto_pass) {
+        if (!size_plan(s, force, p)) return false;
+        // Several boxes: every lane loads its atom's box record, so one lane an atom as soon as that
+        // fills the chip (64 boxes, 428,674 W atoms, density / force 43.8 / 56.2 us with 2 lanes,
+        // 40.8 / 50.4 with 1; 12 boxes, 242,498 atoms 28.5 / 35.7 and 27.8 / 33.1).  In one box the
+        // two are equal from 265,000 atoms on, below two are better (182,250: 21.6 / 25.1 and
+        // 24.5 / 28.5).
+        if (p.tl && p.lanes == 2 && multibox(s) && s->n >= 200000) p.lanes = 1;
+        return true;
+    }
     p.tl = 1;
     p.lanes = force ? lt_force_lanes(s) : fp;
     return s->table_lds && walk_lds_ok(s);
