@@ -298,11 +298,14 @@ int msm_list_stats(msm_sim* sim, long long* total, int* maxk);
  * HIP events around each launch and accumulates per-class device time. */
 #define MSM_OPT_TRACK_DIS     1
 #define MSM_OPT_KERNEL_TIMING 2
-#define MSM_OPT_NLIST_KERNEL  3  /* 0 (default): LDS-staged cell bricks, small or wide by cell
-                                    occupancy; 1: per-atom global scan; 2: small bricks (one lane
-                                    per atom); 3: wide bricks (several lanes per atom) */
+#define MSM_OPT_NLIST_KERNEL  3  /* 0 (default): a wave per cell (where the selected passes read
+                                    halo slots: cell bricks, small or wide by cell occupancy);
+                                    1: per-atom global scan; 2: small LDS-staged cell bricks (one
+                                    lane per atom); 3: wide bricks (several lanes per atom) */
 #define MSM_OPT_FORCE_PATH    4  /* density/force passes: 0 LDS bricks; 1, 2, 4, 8: global list
-                                    with that many lanes per atom (default 2); 3: two lanes per
+                                    with that many lanes per atom (2 is reported until it is
+                                    set; until one of the pass options is set, lanes and table
+                                    placement follow the number of atoms); 3: two lanes per
                                     atom, each 32-byte record gathered by a lane pair; 5: staged
                                     bricks (a brick's halo staged in LDS once, pairs read as halo
                                     slots; needs a list from the brick list kernels, else as 2) */

@@ -21,8 +21,8 @@
 //    its measurements are with the plan in msm_api.hip).
 // Density / force pass, HIP events (about 4 us of them overhead), against the two-lane passes with
 // whole-table windows: 2,000 W atoms 14.9 / 17.5 -> 6.2 / 8.1 us, 16,000 14.9 / 17.8 -> 8.5 / 10.1,
-// 137,000 25.7 / 31.0 -> 17.6 / 20.7, a million 78.7 / 99.5 -> 79.1 / 96.4; Cu-Ni 4,000 atoms
-// 45.0 / 52.4 -> 8.6 / 11.6, 442,000 158 / 195 -> 114 / 140.
+// 137,000 25.7 / 31.0 -> 17.8 / 21.4, a million 78.7 / 99.5 -> 75 / 93; Cu-Ni 4,000 atoms
+// 45.0 / 52.4 -> 8.6 / 11.6, 442,000 158 / 195 -> 121 / 146.
 // The arithmetic of a pair is that of the reference:
 //   T(KK) + DK * (T(KK+1) - T(KK)),  SK = sqrt(sqrt(r2)) * CSI, KK = int(SK), DK = SK - KK
 //   (MD_FS_ForceTable_GPU.F90 PRECALFOR/CALFORCE kernels).
