@@ -345,6 +345,13 @@ void resolve_timing(msm_sim* s) {
     s->pending.clear();
 }
 
+// Start of a call: the context's device, and no error left by an earlier call of this thread, so that
+// hipGetLastError speaks of this call's launches.
+void enter(const msm_sim* s) {
+    (void)hipSetDevice(s->device);
+    (void)hipGetLastError();
+}
+
 // Error flags (pinned host memory): cleared before the launches of a call, whose synchronisation at
 // its end leaves none of its kernels running.
 void clear_flags(msm_sim* s) {
@@ -353,14 +360,16 @@ void clear_flags(msm_sim* s) {
 
 // A device block (its parts in order, without gaps; total a multiple of 4) to the caller's arrays.
 // Up to 64 KB a kernel writes it into the context's pinned words, which spares the copy engine's
-// start-up; beyond, the ring of msm_copy.h.  Returns with the stream idle and the data in place.
+// start-up; beyond, the ring of msm_copy.h.  Returns with the stream idle and the data in place, or
+// the error of a launch of this call that was refused (the pinned words then hold an earlier copy).
 hipError_t pull(msm_sim* s, const void* base, size_t total, const msm::CopyPart* parts,
                 int nparts) {
+    if (total <= kSmallCopy) msm::launch_copy_words(base, s->d_small, total, s->stream);
+    hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return e;
     if (total > kSmallCopy)
         return msm::copy_to_host(s->device, base, total, parts, nparts, s->stream);
-    msm::launch_copy_words(base, s->d_small, total, s->stream);
-    const hipError_t e = hipStreamSynchronize(s->stream);
-    if (e != hipSuccess) return e;
+    if ((e = hipStreamSynchronize(s->stream)) != hipSuccess) return e;
     for (int k = 0; k < nparts; ++k)
         std::memcpy(parts[k].host, s->h_small + parts[k].offset, parts[k].bytes);
     return hipSuccess;
@@ -373,11 +382,17 @@ hipError_t push(msm_sim* s, void* dst, const void* host, size_t total) {
         return msm::copy_to_device(s->device, dst, host, total, s->stream);
     std::memcpy(s->h_small, host, total);
     msm::launch_copy_words(s->d_small, dst, total, s->stream);
-    return hipSuccess;
+    return hipGetLastError();
+}
+
+// The stream's work of a call is done and every launch of it was accepted.
+hipError_t finish(msm_sim* s) {
+    const hipError_t e = hipStreamSynchronize(s->stream);
+    return e != hipSuccess ? e : hipGetLastError();
 }
 
 int read_flags(msm_sim* s) {
-    HIPCHK(s, hipStreamSynchronize(s->stream));
+    HIPCHK(s, finish(s));
     resolve_timing(s);
     if (s->h_err[msm::kErrOutOfBox])
         return set_err(s, MSM_ERR_OUTOFBOX, "an active atom lies outside its box's cell grid");
@@ -848,17 +863,19 @@ int run_segment(msm_sim* s, int rebuild, int nsteps, int last, double h) {
         const int scur0 = s->scur, pcur0 = s->pcur;
         HIPCHK(s, hipStreamBeginCapture(s->stream, hipStreamCaptureModeThreadLocal));
         enqueue_segment(s, rebuild, nsteps, last, h);
+        const hipError_t le = hipGetLastError();  // a refused launch is missing from the graph
         hipGraph_t g = nullptr;
         HIPCHK(s, hipStreamEndCapture(s->stream, &g));
         hipGraphExec_t ge = nullptr;
-        hipError_t e = hipGraphInstantiate(&ge, g, nullptr, nullptr, 0);
+        hipError_t e = le;
+        if (e == hipSuccess) e = hipGraphInstantiate(&ge, g, nullptr, nullptr, 0);
         (void)hipGraphDestroy(g);
-        if (e != hipSuccess)
-            return set_err(s, MSM_ERR_HIP, std::string("hipGraphInstantiate: ") + hipGetErrorString(e));
-        it = s->graphs.emplace(key, ge).first;
         // the capture advanced the host state; rewind so the launch below replays from it
         s->scur = scur0;
         s->pcur = pcur0;
+        if (e != hipSuccess)
+            return set_err(s, MSM_ERR_HIP, std::string("hipGraphInstantiate: ") + hipGetErrorString(e));
+        it = s->graphs.emplace(key, ge).first;
     }
     HIPCHK(s, hipGraphLaunch(it->second, s->stream));
     advance_segment_state(s, rebuild, nsteps, last);
@@ -955,7 +972,7 @@ int msm_create(msm_sim** out, int device) {
 
 int msm_destroy(msm_sim* s) {
     if (!s) return MSM_OK;
-    (void)hipSetDevice(s->device);
+    enter(s);
     if (s->stream) (void)hipStreamSynchronize(s->stream);
     clear_graphs(s);
     free_atoms(s);
@@ -1012,7 +1029,7 @@ int msm_set_force_table(msm_sim* s, int pot_type, int ngroup, int nkind, int nta
                         double rhod, const int* kembd, const double* fembd,
                         const double* dfembd) {
     if (!s) return MSM_ERR_ARG;
-    (void)hipSetDevice(s->device);
+    enter(s);
     // the copies below are not ordered after table kernels still queued on the stream
     if (s->fm_pending) {
         HIPCHK(s, hipEventSynchronize(s->fm_ev));
@@ -1133,7 +1150,7 @@ int msm_set_force_table(msm_sim* s, int pot_type, int ngroup, int nkind, int nta
 int msm_set_ctrl(msm_sim* s, int ngroup, const double* ru, const double* nb_rm, int mxkvois,
                  const double* cm) {
     if (!s) return MSM_ERR_ARG;
-    (void)hipSetDevice(s->device);
+    enter(s);
     if (ngroup < 1 || ngroup > msm::kMaxGroup || !ru || !nb_rm || !cm || mxkvois < 1)
         return set_err(s, MSM_ERR_ARG, "bad control arguments");
     s->ngroup = ngroup;
@@ -1168,7 +1185,7 @@ int msm_set_ctrl(msm_sim* s, int ngroup, const double* ru, const double* nb_rm, 
 int msm_set_boxes(msm_sim* s, int nbox, const int* natoms, const double* lo, const double* len,
                   const int* ifpd) {
     if (!s) return MSM_ERR_ARG;
-    (void)hipSetDevice(s->device);
+    enter(s);
     if (!s->has_ctrl) return set_err(s, MSM_ERR_STATE, "set control parameters before boxes");
     if (nbox < 1 || !natoms || !lo || !len || !ifpd)
         return set_err(s, MSM_ERR_ARG, "bad box arguments");
@@ -1239,7 +1256,7 @@ int msm_set_boxes(msm_sim* s, int nbox, const int* natoms, const double* lo, con
 int msm_set_atoms(msm_sim* s, int n, const double* xp, const double* xp1, const int* ityp,
                   const int* statu) {
     if (!s) return MSM_ERR_ARG;
-    (void)hipSetDevice(s->device);
+    enter(s);
     if (!s->has_boxes) return set_err(s, MSM_ERR_STATE, "set boxes before atoms");
     if (n < 0 || (n > 0 && (!xp || !xp1 || !ityp || !statu)))
         return set_err(s, MSM_ERR_ARG, "bad atom arguments");
@@ -1322,7 +1339,7 @@ int msm_set_atoms(msm_sim* s, int n, const double* xp, const double* xp1, const 
 
 int msm_get_atoms(msm_sim* s, double* xp, double* xp1, double* fp, int* statu, double* dis) {
     if (!s) return MSM_ERR_ARG;
-    (void)hipSetDevice(s->device);
+    enter(s);
     if (!s->has_atoms) return set_err(s, MSM_ERR_STATE, "no atoms");
     const int n = s->n;
     if (n == 0) return MSM_OK;
@@ -1370,7 +1387,7 @@ static int pull_sorted_d(msm_sim* s, const double* src, int comp_pos, double* ho
 
 int msm_put_atoms(msm_sim* s, const double* xp, const double* xp1) {
     if (!s) return MSM_ERR_ARG;
-    (void)hipSetDevice(s->device);
+    enter(s);
     if (!s->has_atoms) return set_err(s, MSM_ERR_STATE, "no atoms");
     const int n = s->n;
     if (n == 0 || (!xp && !xp1)) return MSM_OK;
@@ -1383,13 +1400,13 @@ int msm_put_atoms(msm_sim* s, const double* xp, const double* xp1) {
         msm::launch_sort_pos(s->d_stage, s->pos[s->pcur], z.gid, n, s->stream);
     }
     if (xp1) {
-        if (xp) HIPCHK(s, hipStreamSynchronize(s->stream));  // the block is reused
+        if (xp) HIPCHK(s, finish(s));  // the block is reused
         HIPCHK(s, push(s, s->d_stage, xp1, n3 * sizeof(double)));
         for (int k = 0; k < 3; ++k)
             msm::launch_sort_d(s->d_stage + k * static_cast<size_t>(n), z.v + k * na, z.gid, n,
                                s->stream);
     }
-    HIPCHK(s, hipStreamSynchronize(s->stream));
+    HIPCHK(s, finish(s));
     return MSM_OK;
 }
 
@@ -1398,7 +1415,7 @@ int msm_put_atoms(msm_sim* s, const double* xp, const double* xp1) {
 static int add_caller_order(msm_sim* s, const double* src, int on_device, double* const* dst,
                             int ncomp, const char* what) {
     if (!s) return MSM_ERR_ARG;
-    (void)hipSetDevice(s->device);
+    enter(s);
     if (!s->has_atoms) return set_err(s, MSM_ERR_STATE, "no atoms");
     if (!src) return set_err(s, MSM_ERR_ARG, std::string(what) + ": null array");
     const int n = s->n;
@@ -1441,13 +1458,13 @@ int msm_add_epot(msm_sim* s, const double* eext, int on_device) {
     if (rc != MSM_OK || s->n == 0 || !s->has_list) return rc;
     // keep the box totals of msm_get_box_epot in step with the per-atom energies
     enqueue_box_sums(s, s->epot, 0, 1, s->d_ebox);
-    HIPCHK(s, hipStreamSynchronize(s->stream));
+    HIPCHK(s, finish(s));
     return MSM_OK;
 }
 
 int msm_put_dis(msm_sim* s, const double* dis) {
     if (!s) return MSM_ERR_ARG;
-    (void)hipSetDevice(s->device);
+    enter(s);
     if (!s->has_atoms) return set_err(s, MSM_ERR_STATE, "no atoms");
     if (!dis) return set_err(s, MSM_ERR_ARG, "msm_put_dis: null array");
     const int n = s->n;
@@ -1461,32 +1478,32 @@ int msm_put_dis(msm_sim* s, const double* dis) {
     for (int k = 0; k < 3; ++k)
         msm::launch_sort_d(s->d_stage + k * static_cast<size_t>(n), z.dis + k * na, z.gid, n,
                            s->stream);
-    HIPCHK(s, hipStreamSynchronize(s->stream));
+    HIPCHK(s, finish(s));
     return MSM_OK;
 }
 
 int msm_get_den(msm_sim* s, double* den) {
     if (!s || !den) return MSM_ERR_ARG;
-    (void)hipSetDevice(s->device);
+    enter(s);
     if (!s->has_atoms) return set_err(s, MSM_ERR_STATE, "no atoms");
     return pull_sorted_d(s, nullptr, 3, den);
 }
 
 int msm_get_epot(msm_sim* s, double* epot) {
     if (!s || !epot) return MSM_ERR_ARG;
-    (void)hipSetDevice(s->device);
+    enter(s);
     if (!s->has_atoms) return set_err(s, MSM_ERR_STATE, "no atoms");
     return pull_sorted_d(s, s->epot, -1, epot);
 }
 
 int msm_get_box_epot(msm_sim* s, double* ebox) {
     if (!s || !ebox) return MSM_ERR_ARG;
-    (void)hipSetDevice(s->device);
+    enter(s);
     if (!s->has_list) return set_err(s, MSM_ERR_STATE, "no neighbour list");
     const msm::CopyPart part{0, s->boxes.size() * sizeof(double), ebox};
     if (part.bytes <= kSmallCopy) {  // the sums go straight to the pinned words
         enqueue_box_sums(s, s->epot, 0, 1, reinterpret_cast<double*>(s->d_small));
-        HIPCHK(s, hipStreamSynchronize(s->stream));
+        HIPCHK(s, finish(s));
         std::memcpy(ebox, s->h_small, part.bytes);
         return MSM_OK;
     }
@@ -1498,7 +1515,7 @@ int msm_get_box_epot(msm_sim* s, double* ebox) {
 int msm_build_neighbors(msm_sim* s) {
     int rc = check_ready(s, false);
     if (rc != MSM_OK) return rc;
-    (void)hipSetDevice(s->device);
+    enter(s);
     clear_flags(s);
     enqueue_rebuild(s);
     s->has_list = true;
@@ -1507,7 +1524,7 @@ int msm_build_neighbors(msm_sim* s) {
 
 int msm_get_neighbors(msm_sim* s, int* kvois, int* indi, int ld) {
     if (!s || !kvois || !indi) return MSM_ERR_ARG;
-    (void)hipSetDevice(s->device);
+    enter(s);
     if (!s->has_list) return set_err(s, MSM_ERR_STATE, "no neighbour list");
     const int n = s->n;
     if (ld < n) return set_err(s, MSM_ERR_ARG, "ld smaller than the atom count");
@@ -1530,7 +1547,7 @@ int msm_get_neighbors(msm_sim* s, int* kvois, int* indi, int ld) {
 int msm_calc_force(msm_sim* s) {
     int rc = check_ready(s, true);
     if (rc != MSM_OK) return rc;
-    (void)hipSetDevice(s->device);
+    enter(s);
     clear_flags(s);
     enqueue_density(s);
     enqueue_force(s, 0, 1, 0.0);
@@ -1540,7 +1557,7 @@ int msm_calc_force(msm_sim* s) {
 int msm_calc_density(msm_sim* s) {
     int rc = check_ready(s, true);
     if (rc != MSM_OK) return rc;
-    (void)hipSetDevice(s->device);
+    enter(s);
     clear_flags(s);
     enqueue_density(s);
     return read_flags(s);
@@ -1549,7 +1566,7 @@ int msm_calc_density(msm_sim* s) {
 int msm_calc_epot(msm_sim* s) {
     int rc = check_ready(s, true);
     if (rc != MSM_OK) return rc;
-    (void)hipSetDevice(s->device);
+    enter(s);
     clear_flags(s);
     enqueue_epot(s);
     return read_flags(s);
@@ -1559,7 +1576,7 @@ int msm_calc_ptensor(msm_sim* s, double* vtensor) {
     int rc = check_ready(s, true);
     if (rc != MSM_OK) return rc;
     if (!vtensor) return set_err(s, MSM_ERR_ARG, "null argument");
-    (void)hipSetDevice(s->device);
+    enter(s);
     const int nbox = static_cast<int>(s->boxes.size());
     const size_t n6 = 6 * static_cast<size_t>(std::max(s->n, 1)), nsum = 6 * static_cast<size_t>(nbox);
     rc = dreserve(s, &s->d_stage, n6 + nsum, s->cap_stage);
@@ -1589,7 +1606,7 @@ int msm_calc_ptensor_noalloc(msm_sim* s, double* vtensor) {
     int rc = check_ready(s, true);
     if (rc != MSM_OK) return rc;
     if (!vtensor) return set_err(s, MSM_ERR_ARG, "null argument");
-    (void)hipSetDevice(s->device);
+    enter(s);
     double* ws = scratch_for(s->device);
     if (!ws) return set_err(s, MSM_ERR_STATE, "no workspace address for this device");
     const int nbox = static_cast<int>(s->boxes.size());
@@ -1619,7 +1636,7 @@ int msm_calc_atomic_stress(msm_sim* s, double* avp) {
     int rc = check_ready(s, true);
     if (rc != MSM_OK) return rc;
     if (!avp) return set_err(s, MSM_ERR_ARG, "null argument");
-    (void)hipSetDevice(s->device);
+    enter(s);
     const int n = s->n;
     if (n == 0) return MSM_OK;
     rc = dreserve(s, &s->d_stage, 15 * static_cast<size_t>(n), s->cap_stage);
@@ -1666,7 +1683,7 @@ static int box_kinetic(msm_sim* s, double* ek, std::vector<double>& sum, std::ve
 int msm_damping(msm_sim* s) {
     int rc = check_ready(s, false);
     if (rc != MSM_OK) return rc;
-    (void)hipSetDevice(s->device);
+    enter(s);
     msm::launch_damping(atoms_view(s, s->scur, s->pcur), s->stream);
     HIPCHK(s, hipStreamSynchronize(s->stream));
     return MSM_OK;
@@ -1677,12 +1694,12 @@ int msm_check_timestep(msm_sim* s, double th, double mxd2, int* exceeded) {
     if (rc != MSM_OK) return rc;
     if (!exceeded || !(th > 0.0) || !(mxd2 >= 0.0))
         return set_err(s, MSM_ERR_ARG, "th > 0, mxd2 >= 0 and an output flag are required");
-    (void)hipSetDevice(s->device);
+    enter(s);
     // the context's flag slot (no allocation per call: the step search calls this repeatedly)
     s->h_err[msm::kErrDt] = 0;
     msm::launch_check_dt(atoms_view(s, s->scur, s->pcur), s->tab, th, mxd2,
                          s->d_err + msm::kErrDt, s->stream);
-    HIPCHK(s, hipStreamSynchronize(s->stream));
+    HIPCHK(s, finish(s));
     *exceeded = s->h_err[msm::kErrDt] ? 1 : 0;
     return MSM_OK;
 }
@@ -1692,7 +1709,7 @@ int msm_thermalize(msm_sim* s, double temp, double kb, unsigned long long seed) 
     if (rc != MSM_OK) return rc;
     if (!(temp >= 0.0) || !(kb > 0.0))
         return set_err(s, MSM_ERR_ARG, "temperature >= 0 and kb > 0 are required");
-    (void)hipSetDevice(s->device);
+    enter(s);
     const size_t need = 4 * s->boxes.size();
     if (s->boxwork_cap < need) {
         dfree(&s->d_boxwork);
@@ -1712,7 +1729,7 @@ int msm_calc_ekin(msm_sim* s, double kb, double* ekin, double* tbox) {
     int rc = check_ready(s, true);
     if (rc != MSM_OK) return rc;
     if (!(kb > 0.0)) return set_err(s, MSM_ERR_ARG, "kb must be positive");
-    (void)hipSetDevice(s->device);
+    enter(s);
     double* ek = nullptr;
     if ((rc = dalloc(s, &ek, std::max(s->n, 1))) != MSM_OK) return rc;
     std::vector<double> sum, cnt;
@@ -1730,7 +1747,7 @@ int msm_scale_velocities(msm_sim* s, double temp, double kb) {
     int rc = check_ready(s, true);
     if (rc != MSM_OK) return rc;
     if (!(kb > 0.0) || !(temp >= 0.0)) return set_err(s, MSM_ERR_ARG, "kb > 0 and temp >= 0");
-    (void)hipSetDevice(s->device);
+    enter(s);
     const int nbox = static_cast<int>(s->boxes.size());
     double* ek = nullptr;
     double* scal = nullptr;
@@ -1765,7 +1782,7 @@ int msm_dyn_damp(msm_sim* s, int maxsteps, double mindele, double h, int* steps,
     int rc = check_ready(s, true);
     if (rc != MSM_OK) return rc;
     if (maxsteps < 0) return set_err(s, MSM_ERR_ARG, "maxsteps must be >= 0");
-    (void)hipSetDevice(s->device);
+    enter(s);
     const int n = s->n;
     rc = dreserve(s, &s->d_stage, 4, s->cap_stage);
     if (rc != MSM_OK) return rc;
@@ -1798,16 +1815,22 @@ int msm_dyn_damp(msm_sim* s, int maxsteps, double mindele, double h, int* steps,
         enqueue_force(s, 0, 1, 0.0);
         msm::launch_damp_check(s->epot, s->qwork, n, mindele, work, s->d_note, s->stream);
         ++queued;
-        // the wait ends with the step's note, or with the stream's work or an error
-        for (int spin = 1; note->steps + ahead < queued && !note->converged; ++spin)
+        if ((e = hipGetLastError()) != hipSuccess) break;
+        // the wait ends with the step's note or with the stream's work, which leaves the note behind
+        // it, or with an error
+        auto waiting = [&] { return note->steps + ahead < queued && !note->converged; };
+        for (int spin = 1; waiting(); ++spin)
             if (spin % 4096 == 0 && (e = hipStreamQuery(s->stream)) != hipErrorNotReady) break;
         if (e == hipErrorNotReady) {
             (void)hipGetLastError();
             e = hipSuccess;
         }
+        if (e == hipSuccess && waiting())
+            e = hipErrorLaunchFailure;  // the stream is idle and the step's last kernel has not run
         if (e != hipSuccess) break;
     }
-    e = hipStreamSynchronize(s->stream);
+    const hipError_t idle = hipStreamSynchronize(s->stream);
+    if (e == hipSuccess) e = idle;
     const bool conv = note->converged && maxsteps > 0;
     const double del = note->del;
     const int it = conv ? std::max(static_cast<int>(note->steps), 1) : maxsteps + 1;
@@ -1943,7 +1966,7 @@ int msm_steepest(msm_sim* s, int maxsteps, int linesearch, double alpha, double 
     if (rc != MSM_OK) return rc;
     if (maxsteps < 0 || !(maxdis > 0.0) || !(mindis >= 0.0) || !(alpha > 0.0))
         return set_err(s, MSM_ERR_ARG, "maxsteps >= 0, maxdis > 0, mindis >= 0 and alpha > 0");
-    (void)hipSetDevice(s->device);
+    enter(s);
     Quench q(s);
     if ((rc = q.alloc()) != MSM_OK) return rc;
     clear_flags(s);
@@ -2038,7 +2061,7 @@ int msm_cg(msm_sim* s, int maxsteps, int linesearch, double maxdis, double mindi
     if (rc != MSM_OK) return rc;
     if (maxsteps < 0 || !(maxdis > 0.0) || !(mindis >= 0.0))
         return set_err(s, MSM_ERR_ARG, "maxsteps >= 0, maxdis > 0 and mindis >= 0");
-    (void)hipSetDevice(s->device);
+    enter(s);
     Quench q(s);
     if ((rc = q.alloc()) != MSM_OK) return rc;
     clear_flags(s);
@@ -2126,7 +2149,7 @@ int msm_cg(msm_sim* s, int maxsteps, int linesearch, double maxdis, double mindi
 int msm_predictor(msm_sim* s, double h) {
     int rc = check_ready(s, false);
     if (rc != MSM_OK) return rc;
-    (void)hipSetDevice(s->device);
+    enter(s);
     AtomsDev a = atoms_view(s, s->scur, s->pcur);
     msm::launch_predictor(a, s->tab, s->boxes[0], s->d_boxes, multibox(s), h, s->stream);
     HIPCHK(s, hipStreamSynchronize(s->stream));
@@ -2136,7 +2159,7 @@ int msm_predictor(msm_sim* s, double h) {
 int msm_correction(msm_sim* s, double h) {
     int rc = check_ready(s, false);
     if (rc != MSM_OK) return rc;
-    (void)hipSetDevice(s->device);
+    enter(s);
     AtomsDev a = atoms_view(s, s->scur, s->pcur);
     msm::launch_correction(a, s->tab, h, s->stream);
     HIPCHK(s, hipStreamSynchronize(s->stream));
@@ -2148,7 +2171,7 @@ int msm_run(msm_sim* s, int nsteps, int nb_uptab, int step0, double h) {
     if (rc != MSM_OK) return rc;
     if (nsteps < 0) return set_err(s, MSM_ERR_ARG, "nsteps must be >= 0");
     if (nsteps == 0) return MSM_OK;
-    (void)hipSetDevice(s->device);
+    enter(s);
     clear_flags(s);
     // predictor of the first step (stand-alone kernel; later predictors run fused)
     {
@@ -2327,7 +2350,7 @@ int msm_autotune(msm_sim* s, int reps, int* choice, double* best_ms) {
     int rc = check_ready(s, true);
     if (rc != MSM_OK) return rc;
     if (reps < 1 || reps > 1000) return set_err(s, MSM_ERR_ARG, "reps must be 1..1000");
-    (void)hipSetDevice(s->device);
+    enter(s);
     struct Cand {
         int fp, lds, bd, wd, bf, wf, lanes, flanes = 0, autop = 0;
     };
@@ -2518,7 +2541,7 @@ int msm_adjoint(msm_sim* s, const double* dldf, const double* dlde, double* g_po
     const bool eam = s->tab.pot_type != 0;
     if (eam && (!g_fembd || !g_dfembd))
         return set_err(s, MSM_ERR_ARG, "EAM tables need the embedding gradient arrays");
-    (void)hipSetDevice(s->device);
+    enter(s);
     const int n = s->n, nbox = static_cast<int>(s->boxes.size());
     const int nt = s->tab.ntab2, ne = eam ? s->tab.nembd2 : 0;
     size_t nb1 = 0, nb2 = 0, stride = 0;
@@ -2621,7 +2644,7 @@ int msm_set_spline_table(msm_sim* s, const double* coef, int ld, int coef_on_dev
     if (!s->has_table) return set_err(s, MSM_ERR_STATE, "no force table (msm_set_force_table)");
     int rc = fm_check_model(s, ld);
     if (rc != MSM_OK) return rc;
-    (void)hipSetDevice(s->device);
+    enter(s);
     if (!s->fm_ev) HIPCHK(s, hipEventCreateWithFlags(&s->fm_ev, hipEventDisableTiming));
     // the staging buffer and the table buffers are free once the previous build has run
     if (s->fm_pending) HIPCHK(s, hipEventSynchronize(s->fm_ev));
@@ -2655,7 +2678,7 @@ int msm_fm_set_targets(msm_sim* s, const double* f_target, const double* e_targe
     if (!s || !f_target || !e_target) return MSM_ERR_ARG;
     if (!s->has_atoms || !s->has_boxes) return set_err(s, MSM_ERR_STATE, "no atoms or boxes");
     if (!(w_e >= 0.0)) return set_err(s, MSM_ERR_ARG, "w_e must be non-negative");
-    (void)hipSetDevice(s->device);
+    enter(s);
     const size_t n3 = 3 * static_cast<size_t>(std::max(s->n, 1));
     const size_t nbox = s->boxes.size();
     int rc = fm_reserve(s, &s->fm_ft, n3, s->fm_cap_ft);
@@ -2678,7 +2701,7 @@ int msm_fm_loss_grad(msm_sim* s, double* loss, double* coef_grad, int ld, int gr
     if (s->fm_n != s->n || s->n < 1)
         return set_err(s, MSM_ERR_STATE, "no targets for these atoms (msm_fm_set_targets)");
     if (coef_grad && (rc = fm_check_model(s, ld)) != MSM_OK) return rc;
-    (void)hipSetDevice(s->device);
+    enter(s);
     const int n = s->n, nbox = static_cast<int>(s->boxes.size());
     size_t nb1 = 0, nb2 = 0, stride = 0;
     if ((rc = adj_reserve(s, nb1, nb2, stride)) != MSM_OK) return rc;
@@ -2739,6 +2762,7 @@ int msm_fm_loss_grad(msm_sim* s, double* loss, double* coef_grad, int ld, int gr
             }
             HIPCHK(s, hipStreamBeginCapture(s->stream, hipStreamCaptureModeThreadLocal));
             enqueue();
+            if (ce == hipSuccess) ce = hipGetLastError();
             hipGraph_t gr = nullptr;
             const hipError_t ee = hipStreamEndCapture(s->stream, &gr);
             if (ce == hipSuccess) ce = ee;
@@ -2761,7 +2785,7 @@ int msm_fm_loss_grad(msm_sim* s, double* loss, double* coef_grad, int ld, int gr
 int msm_list_stats(msm_sim* s, long long* total, int* maxk) {
     if (!s || !total || !maxk) return MSM_ERR_ARG;
     if (!s->has_list) return set_err(s, MSM_ERR_STATE, "no neighbour list");
-    (void)hipSetDevice(s->device);
+    enter(s);
     msm::launch_fill_int(reinterpret_cast<int*>(s->d_stats), 0, 4, s->stream);
     msm::launch_list_stats(s->kvois, s->n, s->d_stats,
                            reinterpret_cast<int*>(s->d_stats + 1), s->stream);

@@ -1,0 +1,111 @@
+"""The C-ABI's host paths on a runtime of host memory whose kernels do nothing (fake_hip.c): what a
+call reports when a launch or an allocation fails.  Each case runs in a process of its own, since the
+runtime has to be loaded before the library."""
+import os
+import subprocess
+import sys
+
+import numpy as np
+import pytest
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+CASES = {}
+
+
+def case(f):
+    CASES[f.__name__] = f
+    return f
+
+
+@pytest.fixture(scope="module")
+def fake(tmp_path_factory):
+    so = str(tmp_path_factory.mktemp("fake") / "libfake_hip.so")
+    subprocess.run(["gcc", "-O1", "-shared", "-fPIC", "-o", so, os.path.join(HERE, "fake_hip.c"),
+                    "-lpthread"], check=True)
+    return so
+
+
+def _device(cells=(5, 5, 5), nbox=1):
+    import msmpscu_amd.configs as cfg
+    import msmpscu_amd.mdlib as md
+    boxes = [cfg.make_bcc_box(cells, cfg.W_A, 0.05, 300.0, 3 + k) for k in range(nbox)]
+    ctrl = cfg.w_ctrl(mx=32)
+    fc = md.MDForceClassGPU(ForceTable=cfg.w_forcetable(boxes[0], ctrl))
+    md.Register_ForceClass("FS_TYPE", fc)
+    md.Initialize_Globle_Variables_DEV(boxes, ctrl, fc)
+    md.Init_Forcetable_Dev(boxes, ctrl, fc)
+    return fc.Device, boxes, ctrl
+
+
+def _hip_error(call):
+    try:
+        call()
+    except RuntimeError as e:
+        assert "MSM_ERR_HIP" in str(e), e
+        return True
+    return False
+
+
+@case
+def refused_copies(f):
+    """A copy whose kernel was not launched is an error, not the bytes of an earlier copy."""
+    dev, boxes, _ = _device()
+    x = np.array(boxes[0].XP)
+    dev.get_atoms()
+    f.fake_refuse(b"k_copy_words")
+    assert _hip_error(dev.get_atoms)
+    assert _hip_error(dev.get_epot)
+    assert _hip_error(lambda: dev.put_atoms(x))
+    assert _hip_error(lambda: dev.put_dis(x))
+    dev.build_neighbors()
+    f.fake_refuse(b"k_sum_chunks")
+    assert _hip_error(dev.get_box_epot)
+    f.fake_refuse(b"k_copy_out")
+    assert _hip_error(dev.get_atoms)
+    f.fake_refuse(b"k_sort_pos")
+    assert _hip_error(lambda: dev.put_atoms(x))
+    f.fake_refuse(b"")
+    dev.get_atoms()     # and the error is not kept
+
+
+@case
+def refused_passes(f):
+    """A call of which a kernel was not launched is an error; so is a quench whose step gives no
+    note (here no kernel ever does)."""
+    dev, _, ctrl = _device()
+    dev.build_neighbors()
+    for kernel, call in ((b"k_density", dev.calc_force), (b"k_force", dev.calc_force),
+                         (b"k_energy", dev.calc_epot), (b"k_virial", dev.calc_atomic_stress),
+                         (b"k_force", lambda: dev.run(2, ctrl.NB_UPTAB, 0, ctrl.H)),
+                         (b"k_nlist", dev.build_neighbors),
+                         (b"k_predictor", lambda: dev.dyn_damp(3, 0.0, ctrl.H)),
+                         (b"k_damp_check", lambda: dev.dyn_damp(3, 0.0, ctrl.H))):
+        f.fake_refuse(kernel)
+        assert _hip_error(call), kernel
+        f.fake_refuse(b"")
+    dev.calc_force()
+    dev.run(2, ctrl.NB_UPTAB, 0, ctrl.H)
+    assert _hip_error(lambda: dev.dyn_damp(3, 0.0, ctrl.H))
+    steps, _ = dev.dyn_damp(0, 0.0, ctrl.H)
+    assert steps == 1
+
+
+@pytest.mark.parametrize("name", sorted(CASES))
+def test_host_path(fake, name):
+    r = subprocess.run([sys.executable, os.path.abspath(__file__), name, fake],
+                       cwd=os.path.dirname(HERE), stdout=subprocess.PIPE, stderr=subprocess.STDOUT,
+                       text=True, timeout=300)
+    assert r.returncode == 0, r.stdout
+
+
+if __name__ == "__main__":
+    import ctypes
+    runtime = ctypes.CDLL(sys.argv[2], mode=ctypes.RTLD_GLOBAL)
+    for fn in ("fake_host_bytes", "fake_host_allocs", "fake_dev_bytes", "fake_memsets"):
+        getattr(runtime, fn).restype = ctypes.c_long
+    for fn in ("fake_host_limit", "fake_dev_limit"):
+        getattr(runtime, fn).argtypes = [ctypes.c_long]
+        getattr(runtime, fn).restype = None
+    sys.path.insert(0, os.path.dirname(HERE))
+    CASES[sys.argv[1]](runtime)
+    print("ok")
