@@ -93,6 +93,7 @@ struct msm_sim {
     // sort + list
     SortBufs sb{};
     int sort_cap = 0;
+    bool counts_zero = true;  // sb.count holds zeros, as a rebuild leaves it
     int* kvois = nullptr;
     int* indi = nullptr;
     unsigned short* sidx = nullptr;
@@ -181,6 +182,7 @@ namespace {
 
 int set_err(msm_sim* s, int code, const std::string& msg) {
     if (s) s->err = msg;
+    if (s && code == MSM_ERR_HIP) s->counts_zero = false;  // a rebuild may have ended half-way
     return code;
 }
 
@@ -408,6 +410,12 @@ int read_flags(msm_sim* s) {
 // global list until the next rebuild).
 bool want_sidx(const msm_sim* s) {
     return s->force_path == 0 || s->force_path == 5 || s->tuning;
+}
+
+// In front of the first rebuild of a call (not part of a captured segment).
+void ready_counts(msm_sim* s) {
+    if (!s->counts_zero) msm::launch_fill_int(s->sb.count, 0, s->sort_cap, s->stream);
+    s->counts_zero = true;
 }
 
 // Neighbour-list rebuild on the stream (capturable: kernels only).  Reads the current set and
@@ -1220,6 +1228,9 @@ int msm_set_boxes(msm_sim* s, int nbox, const int* natoms, const double* lo, con
         cells += nc;
         if (cells > (1LL << 30)) return set_err(s, MSM_ERR_ARG, "too many cells");
     }
+    // from here on the old boxes are gone, also where an allocation fails
+    s->has_boxes = s->has_atoms = s->has_list = false;
+    clear_graphs(s);
     int rc = dalloc(s, &s->d_boxes, bx.size());
     if (rc != MSM_OK) return rc;
     HIPCHK(s, hipMemcpy(s->d_boxes, bx.data(), bx.size() * sizeof(BoxDev), hipMemcpyHostToDevice));
@@ -1227,13 +1238,15 @@ int msm_set_boxes(msm_sim* s, int nbox, const int* natoms, const double* lo, con
     s->ncell_total = static_cast<int>(cells);
     const int need = s->ncell_total + 2;
     if (need > s->sort_cap) {
+        s->sort_cap = 0;
         rc = dalloc(s, &s->sb.count, need);
         if (rc == MSM_OK) rc = dalloc(s, &s->sb.start, need);
         if (rc == MSM_OK) rc = dalloc(s, &s->sb.scan_tmp, need / 1024 + 2);
         if (rc != MSM_OK) return rc;
-        s->sort_cap = need;
         // every rebuild leaves the counts at zero
         HIPCHK(s, hipMemset(s->sb.count, 0, need * sizeof(int)));
+        s->sort_cap = need;
+        s->counts_zero = true;
     }
     s->half_min = HUGE_VAL;
     for (const BoxDev& b : s->boxes)
@@ -1247,9 +1260,6 @@ int msm_set_boxes(msm_sim* s, int nbox, const int* natoms, const double* lo, con
     HIPCHK(s, hipMemcpy(s->d_chunk_box, chunk_box.data(), chunk_box.size() * sizeof(int),
                         hipMemcpyHostToDevice));
     s->has_boxes = true;
-    s->has_atoms = false;
-    s->has_list = false;
-    clear_graphs(s);
     return MSM_OK;
 }
 
@@ -1517,6 +1527,7 @@ int msm_build_neighbors(msm_sim* s) {
     if (rc != MSM_OK) return rc;
     enter(s);
     clear_flags(s);
+    ready_counts(s);
     enqueue_rebuild(s);
     s->has_list = true;
     return read_flags(s);
@@ -2173,6 +2184,7 @@ int msm_run(msm_sim* s, int nsteps, int nb_uptab, int step0, double h) {
     if (nsteps == 0) return MSM_OK;
     enter(s);
     clear_flags(s);
+    ready_counts(s);
     // predictor of the first step (stand-alone kernel; later predictors run fused)
     {
         TimedScope ts(s, MSM_KCLASS_PREDICTOR);
@@ -2385,6 +2397,7 @@ int msm_autotune(msm_sim* s, int reps, int* choice, double* best_ms) {
         return MSM_OK;
     };
     clear_flags(s);
+    ready_counts(s);
     // list-build kernel (a rebuild of unchanged positions reproduces the same order and list)
     float best_nl = 0.f;
     int nl_choice = s->nlist_kind;

@@ -18,11 +18,13 @@ static struct { const void* host; const char* name; int launches; } fn[4096];
 static int nfn;
 static char refuse[128];    /* launches of kernels with this in their name are refused */
 static long host_limit = -1, dev_limit = -1;    /* allocations beyond this many bytes fail */
+static int dev_fail;    /* k > 0: the k-th device allocation from now fails */
 static long host_allocs, host_bytes, dev_bytes, memsets;
 
 void fake_refuse(const char* part) { strncpy(refuse, part, sizeof(refuse) - 1); }
 void fake_host_limit(long bytes) { host_limit = bytes; }
 void fake_dev_limit(long bytes) { dev_limit = bytes; }
+void fake_dev_fail(int k) { dev_fail = k; }
 long fake_host_bytes(void) { return host_bytes; }
 long fake_host_allocs(void) { return host_allocs; }
 long fake_dev_bytes(void) { return dev_bytes; }
@@ -106,7 +108,10 @@ static err_t give(void* p, long* total) {
     free((char*)p - 64);
     return OK;
 }
-err_t hipMalloc(void** p, size_t n) { return take(p, n, dev_limit, &dev_bytes); }
+err_t hipMalloc(void** p, size_t n) {
+    if (dev_fail && --dev_fail == 0) { *p = 0; return fail(OUT_OF_MEMORY); }
+    return take(p, n, dev_limit, &dev_bytes);
+}
 err_t hipFree(void* p) { return give(p, &dev_bytes); }
 err_t hipHostMalloc(void** p, size_t n, unsigned f) {
     (void)f;

@@ -90,6 +90,44 @@ def refused_passes(f):
     assert steps == 1
 
 
+@case
+def sort_buffers_after_failures(f):
+    """The cell counts are zero when a rebuild starts: after a set_boxes that failed between its
+    buffers, whatever grid the next one has, and after a rebuild of which a kernel was refused."""
+    import ctypes as C
+
+    import msmpscu_amd._lib as L
+    dev, boxes, ctrl = _device((16, 16, 17))        # 8704 atoms: the sort of several launches
+    box = boxes[0]
+
+    def set_boxes(scale):
+        n = np.array([box.NPRT], dtype=np.int32)
+        lo, ln = np.array(box.BOXLOW, dtype=float), np.array(box.ZL, dtype=float) * scale
+        return L.lib().msm_set_boxes(dev.h, 1, L.iptr(n), L.dptr(lo), L.dptr(ln),
+                                     L.iptr(np.array([1, 1, 1], dtype=np.int32)))
+
+    for k in (2, 3, 4):          # counts, starts, scan
+        f.fake_dev_fail(k)
+        assert set_boxes(2.0) == 3                          # MSM_ERR_NOMEM
+        f.fake_dev_fail(0)
+        assert L.lib().msm_build_neighbors(dev.h) == 7      # MSM_ERR_STATE: no boxes
+        before = f.fake_memsets()
+        assert set_boxes(1.0) == 0
+        assert f.fake_memsets() == before + 1, k
+    dev.set_atoms(box.XP, box.XP1, box.ITYP, box.STATU)
+    dev.build_neighbors()
+    for call in (dev.build_neighbors, lambda: dev.run(3, 1, 0, ctrl.H)):
+        dev.build_neighbors()
+        f.fake_refuse(b"k_scan_blocks")
+        assert _hip_error(dev.build_neighbors)
+        f.fake_refuse(b"")
+        fills = f.fake_launches(b"k_fill_int")
+        call()
+        assert f.fake_launches(b"k_fill_int") == fills + 1
+        call()
+        assert f.fake_launches(b"k_fill_int") == fills + 1
+
+
 @pytest.mark.parametrize("name", sorted(CASES))
 def test_host_path(fake, name):
     r = subprocess.run([sys.executable, os.path.abspath(__file__), name, fake],
