@@ -12,9 +12,9 @@ namespace msm {
 namespace {
 
 struct Ring {
-    std::mutex life;          // users, base, ev
-    std::mutex use;           // one transfer at a time
+    std::mutex mu;            // everything below, and one transfer at a time
     int users = 0;
+    bool refused = false;     // the memory could not be pinned
     char* base = nullptr;
     hipEvent_t ev[kCopySlots] = {};
 };
@@ -33,6 +33,21 @@ void drop(Ring& r) {
     }
     if (r.base) (void)hipHostFree(r.base);
     r.base = nullptr;
+}
+
+// Whether there is a ring (r.mu held): the first copy that asks pins it.
+bool pinned(Ring& r) {
+    if (r.base) return true;
+    if (r.users == 0 || r.refused) return false;
+    hipError_t e = hipHostMalloc(reinterpret_cast<void**>(&r.base), kCopySlots * kCopySlotBytes);
+    if (e != hipSuccess) r.base = nullptr;
+    for (int k = 0; k < kCopySlots && e == hipSuccess; ++k)
+        e = hipEventCreateWithFlags(&r.ev[k], hipEventDisableTiming);
+    if (e == hipSuccess) return true;
+    drop(r);
+    r.refused = true;
+    (void)hipGetLastError();
+    return false;
 }
 
 // Runs work(slot) on the calling thread (slot 0) and up to extra others; a thread that cannot be
@@ -62,39 +77,39 @@ void shape(size_t total, size_t& chunk, int& extra) {
 
 }  // namespace
 
-hipError_t copy_ring_acquire(int device) {
+void copy_ring_acquire(int device) {
     Ring* r = ring_of(device);
-    if (!r) return hipErrorInvalidDevice;
-    std::lock_guard<std::mutex> g(r->life);
-    if (r->users == 0) {
-        hipError_t e = hipHostMalloc(reinterpret_cast<void**>(&r->base),
-                                     kCopySlots * kCopySlotBytes);
-        for (int k = 0; k < kCopySlots && e == hipSuccess; ++k)
-            e = hipEventCreateWithFlags(&r->ev[k], hipEventDisableTiming);
-        if (e != hipSuccess) {
-            drop(*r);
-            return e;
-        }
-    }
+    if (!r) return;
+    std::lock_guard<std::mutex> g(r->mu);
     ++r->users;
-    return hipSuccess;
 }
 
 void copy_ring_release(int device) {
     Ring* r = ring_of(device);
     if (!r) return;
-    std::lock_guard<std::mutex> g(r->life);
-    if (r->users > 0 && --r->users == 0) drop(*r);
+    std::lock_guard<std::mutex> g(r->mu);
+    if (r->users == 0 || --r->users > 0) return;
+    drop(*r);
+    r->refused = false;
 }
 
 hipError_t copy_to_host(int device, const void* base, size_t total, const CopyPart* parts,
                         int nparts, hipStream_t stream) {
-    Ring* r = ring_of(device);
-    if (!r || total == 0) return r ? hipStreamSynchronize(stream) : hipErrorInvalidDevice;
     // the stream's earlier work ends before the ring is taken, for other streams to use it meanwhile
     const hipError_t idle = hipStreamSynchronize(stream);
-    if (idle != hipSuccess) return idle;
-    std::lock_guard<std::mutex> g(r->use);
+    Ring* r = ring_of(device);
+    if (idle != hipSuccess || total == 0) return idle;
+    std::unique_lock<std::mutex> g;
+    if (r) g = std::unique_lock<std::mutex>(r->mu);
+    if (!r || !pinned(*r)) {
+        if (r) g.unlock();
+        hipError_t e = hipSuccess;
+        for (int k = 0; k < nparts && e == hipSuccess; ++k)
+            e = hipMemcpyAsync(parts[k].host, static_cast<const char*>(base) + parts[k].offset,
+                               parts[k].bytes, hipMemcpyDeviceToHost, stream);
+        const hipError_t done = hipStreamSynchronize(stream);
+        return e != hipSuccess ? e : done;
+    }
     size_t chunk;
     int extra;
     shape(total, chunk, extra);
@@ -129,10 +144,16 @@ hipError_t copy_to_host(int device, const void* base, size_t total, const CopyPa
 
 hipError_t copy_to_device(int device, void* dst, const void* host, size_t total,
                           hipStream_t stream) {
-    Ring* r = ring_of(device);
-    if (!r) return hipErrorInvalidDevice;
     if (total == 0) return hipSuccess;
-    std::lock_guard<std::mutex> g(r->use);
+    Ring* r = ring_of(device);
+    std::unique_lock<std::mutex> g;
+    if (r) g = std::unique_lock<std::mutex>(r->mu);
+    if (!r || !pinned(*r)) {
+        if (r) g.unlock();
+        const hipError_t e = hipMemcpyAsync(dst, host, total, hipMemcpyHostToDevice, stream);
+        const hipError_t done = hipStreamSynchronize(stream);
+        return e != hipSuccess ? e : done;
+    }
     size_t chunk;
     int extra;
     shape(total, chunk, extra);

@@ -19,8 +19,9 @@ namespace msm {
 constexpr int kCopySlots = 8;
 constexpr size_t kCopySlotBytes = size_t(1) << 20;
 
-// The rings are shared by the contexts of a GPU and live as long as one of them does.
-hipError_t copy_ring_acquire(int device);
+// A GPU's contexts share its ring, one transfer at a time.  The first large copy pins it (0.13 ms), and
+// it is given back with the last context; where it cannot be pinned, copies are plain ones.
+void copy_ring_acquire(int device);
 void copy_ring_release(int device);
 
 // One piece of a device block and its place on the host.

@@ -128,6 +128,35 @@ def sort_buffers_after_failures(f):
         assert f.fake_launches(b"k_fill_int") == fills + 1
 
 
+@case
+def pinned_ring(f):
+    """Creating a context pins its own few words only, and works where no more can be pinned: large
+    copies are then plain ones.  Else the first large copy pins the ring, which goes with the last
+    context."""
+    ring = 8 << 20
+    for limit in (ring - 1, -1):
+        f.fake_host_limit(limit)
+        dev, boxes, _ = _device((16, 16, 17))
+        other, _, _ = _device((4, 4, 4))
+        other.get_atoms()
+        small = f.fake_host_bytes()
+        assert small < ring // 8
+        have = small + (0 if limit > 0 else ring)
+        for _ in range(2):
+            # the runtime's memory holds 0x5a, and the kernels leave it
+            assert all(set(a.tobytes()) == {0x5a} for a in dev.get_atoms())
+            assert f.fake_host_bytes() == have
+        tries = f.fake_host_allocs()
+        dev.put_atoms(boxes[0].XP, boxes[0].XP1)
+        x = dev.get_atoms()[0]      # the staging block as put_atoms left it: the velocities
+        assert np.array_equal(x, boxes[0].XP1)
+        assert f.fake_host_allocs() == tries        # refused once is refused while contexts live
+        dev.close()
+        assert f.fake_host_bytes() >= have - small
+        other.close()
+        assert f.fake_host_bytes() == 0
+
+
 @pytest.mark.parametrize("name", sorted(CASES))
 def test_host_path(fake, name):
     r = subprocess.run([sys.executable, os.path.abspath(__file__), name, fake],
