@@ -302,10 +302,14 @@ int msm_list_stats(msm_sim* sim, long long* total, int* maxk);
                                     halo slots: cell bricks, small or wide by cell occupancy);
                                     1: per-atom global scan; 2: small LDS-staged cell bricks (one
                                     lane per atom); 3: wide bricks (several lanes per atom) */
-#define MSM_OPT_FORCE_PATH    4  /* density/force passes: 0 LDS bricks; 1, 2, 4, 8: global list
-                                    with that many lanes per atom (2 is reported until it is
-                                    set; until one of the pass options is set, lanes and table
-                                    placement follow the number of atoms); 3: two lanes per
+#define MSM_PATH_BY_SIZE    (-1)
+#define MSM_OPT_FORCE_PATH    4  /* density/force passes: MSM_PATH_BY_SIZE (default): lanes per
+                                    atom and table placement follow the number of atoms, until
+                                    this, MSM_OPT_TABLE_LDS, MSM_OPT_FORCE_LANES,
+                                    MSM_OPT_CHUNK_SWEEP or an MSM_OPT_LT_* option is changed
+                                    (which then start from path 2); setting it again gives those
+                                    options their defaults; 0 LDS bricks; 1, 2, 4, 8: global list
+                                    with that many lanes per atom; 3: two lanes per
                                     atom, each 32-byte record gathered by a lane pair; 5: staged
                                     bricks (a brick's halo staged in LDS once, pairs read as halo
                                     slots; needs a list from the brick list kernels, else as 2) */
@@ -408,7 +412,7 @@ int msm_fm_loss_grad(msm_sim* sim, double* loss, double* coef_grad, int ld, int 
  * kernel and `reps` density + force passes (no integration) of every applicable variant of the
  * density/force kernels (lanes per atom, LDS table and its workgroup shape, lane-pair gather,
  * LDS bricks), sets the options to the fastest, and recomputes F' and F with it.  choice[8]
- * (may be NULL) receives {force path, table LDS, density block, density workgroups per CU, force
+ * (may be NULL) receives {force path (MSM_PATH_BY_SIZE or a path), table LDS, density block, density workgroups per CU, force
  * block, force workgroups per CU, list kernel (MSM_OPT_NLIST_KERNEL value), brick lanes
  * (MSM_OPT_BRICK_LANES value)}; best_ms[2] (may
  * be NULL) the chosen density+force and rebuild times in ms.  Positions and velocities are

@@ -125,6 +125,7 @@ MSM_OPT_CELL_BRICK = 11
 MSM_OPT_BRICK_LANES = 12
 MSM_OPT_PASS_KERNEL = 13
 MSM_OPT_FORCE_LANES = 14
+MSM_PATH_BY_SIZE = -1
 PASS_KERNELS = ["bricks", "global", "lanes", "lane_pair", "lds_table", "brick_table", "staged",
                 "wide"]
 KCLASS = ["density", "force", "rebuild", "predictor", "nlist", "adjoint"]

@@ -53,6 +53,8 @@ struct GraphKey {
 // The context's pinned words: flags and the quench's note ahead, then room for small copies.
 constexpr size_t kPinnedHead = 64, kSmallCopy = size_t(64) << 10;
 
+constexpr msm::LtShape kLtDefault{1024, 1, 1024, 1, 0};
+
 struct msm_sim {
     int device = 0;
     hipStream_t stream = nullptr;
@@ -133,8 +135,8 @@ struct msm_sim {
     int bt_lanes = 1;      // lanes per home atom of the brick passes with the table in LDS
     int force_lanes = 0;   // lanes per atom of the LDS-table force pass (0: as force_path)
     int cell_brick = 1;    // cells are numbered in bricks of cell_brick^3 (1: row-major)
-    msm::LtShape lt{1024, 1, 1024, 1};  // block / workgroups per CU of the LDS-table passes
-    int auto_pass = 1;     // no pass option set: lanes and table placement by size (walk_plan)
+    msm::LtShape lt = kLtDefault;  // block / workgroups per CU of the LDS-table passes
+    int auto_pass = 1;     // MSM_PATH_BY_SIZE: lanes and table placement by size (walk_plan)
     int compact = 0;       // global-list path: force pass reads the density pass's in-cutoff list
 
     // adjoint scratch (allocated on first use)
@@ -663,9 +665,8 @@ bool use_brick_table(const msm_sim* s) {
            p.cap_f > 0;
 }
 
-// Lanes per atom of a pass when no option fixes the kernel (MSM_OPT_FORCE_PATH and the other
-// pass options leave s->auto_pass): enough that the pass holds about 120,000 lanes (twice that
-// for long lists), at least 2 (4).  Measured, density + force + 1/10 list per step: 2,000 W atoms
+// Lanes per atom of a pass when no option fixes the kernel (s->auto_pass): enough that the pass
+// holds about 120,000 lanes (twice that for long lists), at least 2 (4).  Measured, density + force + 1/10 list per step: 2,000 W atoms
 // (26 neighbours) 37.9 us at 2 lanes, 21.2 / 19.5 / 19.2 at 8 / 16 / 32; 16,000 atoms 38.0 at 2,
 // 23.3 / 24.7 / 30.1; 54,000 atoms 30.1 / 32.0 / 38.1 at 2 / 4 / 8, 137,000 48.7 / 51.0 / 64.1;
 // Cu-Ni (86 neighbours) 42,600 atoms 131.9 / 100.5 / 93.8 at 2 / 4 / 8, 442,000 atoms 377.7 /
@@ -2215,6 +2216,23 @@ int msm_sync(msm_sim* s) {
     return MSM_OK;
 }
 
+// The pass options of a new context: lanes and table placement by the number of atoms.
+static void passes_by_size(msm_sim* s) {
+    s->auto_pass = 1;
+    s->force_path = 2;
+    s->table_lds = 1;
+    s->force_lanes = 0;
+    s->lt = kLtDefault;
+}
+
+// A pass option: changing it ends the choice by size, setting it to what it is does not.
+static void set_pass(msm_sim* s, int& field, int value) {
+    if (field == value) return;
+    field = value;
+    s->auto_pass = 0;
+    clear_graphs(s);
+}
+
 int msm_set_option(msm_sim* s, int option, int value) {
     if (!s) return MSM_ERR_ARG;
     switch (option) {
@@ -2237,26 +2255,25 @@ int msm_set_option(msm_sim* s, int option, int value) {
             return MSM_OK;
         }
         case MSM_OPT_FORCE_PATH:
-            if (value < 0 || value > 8 || (value > 5 && value != 8))
-                return set_err(s, MSM_ERR_ARG, "force path must be 0, 1, 2, 3, 4, 5 or 8");
-            s->force_path = value;
-            s->auto_pass = 0;
+            if (value < MSM_PATH_BY_SIZE || value > 8 || (value > 5 && value != 8))
+                return set_err(s, MSM_ERR_ARG, "force path must be -1, 0, 1, 2, 3, 4, 5 or 8");
+            if (value == MSM_PATH_BY_SIZE) {
+                passes_by_size(s);
+            } else {
+                s->force_path = value;
+                s->auto_pass = 0;
+            }
             clear_graphs(s);
             return MSM_OK;
-        case MSM_OPT_COMPACT_LIST:
+        case MSM_OPT_COMPACT_LIST:  // (no list walk while it is on)
             s->compact = value ? 1 : 0;
-            s->auto_pass = 0;
             clear_graphs(s);
             return MSM_OK;
         case MSM_OPT_CHUNK_SWEEP:
-            s->lt.sweep = value ? 1 : 0;
-            s->auto_pass = 0;
-            clear_graphs(s);
+            set_pass(s, s->lt.sweep, value ? 1 : 0);
             return MSM_OK;
         case MSM_OPT_TABLE_LDS:
-            s->table_lds = value ? 1 : 0;
-            s->auto_pass = 0;
-            clear_graphs(s);
+            set_pass(s, s->table_lds, value ? 1 : 0);
             return MSM_OK;
         case MSM_OPT_CELL_BRICK:
             if (value < 1 || value > 16)
@@ -2278,25 +2295,19 @@ int msm_set_option(msm_sim* s, int option, int value) {
         case MSM_OPT_FORCE_LANES:
             if (value != 0 && value != 1 && value != 2 && value != 4)
                 return set_err(s, MSM_ERR_ARG, "force lanes must be 0, 1, 2 or 4");
-            s->force_lanes = value;
-            s->auto_pass = 0;
-            clear_graphs(s);
+            set_pass(s, s->force_lanes, value);
             return MSM_OK;
         case MSM_OPT_LT_DENSITY_BLOCK:
         case MSM_OPT_LT_FORCE_BLOCK:
             if (value != 256 && value != 512 && value != 1024)
                 return set_err(s, MSM_ERR_ARG, "LDS-table block must be 256, 512 or 1024");
-            (option == MSM_OPT_LT_DENSITY_BLOCK ? s->lt.block_d : s->lt.block_f) = value;
-            s->auto_pass = 0;
-            clear_graphs(s);
+            set_pass(s, option == MSM_OPT_LT_DENSITY_BLOCK ? s->lt.block_d : s->lt.block_f, value);
             return MSM_OK;
         case MSM_OPT_LT_DENSITY_WGS:
         case MSM_OPT_LT_FORCE_WGS:
             if (value < 1 || value > 16)
                 return set_err(s, MSM_ERR_ARG, "LDS-table workgroups per CU must be 1..16");
-            (option == MSM_OPT_LT_DENSITY_WGS ? s->lt.wgs_d : s->lt.wgs_f) = value;
-            s->auto_pass = 0;
-            clear_graphs(s);
+            set_pass(s, option == MSM_OPT_LT_DENSITY_WGS ? s->lt.wgs_d : s->lt.wgs_f, value);
             return MSM_OK;
         default:
             return set_err(s, MSM_ERR_ARG, "unknown option");
@@ -2322,7 +2333,9 @@ int msm_get_option(msm_sim* s, int option, int* value) {
         case MSM_OPT_TRACK_DIS: *value = s->track_dis; return MSM_OK;
         case MSM_OPT_KERNEL_TIMING: *value = s->timing; return MSM_OK;
         case MSM_OPT_NLIST_KERNEL: *value = s->nlist_kind; return MSM_OK;
-        case MSM_OPT_FORCE_PATH: *value = s->force_path; return MSM_OK;
+        case MSM_OPT_FORCE_PATH:
+            *value = s->auto_pass ? MSM_PATH_BY_SIZE : s->force_path;
+            return MSM_OK;
         case MSM_OPT_COMPACT_LIST: *value = s->compact; return MSM_OK;
         case MSM_OPT_TABLE_LDS: *value = s->table_lds; return MSM_OK;
         case MSM_OPT_LT_DENSITY_BLOCK: *value = s->lt.block_d; return MSM_OK;
@@ -2366,7 +2379,7 @@ int msm_autotune(msm_sim* s, int reps, int* choice, double* best_ms) {
     struct Cand {
         int fp, lds, bd, wd, bf, wf, lanes, flanes = 0, autop = 0;
     };
-    // the choice by size first (reported as its path and shape)
+    // the choice by size first
     std::vector<Cand> cands{{2, 1, 1024, 1, 1024, 1, 1, 0, 1}};
     if (msm::lt_window(s->tab, 1, 1).wf * 2 >= s->tab.ntab2) {
         for (int fp : {2, 3, 1, 4}) {
@@ -2473,7 +2486,7 @@ int msm_autotune(msm_sim* s, int reps, int* choice, double* best_ms) {
     enqueue_density(s);
     enqueue_force(s, 0, 1, 0.0);
     if (choice) {
-        const int c[8] = {w.fp, w.lds, w.bd, w.wd, w.bf, w.wf, s->nlist_kind, w.lanes};
+        const int c[8] = {w.autop ? MSM_PATH_BY_SIZE : w.fp, w.lds, w.bd, w.wd, w.bf, w.wf, s->nlist_kind, w.lanes};
         for (int k = 0; k < 8; ++k) choice[k] = c[k];
     }
     if (best_ms) {

@@ -157,6 +157,37 @@ def pinned_ring(f):
         assert f.fake_host_bytes() == 0
 
 
+@case
+def pass_options(f):
+    """The choice of the passes by size survives options set to what they are, and compaction switched
+    on and off; MSM_PATH_BY_SIZE is reported for it and brings it back."""
+    import msmpscu_amd._lib as L
+    dev, _, _ = _device()
+    opts = [L.MSM_OPT_FORCE_PATH, L.MSM_OPT_COMPACT_LIST, L.MSM_OPT_CHUNK_SWEEP, L.MSM_OPT_TABLE_LDS,
+            L.MSM_OPT_LT_DENSITY_BLOCK, L.MSM_OPT_LT_DENSITY_WGS, L.MSM_OPT_LT_FORCE_BLOCK,
+            L.MSM_OPT_LT_FORCE_WGS, L.MSM_OPT_FORCE_LANES]
+    first = {o: dev.get_option(o) for o in opts}
+    assert first[L.MSM_OPT_FORCE_PATH] == L.MSM_PATH_BY_SIZE == -1
+    assert dev.pass_kernel() == "wide"
+    for o in opts:
+        dev.set_option(o, first[o])
+        assert dev.pass_kernel() == "wide", o
+    dev.set_option(L.MSM_OPT_COMPACT_LIST, 1)
+    assert dev.pass_kernel() == "lds_table"
+    dev.set_option(L.MSM_OPT_COMPACT_LIST, 0)
+    assert dev.pass_kernel() == "wide"
+    for o, v, kernel in ((L.MSM_OPT_FORCE_PATH, 2, "lds_table"), (L.MSM_OPT_TABLE_LDS, 0, "lanes"),
+                         (L.MSM_OPT_LT_FORCE_BLOCK, 256, "lds_table"),
+                         (L.MSM_OPT_FORCE_LANES, 1, "lds_table")):
+        dev.set_option(o, v)
+        assert dev.pass_kernel() == kernel and dev.get_option(o) == v
+        assert dev.get_option(L.MSM_OPT_FORCE_PATH) == 2
+        dev.set_option(L.MSM_OPT_FORCE_PATH, L.MSM_PATH_BY_SIZE)
+        assert dev.pass_kernel() == "wide"
+        assert {q: dev.get_option(q) for q in opts} == first
+    assert L.lib().msm_set_option(dev.h, L.MSM_OPT_FORCE_PATH, -2) == 1      # MSM_ERR_ARG
+
+
 @pytest.mark.parametrize("name", sorted(CASES))
 def test_host_path(fake, name):
     r = subprocess.run([sys.executable, os.path.abspath(__file__), name, fake],
