@@ -321,7 +321,8 @@ int msm_list_stats(msm_sim* sim, long long* total, int* maxk);
                                     window held in LDS (persistent grid) -- on the global-list
                                     paths 1, 2, 3, 4 (no compaction) and, when the list was
                                     built by the LDS-brick kernels, on path 0 (then positions
-                                    and knots both come from LDS) */
+                                    and knots both come from LDS); 0: from global memory, also in
+                                    the energy and stress passes */
 /* Shape of the LDS-table passes: threads per workgroup (256, 512, 1024; default 1024) and
  * workgroups per CU (1..16, default 1; capped by what fits); the LDS window is the CU's LDS
  * divided by the workgroups per CU. */

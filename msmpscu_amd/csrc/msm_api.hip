@@ -697,7 +697,8 @@ void walk_geometry(const msm_sim* s, msm::WalkPlan& p) {
 // 108.4 without.  false: a table too large for the LDS on a large box (the general passes).
 bool size_plan(const msm_sim* s, int force, msm::WalkPlan& p) {
     p.lanes = auto_lanes(s);
-    p.tl = p.lanes <= 8 && s->n * s->kmean >= 8.0e5 && msm::walk_window_ok(s->tab, force, p.wgs);
+    p.tl = s->table_lds && p.lanes <= 8 && s->n * s->kmean >= 8.0e5 &&
+           msm::walk_window_ok(s->tab, force, p.wgs);
     if (!p.tl) {
         if (s->n * s->kmean >= 8.0e6) return false;
         p.lanes = std::max(p.lanes, 8);

@@ -188,6 +188,25 @@ def pass_options(f):
     assert L.lib().msm_set_option(dev.h, L.MSM_OPT_FORCE_PATH, -2) == 1      # MSM_ERR_ARG
 
 
+@case
+def table_lds_off(f):
+    """MSM_OPT_TABLE_LDS 0 keeps the knots of the energy and stress passes out of LDS too."""
+    import msmpscu_amd._lib as L
+    dev, _, _ = _device((30, 30, 30))       # 54,000 atoms: knots in LDS by size
+    dev.build_neighbors()
+
+    def launches():     # k_*_w<..., lanes, TL>
+        return [f.fake_launches(k) for k in (b"ELi1EEEvNS_8AtomsDevENS_7ListDevE", b"Li8ELi0EEEvNS_8AtomsDevENS_7ListDevE")]
+    dev.calc_epot()
+    dev.calc_atomic_stress()
+    lds, glob = launches()
+    assert lds == 3 and glob == 0       # energy; density and virial
+    dev.set_option(L.MSM_OPT_TABLE_LDS, 0)
+    dev.calc_epot()
+    dev.calc_atomic_stress()
+    assert launches() == [lds, 2]
+
+
 @pytest.mark.parametrize("name", sorted(CASES))
 def test_host_path(fake, name):
     r = subprocess.run([sys.executable, os.path.abspath(__file__), name, fake],
