@@ -2393,12 +2393,27 @@ int msm_autotune(msm_sim* s, int reps, int* choice, double* best_ms) {
     for (int fp : {2, 1, 3, 4, 8, 0}) cands.push_back({fp, 0, s->lt.block_d, s->lt.wgs_d,
                                                        s->lt.block_f, s->lt.wgs_f, 1});
     const bool brick_list = s->nlist_kind != 1;  // the list-kernel choice below keeps this
+    hipEvent_t e0 = nullptr, e1 = nullptr;
+    HIPCHK(s, hipEventCreate(&e0));
+    if (hipError_t e = hipEventCreate(&e1); e != hipSuccess) {
+        (void)hipEventDestroy(e0);
+        return set_err(s, MSM_ERR_HIP, hipGetErrorString(e));
+    }
+    // what an error puts back
+    const Cand was{s->force_path, s->table_lds, s->lt.block_d, s->lt.wgs_d, s->lt.block_f,
+                   s->lt.wgs_f, s->bt_lanes, s->force_lanes, s->auto_pass};
+    const int was_sweep = s->lt.sweep, was_compact = s->compact, was_nlist = s->nlist_kind;
+    auto select = [&](const Cand& c) {
+        s->force_path = c.fp;
+        s->table_lds = c.lds;
+        s->lt = msm::LtShape{c.bd, c.wd, c.bf, c.wf, 0};
+        s->bt_lanes = c.lanes;
+        s->force_lanes = c.flanes;
+        s->auto_pass = c.autop;
+    };
     const int saved_timing = s->timing;
     s->timing = 0;
     s->compact = 0;
-    hipEvent_t e0 = nullptr, e1 = nullptr;
-    HIPCHK(s, hipEventCreate(&e0));
-    HIPCHK(s, hipEventCreate(&e1));
     s->tuning = 1;  // cleared below on every path after this point
     auto time_it = [&](auto&& body, float& ms) -> int {
         body();  // warm-up (code object load, occupancy query)
@@ -2454,12 +2469,7 @@ int msm_autotune(msm_sim* s, int reps, int* choice, double* best_ms) {
     float best = 0.f;
     size_t bi = 0;
     for (size_t c = 0; c < cands.size() && rc == MSM_OK; ++c) {
-        s->force_path = cands[c].fp;
-        s->table_lds = cands[c].lds;
-        s->lt = msm::LtShape{cands[c].bd, cands[c].wd, cands[c].bf, cands[c].wf};
-        s->bt_lanes = cands[c].lanes;
-        s->force_lanes = cands[c].flanes;
-        s->auto_pass = cands[c].autop;
+        select(cands[c]);
         float ms = 0.f;
         rc = time_it([&] {
             enqueue_density(s);
@@ -2474,15 +2484,18 @@ int msm_autotune(msm_sim* s, int reps, int* choice, double* best_ms) {
     (void)hipEventDestroy(e1);
     s->timing = saved_timing;
     s->tuning = 0;
-    if (rc != MSM_OK) return rc;
-    const Cand& w = cands[bi];
-    s->force_path = w.fp;
-    s->table_lds = w.lds;
-    s->lt = msm::LtShape{w.bd, w.wd, w.bf, w.wf};
-    s->bt_lanes = w.lanes;
-    s->force_lanes = w.flanes;
-    s->auto_pass = w.autop;
     clear_graphs(s);
+    if (rc != MSM_OK) {
+        select(was);
+        s->lt.sweep = was_sweep;
+        s->compact = was_compact;
+        s->nlist_kind = was_nlist;
+        s->has_list = false;  // any of the list kernels' lists
+        const int rr = replan_bricks(s);
+        return rr != MSM_OK ? rr : rc;
+    }
+    const Cand& w = cands[bi];
+    select(w);
     // leave F' and F as the chosen kernels compute them
     enqueue_density(s);
     enqueue_force(s, 0, 1, 0.0);

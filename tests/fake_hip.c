@@ -24,6 +24,8 @@ static long host_allocs, host_bytes, dev_bytes, memsets;
 void fake_refuse(const char* part) { strncpy(refuse, part, sizeof(refuse) - 1); }
 void fake_host_limit(long bytes) { host_limit = bytes; }
 void fake_dev_limit(long bytes) { dev_limit = bytes; }
+static int time_fail;   /* k > 0: the k-th reading of an event pair from now fails */
+void fake_time_fail(int k) { time_fail = k; }
 void fake_dev_fail(int k) { dev_fail = k; }
 long fake_host_bytes(void) { return host_bytes; }
 long fake_host_allocs(void) { return host_allocs; }
@@ -148,4 +150,8 @@ err_t hipEventCreateWithFlags(void** e, unsigned f) { (void)f; return hipEventCr
 err_t hipEventDestroy(void* e) { free(e); return OK; }
 err_t hipEventRecord(void* e, void* s) { (void)e; (void)s; return OK; }
 err_t hipEventSynchronize(void* e) { (void)e; return OK; }
-err_t hipEventElapsedTime(float* ms, void* a, void* b) { (void)a; (void)b; *ms = 0.001f; return OK; }
+err_t hipEventElapsedTime(float* ms, void* a, void* b) { 
+    (void)a; (void)b;
+    *ms = 0.001f;
+    return time_fail && --time_fail == 0 ? fail(LAUNCH_FAILED) : OK;
+}

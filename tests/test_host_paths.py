@@ -207,6 +207,32 @@ def table_lds_off(f):
     assert launches() == [lds, 2]
 
 
+@case
+def autotune_fails(f):
+    """An autotuner whose timing fails leaves every option as it was."""
+    import msmpscu_amd._lib as L
+    dev, _, _ = _device()
+    dev.build_neighbors()
+    opts = range(L.MSM_OPT_TRACK_DIS, L.MSM_OPT_CHUNK_SWEEP + 1)
+
+    def state():
+        return [dev.get_option(o) for o in opts]
+    for setting in ((), ((L.MSM_OPT_FORCE_PATH, 4), (L.MSM_OPT_LT_FORCE_BLOCK, 512),
+                         (L.MSM_OPT_BRICK_LANES, 4), (L.MSM_OPT_KERNEL_TIMING, 1)),
+                    ((L.MSM_OPT_NLIST_KERNEL, 3), (L.MSM_OPT_COMPACT_LIST, 1))):
+        for o, v in setting:
+            dev.set_option(o, v)
+        dev.build_neighbors()
+        before = state()
+        for k in (1, 3, 4, 5, 9, 15):       # the list kernels, then the passes
+            f.fake_time_fail(k)
+            assert _hip_error(lambda: dev.autotune(1))
+            f.fake_time_fail(0)
+            assert state() == before, k
+            dev.build_neighbors()
+    dev.autotune(1)
+
+
 @pytest.mark.parametrize("name", sorted(CASES))
 def test_host_path(fake, name):
     r = subprocess.run([sys.executable, os.path.abspath(__file__), name, fake],
