@@ -1838,13 +1838,13 @@ int msm_dyn_damp(msm_sim* s, int maxsteps, double mindele, double h, int* steps,
             (void)hipGetLastError();
             e = hipSuccess;
         }
-        if (e == hipSuccess && waiting())
-            e = hipErrorLaunchFailure;  // the stream is idle and the step's last kernel has not run
-        if (e != hipSuccess) break;
+        if (e != hipSuccess || waiting()) break;
     }
     const hipError_t idle = hipStreamSynchronize(s->stream);
     if (e == hipSuccess) e = idle;
     const bool conv = note->converged && maxsteps > 0;
+    // the stream is idle: without convergence every step has left its note
+    if (e == hipSuccess && !conv && note->steps < queued) e = hipErrorLaunchFailure;
     const double del = note->del;
     const int it = conv ? std::max(static_cast<int>(note->steps), 1) : maxsteps + 1;
     if (e == hipSuccess && !conv && maxsteps > 0) {

@@ -85,7 +85,8 @@ def refused_passes(f):
         f.fake_refuse(b"")
     dev.calc_force()
     dev.run(2, ctrl.NB_UPTAB, 0, ctrl.H)
-    assert _hip_error(lambda: dev.dyn_damp(3, 0.0, ctrl.H))
+    for maxsteps in (1, 2, 3):
+        assert _hip_error(lambda: dev.dyn_damp(maxsteps, 0.0, ctrl.H))
     steps, _ = dev.dyn_damp(0, 0.0, ctrl.H)
     assert steps == 1
 
