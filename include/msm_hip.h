@@ -421,7 +421,8 @@ int msm_fm_loss_grad(msm_sim* sim, double* loss, double* coef_grad, int ld, int 
 int msm_autotune(msm_sim* sim, int reps, int* choice, double* best_ms);
 
 /* Kernel classes for msm_kernel_times. */
-#define MSM_KCLASS_DENSITY   0
+#define MSM_KCLASS_DENSITY   0  /* also the energy pass where it makes the densities as well
+                                   (msm_fm_loss_grad, msm_dyn_damp) */
 #define MSM_KCLASS_FORCE     1  /* force pass with the fused corrector/predictor */
 #define MSM_KCLASS_REBUILD   2  /* whole neighbour-list rebuild (binning, sort, gather, list) */
 #define MSM_KCLASS_PREDICTOR 3

@@ -9,6 +9,7 @@
 #include <cstring>
 #include <map>
 #include <mutex>
+#include <optional>
 #include <string>
 #include <tuple>
 #include <vector>
@@ -743,12 +744,14 @@ bool aux_plan(const msm_sim* s, msm::WalkPlan& p) {
 }
 
 // Per-atom energies; rho_out (may be null) also the densities, write_fp: F' in pos.w as the density
-// pass leaves it.
+// pass leaves it (the walk's pass is then the density pass, and timed as such).
 void enqueue_epot(msm_sim* s, double* rho_out = nullptr, int write_fp = 0) {
     AtomsDev a = atoms_view(s, s->scur, s->pcur);
     msm::WalkPlan wp{};
     // (a compacted force pass reads what the density pass records beside F')
     if (!(write_fp && s->compact) && aux_plan(s, wp)) {
+        std::optional<TimedScope> ts;
+        if (write_fp) ts.emplace(s, MSM_KCLASS_DENSITY);
         msm::launch_energy_walk(wp, a, list_view(s), s->tab, s->boxes[0], s->d_boxes,
                                 multibox(s), rho_out, write_fp, s->d_err, s->stream);
         return;
@@ -2757,12 +2760,9 @@ int msm_fm_loss_grad(msm_sim* s, double* loss, double* coef_grad, int ld, int gr
     hipError_t ce = hipSuccess;
     clear_flags(s);
     auto enqueue = [&]() {
-        {
-            // the energy pass is the density pass too: it leaves F' in pos.w and, with a gradient,
-            // keeps rho for the adjoint, whose own rho pass is skipped
-            TimedScope ts(s, MSM_KCLASS_DENSITY);
-            enqueue_epot(s, coef_grad ? s->adj_rho : nullptr, 1);
-        }
+        // the energy pass is the density pass too: it leaves F' in pos.w and, with a gradient,
+        // keeps rho for the adjoint, whose own rho pass is skipped
+        enqueue_epot(s, coef_grad ? s->adj_rho : nullptr, 1);
         enqueue_force(s, 0, 1, 0.0);
         enqueue_box_sums(s, s->epot, 0, 1, s->d_ebox);
         const AtomSet& z = s->set[s->scur];

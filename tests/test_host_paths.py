@@ -234,6 +234,28 @@ def autotune_fails(f):
     dev.autotune(1)
 
 
+@case
+def density_is_timed_once(f):
+    """MSM_OPT_KERNEL_TIMING counts one density pass an evaluation of the loss and a quench step,
+    whichever kernel makes it."""
+    import msmpscu_amd._lib as L
+    dev, boxes, ctrl = _device()
+    dev.build_neighbors()
+    n = boxes[0].NPRT
+    ft, et, loss = np.zeros(3 * n), np.zeros(1), np.zeros(1)
+    assert L.lib().msm_fm_set_targets(dev.h, L.dptr(ft), L.dptr(et), 1.0) == 0
+    dev.set_option(L.MSM_OPT_KERNEL_TIMING, 1)
+    for compact in (0, 1):
+        dev.set_option(L.MSM_OPT_COMPACT_LIST, compact)
+        dev.kernel_times()
+        assert L.lib().msm_fm_loss_grad(dev.h, L.dptr(loss), None, 0, 0) == 0
+        t = dev.kernel_times()
+        assert (t["density"][1], t["force"][1]) == (1, 1), (compact, t)
+        assert _hip_error(lambda: dev.dyn_damp(1, 0.0, ctrl.H))      # (no kernel leaves the note)
+        t = dev.kernel_times()
+        assert (t["density"][1], t["force"][1]) == (1, 1), (compact, t)
+
+
 @pytest.mark.parametrize("name", sorted(CASES))
 def test_host_path(fake, name):
     r = subprocess.run([sys.executable, os.path.abspath(__file__), name, fake],
