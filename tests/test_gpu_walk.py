@@ -70,3 +70,52 @@ def test_walk_passes_vs_oracle(orc, name):
     assert dd <= 1e-13
     assert de <= 1e-13 and et <= 1e-12
     assert da <= 1e-13
+
+
+@pytest.mark.parametrize("name", ["fs-250", "eam-8k", "fs-16k", "eam-39k", "fs-130k", "cuni-1k",
+                                  "cuni-41k"])
+def test_lost_atoms_leave_their_neighbours_alone(orc, name):
+    """Atoms that went to NaN, infinity or 1e200 A since the list was built are outside every cutoff:
+    energies and stresses of the others, the forces that come with them, and those of the force pass
+    with a global table are those of the sums without them."""
+    box, ctrl, ft, _ = _case(name)
+    fc = md.MDForceClassGPU(ForceTable=ft)
+    md.Register_ForceClass(ft.PotType, fc)
+    md.Initialize_Globle_Variables_DEV(box, ctrl, fc)
+    md.Init_Forcetable_Dev(box, ctrl, fc)
+    dev = fc.Device
+    dev.build_neighbors()
+    x = box.XP.copy()
+    lost = [7, 100, 150, 201]
+    x[7, 0] = np.nan
+    x[100] = [np.inf, 0.0, -np.inf]
+    x[150, 2] = 1e200
+    x[201] = np.nan
+    dev.put_atoms(x)
+    it = box.ITYP - 1
+    kv, ind = orc.nlist("full", box.XP, it, box.STATU, box.BOXLOW, box.ZL, ctrl.IFPD, ctrl.NB_RM,
+                        ctrl.NB_MXNBS)
+    ru2, t = float(np.max(ctrl.RU)) ** 2, orc.from_mdlib(ft)
+    fo, do, eo = orc.force_full(np.asfortranarray(x), it, box.STATU, kv, ind, box.ZL, ctrl.IFPD,
+                                ru2, t)
+    ao, aabs = orc.atomic_stress_full(np.asfortranarray(x), it, box.STATU, kv, ind, box.ZL,
+                                      ctrl.IFPD, ru2, t, do, with_abs=True)
+    rest = np.setdiff1d(np.arange(box.NPRT), lost)
+    assert np.isfinite(fo[rest]).all() and np.isfinite(ao[rest]).all()
+    dev.calc_epot()
+    e = dev.get_epot()[rest]
+    dev.calc_force()
+    f, d = dev.get_forces()[rest], dev.get_den()[rest]
+    a = dev.calc_atomic_stress()[rest]
+    fs = dev.get_forces()[rest]
+    if dev.pass_kernel() == "lds_table":
+        f = fs
+    dev.close()
+    bad = {k: int(np.sum(~np.isfinite(v).reshape(len(rest), -1).all(axis=1)))
+           for k, v in (("e", e), ("f", f), ("d", d), ("stress", a), ("f of stress", fs))}
+    print(f"{name}: n={box.NPRT} not finite {bad}")
+    assert not any(bad.values()), bad
+    assert np.max(np.abs(f - fo[rest])) <= 1e-10 and np.max(np.abs(fs - fo[rest])) <= 1e-10
+    assert np.max(np.abs(d - do[rest]) / np.maximum(1.0, np.abs(do[rest]))) <= 1e-13
+    assert np.max(np.abs(e - eo[rest])) <= 1e-13 * np.max(np.abs(eo[rest]))
+    assert np.max(np.abs(a - ao[rest])) <= 1e-13 * np.max(aabs[rest])
