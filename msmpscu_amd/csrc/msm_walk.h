@@ -73,7 +73,6 @@ struct Lane {
     unsigned ib;      // atom index
     int kv;           // list length (0: inactive)
     int sub;          // lane within the atom
-    int last;         // the lane's last slot
     int ti;           // type
 };
 
@@ -156,7 +155,7 @@ struct Knots<0> {
 };
 
 // A pair's place in the table.  ok: inside the cutoff with its knots in the window (q is in
-// bounds either way); odd: the pair goes the side road, which looks at it once more: those below
+// bounds either way); odd: the pair goes the side road: those below
 // the window, those that may need the minimum image (IMG = 0) and, where the cutoff does not lie
 // within the table, those above it (one unsigned comparison for all three).
 struct Place {
@@ -214,26 +213,50 @@ __device__ __forceinline__ void add_virial(double h, double sx, double sy, doubl
     v[5] = v[5] + sy * sz * h;
 }
 
-// V = 1: the half virial of every pair as well (components xx, yy, zz, xy, xz, yz).
-template <int MT, int IMG, int LG, int V>
-__device__ __forceinline__ void force_odd(const AtomsDev& a, const TabDev& t, const WalkDev& w,
-                                          const BoxDev& b, const Lane& q, int s, int cnt,
-                                          const double4& pi, double& fx, double& fy, double& fz,
-                                          double (&vir)[6]) {
+// The odd pairs of a group, one bit a slot.  The side road takes them from here and decides nothing
+// itself: the same comparison compiled twice may round differently, and a pair on the edge would be
+// lost or count twice.  WAVE: as masks of the wave, in scalar registers (full groups of the passes with
+// the knots in LDS); else every lane keeps its own bits (in a list's last group lanes stop at different
+// slots; 200 steps of 2,000 W atoms, with a global table, 2,152 us against 2,183 with masks).
+template <int G, int WAVE>
+struct OddPairs {
+    unsigned long long m[WAVE ? G : 1] = {}, any = 0;
+    unsigned bits = 0;
+    __device__ __forceinline__ void note(int u, bool odd) {
+        if constexpr (WAVE) {
+            m[u] = lanes_of(odd);
+            any |= m[u];
+        } else {
+            bits |= odd ? 1u << u : 0u;
+        }
+    }
+    __device__ __forceinline__ bool some() const { return WAVE ? any != 0 : bits != 0; }
+    __device__ __forceinline__ unsigned slots() const {
+        unsigned b = bits;
+        if constexpr (WAVE) {
+#pragma unroll
+            for (int u = 0; u < G; ++u) b |= (m[u] >> (threadIdx.x & 63) & 1ull) ? 1u << u : 0u;
+        }
+        return b;
+    }
+};
+
+// Forces of the odd pairs among slots s, s + 1, ... (bits), by the general formula from the global
+// table.  V = 1: the half virial of every pair as well (components xx, yy, zz, xy, xz, yz).
+template <int MT, int LG, int V>
+__device__ __forceinline__ void force_odd(const AtomsDev& a, const TabDev& t, const BoxDev& b,
+                                          const Lane& q, int s, unsigned bits, const double4& pi,
+                                          double& fx, double& fy, double& fz, double (&vir)[6]) {
 #pragma unroll 1
-    for (int u = 0; u < cnt; ++u) {
-        if (s + u > q.last) break;
-        const int j = slot_index(q, s + u, 8 + LG);
+    for (; bits; bits &= bits - 1) {
+        const int j = slot_index(q, s + __builtin_ctz(bits), 8 + LG);
         const double4 pj = a.pos[j];
         double sx = pi.x - pj.x, sy = pi.y - pj.y, sz = pi.z - pj.z;
-        if constexpr (IMG == 0) {
-            if (!place<0>(t, w, sx * sx + sy * sy + sz * sz).odd) continue;
-        }
         sx = min_image(sx, b.len[0], b.ilen[0]);
         sy = min_image(sy, b.len[1], b.ilen[1]);
         sz = min_image(sz, b.len[2], b.ilen[2]);
         const double r2 = sx * sx + sy * sy + sz * sz;
-        if (!(r2 <= t.ru2max) || (IMG == 1 && !place<1>(t, w, r2).odd)) continue;
+        if (!(r2 <= t.ru2max)) continue;
         int kind = t.kpair[0], kind1 = t.kpair[0];
         if constexpr (MT) {
             const int tj = a.ityp[j];
@@ -272,7 +295,7 @@ __device__ __forceinline__ void force_slots(const AtomsDev& a, const TabDev& t, 
         tj[u] = MT ? at(a.ityp, j << 2) : 0;
     }
     if constexpr (FULL) next_slots<G, LG>(q, s, js);
-    unsigned long long odd = 0;
+    OddPairs<G, FULL && TL> odd;
 #pragma unroll
     for (int u = 0; u < G; ++u) {
         if (!FULL && u > 0 && (s + u) * L >= q.kv) break;
@@ -309,9 +332,10 @@ __device__ __forceinline__ void force_slots(const AtomsDev& a, const TabDev& t, 
         fy = fy + ft * sy;
         fz = fz + ft * sz;
         if constexpr (V) add_virial(0.5 * ft, sx, sy, sz, vir);
-        odd |= lanes_of(p.odd && valid);
+        odd.note(u, p.odd && valid);
     }
-    if (odd) force_odd<MT, IMG, LG, V>(a, t, w, b, q, s, G, pi, fx, fy, fz, vir);
+    if (__builtin_expect(odd.some(), 0))
+        force_odd<MT, LG, V>(a, t, b, q, s, odd.slots(), pi, fx, fy, fz, vir);
 }
 
 // Window of the upper part of the table for an LDS share: knots from k0 on.

@@ -34,27 +34,23 @@ namespace msm {
 // density
 // --------------------------------------------------------------------------------------------
 
-// Terms of the odd pairs among slots s .. s + cnt - 1, by the general formula from the global
+// Terms of the odd pairs among slots s, s + 1, ... (bits), by the general formula from the global
 // table.
-template <int MT, int IMG, int LG>
-__device__ __forceinline__ double density_odd(const AtomsDev& a, const TabDev& t, const WalkDev& w,
-                                              const BoxDev& b, const Lane& q, int s, int cnt,
-                                              double px, double py, double pz, double den) {
+template <int MT, int LG>
+__device__ __forceinline__ double density_odd(const AtomsDev& a, const TabDev& t, const BoxDev& b,
+                                              const Lane& q, int s, unsigned bits, double px,
+                                              double py, double pz, double den) {
 #pragma unroll 1
-    for (int u = 0; u < cnt; ++u) {
-        if (s + u > q.last) break;
-        const int j = slot_index(q, s + u, 8 + LG);
+    for (; bits; bits &= bits - 1) {
+        const int j = slot_index(q, s + __builtin_ctz(bits), 8 + LG);
         const double2 qxy = *reinterpret_cast<const double2*>(&a.pos[j]);
         const double qz = a.pos[j].z;
         double sx = px - qxy.x, sy = py - qxy.y, sz = pz - qz;
-        if constexpr (IMG == 0) {
-            if (!place<0>(t, w, sx * sx + sy * sy + sz * sz).odd) continue;
-        }
         sx = min_image(sx, b.len[0], b.ilen[0]);
         sy = min_image(sy, b.len[1], b.ilen[1]);
         sz = min_image(sz, b.len[2], b.ilen[2]);
         const double r2 = sx * sx + sy * sy + sz * sz;
-        if (!(r2 <= t.ru2max) || (IMG == 1 && !place<1>(t, w, r2).odd)) continue;
+        if (!(r2 <= t.ru2max)) continue;
         const int kind = MT ? t.kpair[q.ti * t.ngroup + a.ityp[j]] : t.kpair[0];
         double inv_r;
         const double sk = table_coord(r2, t.csi, inv_r);
@@ -87,7 +83,7 @@ __device__ __forceinline__ double density_slots(const AtomsDev& a, const TabDev&
         tj[u] = MT ? at(a.ityp, j << 2) : 0;
     }
     if constexpr (FULL) next_slots<G, LG>(q, s, js);
-    unsigned long long odd = 0;
+    OddPairs<G, FULL && TL> odd;
 #pragma unroll
     for (int u = 0; u < G; ++u) {
         if (!FULL && u > 0 && (s + u) * L >= q.kv) break;
@@ -103,9 +99,10 @@ __device__ __forceinline__ double density_slots(const AtomsDev& a, const TabDev&
         kn.den(p.q + (MT ? s_row[q.ti * t.ngroup + tj[u]] : 0), v, dv);
         v = v + p.dk * dv;
         den = den + ((p.ok && valid) ? v : 0.0);
-        odd |= lanes_of(p.odd && valid);
+        odd.note(u, p.odd && valid);
     }
-    if (odd) den = density_odd<MT, IMG, LG>(a, t, w, b, q, s, G, px, py, pz, den);
+    if (__builtin_expect(odd.some(), 0))
+        den = density_odd<MT, LG>(a, t, b, q, s, odd.slots(), px, py, pz, den);
     return den;
 }
 
@@ -113,7 +110,7 @@ template <int MB, int MT, int EAM, int L, int TL>
 __global__ __launch_bounds__(TL ? kLtMaxBlock : kBlock) void k_density_w(
     AtomsDev a, ListDev l, TabDev t, BoxDev box0, const BoxDev* __restrict__ boxes, WalkDev w,
     int* err) {
-    constexpr int LG = ilog2(L), G = group_d(L), A = 64 / L;
+    constexpr int G = group_d(L), A = 64 / L;
     extern __shared__ double s_dyn[];
     __shared__ int s_row[MT ? kMaxGroup * kMaxGroup : 1];
     Knots<TL> kn;
@@ -160,7 +157,6 @@ __global__ __launch_bounds__(TL ? kLtMaxBlock : kBlock) void k_density_w(
         const bool active = have && (st & STATU_ACTIVE) == STATU_ACTIVE;
         q.kv = active ? kv : 0;
         q.sub = sub;
-        q.last = ((q.kv - sub + L - 1) >> LG) - 1;
         const bool fast = w.kimg > 0 && !__any(active && !inner(b, w.margin, pxy.x, pxy.y, pz));
         double den = 0.0;
         if (q.kv > 0) {
@@ -207,7 +203,7 @@ template <int MB, int MT, int MODE, int L, int TL>
 __global__ __launch_bounds__(TL ? kLtMaxBlock : kBlock) void k_force_w(
     AtomsDev a, ListDev l, TabDev t, BoxDev box0, const BoxDev* __restrict__ boxes, StepParams sp,
     WalkDev w) {
-    constexpr int LG = ilog2(L), G = group_f(L), A = 64 / L;
+    constexpr int G = group_f(L), A = 64 / L;
     extern __shared__ double2 s_dyn2[];
     __shared__ int s_row[MT ? kMaxGroup * kMaxGroup : 1];
     Knots<TL> kn;
@@ -256,7 +252,6 @@ __global__ __launch_bounds__(TL ? kLtMaxBlock : kBlock) void k_force_w(
         const bool active = have && (st & STATU_ACTIVE) == STATU_ACTIVE;
         q.kv = active ? kv : 0;
         q.sub = sub;
-        q.last = ((q.kv - sub + L - 1) >> LG) - 1;
         const bool fast = w.kimg > 0 && !__any(active && !inner(b, w.margin, pi.x, pi.y, pi.z));
         double fx = 0.0, fy = 0.0, fz = 0.0, vir[6];
         if (q.kv > 0) {

@@ -12,26 +12,21 @@ namespace msm {
 
 namespace {
 
-template <int MT, int IMG, int LG>
-__device__ __forceinline__ void energy_odd(const AtomsDev& a, const TabDev& t, const WalkDev& w,
-                                           const BoxDev& b, const Lane& q, int s, int cnt,
-                                           double px, double py, double pz, double& er,
-                                           double& den) {
+template <int MT, int LG>
+__device__ __forceinline__ void energy_odd(const AtomsDev& a, const TabDev& t, const BoxDev& b,
+                                           const Lane& q, int s, unsigned bits, double px,
+                                           double py, double pz, double& er, double& den) {
 #pragma unroll 1
-    for (int u = 0; u < cnt; ++u) {
-        if (s + u > q.last) break;
-        const int j = slot_index(q, s + u, 8 + LG);
+    for (; bits; bits &= bits - 1) {
+        const int j = slot_index(q, s + __builtin_ctz(bits), 8 + LG);
         const double2 qxy = *reinterpret_cast<const double2*>(&a.pos[j]);
         const double qz = a.pos[j].z;
         double sx = px - qxy.x, sy = py - qxy.y, sz = pz - qz;
-        if constexpr (IMG == 0) {
-            if (!place<0>(t, w, sx * sx + sy * sy + sz * sz).odd) continue;
-        }
         sx = min_image(sx, b.len[0], b.ilen[0]);
         sy = min_image(sy, b.len[1], b.ilen[1]);
         sz = min_image(sz, b.len[2], b.ilen[2]);
         const double r2 = sx * sx + sy * sy + sz * sz;
-        if (!(r2 <= t.ru2max) || (IMG == 1 && !place<1>(t, w, r2).odd)) continue;
+        if (!(r2 <= t.ru2max)) continue;
         const int kind = MT ? t.kpair[q.ti * t.ngroup + a.ityp[j]] : t.kpair[0];
         double inv_r;
         const double sk = table_coord(r2, t.csi, inv_r);
@@ -63,7 +58,7 @@ __device__ __forceinline__ void energy_slots(const AtomsDev& a, const TabDev& t,
         tj[u] = MT ? at(a.ityp, j << 2) : 0;
     }
     if constexpr (FULL) next_slots<G, LG>(q, s, js);
-    unsigned long long odd = 0;
+    OddPairs<G, FULL && TL> odd;
 #pragma unroll
     for (int u = 0; u < G; ++u) {
         if (!FULL && u > 0 && (s + u) * L >= q.kv) break;
@@ -81,9 +76,10 @@ __device__ __forceinline__ void energy_slots(const AtomsDev& a, const TabDev& t,
         d = d + p.dk * dd;
         er = er + (use ? v : 0.0);
         den = den + (use ? d : 0.0);
-        odd |= lanes_of(p.odd && (FULL || listed<L>(q, s + u)));
+        odd.note(u, p.odd && (FULL || listed<L>(q, s + u)));
     }
-    if (odd) energy_odd<MT, IMG, LG>(a, t, w, b, q, s, G, px, py, pz, er, den);
+    if (__builtin_expect(odd.some(), 0))
+        energy_odd<MT, LG>(a, t, b, q, s, odd.slots(), px, py, pz, er, den);
 }
 
 }  // namespace
@@ -93,7 +89,7 @@ template <int MB, int MT, int EAM, int L, int TL>
 __global__ __launch_bounds__(TL ? kLtMaxBlock : kBlock) void k_energy_w(
     AtomsDev a, ListDev l, TabDev t, BoxDev box0, const BoxDev* __restrict__ boxes, WalkDev w,
     double* __restrict__ rho_out, int write_fp, int* err) {
-    constexpr int LG = ilog2(L), G = 3, A = 64 / L;
+    constexpr int G = 3, A = 64 / L;
     extern __shared__ double2 s_dyn2[];
     __shared__ int s_row[MT ? kMaxGroup * kMaxGroup : 1];
     Knots<TL> kn;
@@ -137,7 +133,6 @@ __global__ __launch_bounds__(TL ? kLtMaxBlock : kBlock) void k_energy_w(
         const bool active = have && (st & STATU_ACTIVE) == STATU_ACTIVE;
         q.kv = active ? kv : 0;
         q.sub = sub;
-        q.last = ((q.kv - sub + L - 1) >> LG) - 1;
         const bool fast = w.kimg > 0 && !__any(active && !inner(b, w.margin, pxy.x, pxy.y, pz));
         double er = 0.0, den = 0.0;
         if (q.kv > 0) {
@@ -188,7 +183,7 @@ template <int MB, int MT, int L, int TL>
 __global__ __launch_bounds__(TL ? kLtMaxBlock : kBlock) void k_virial_w(
     AtomsDev a, ListDev l, TabDev t, BoxDev box0, const BoxDev* __restrict__ boxes, WalkDev w,
     double* __restrict__ vir) {
-    constexpr int LG = ilog2(L), G = 3, A = 64 / L;
+    constexpr int G = 3, A = 64 / L;
     extern __shared__ double2 s_dyn2[];
     __shared__ int s_row[MT ? kMaxGroup * kMaxGroup : 1];
     Knots<TL> kn;
@@ -231,7 +226,6 @@ __global__ __launch_bounds__(TL ? kLtMaxBlock : kBlock) void k_virial_w(
         const bool active = have && (st & STATU_ACTIVE) == STATU_ACTIVE;
         q.kv = active ? kv : 0;
         q.sub = sub;
-        q.last = ((q.kv - sub + L - 1) >> LG) - 1;
         const bool fast = w.kimg > 0 && !__any(active && !inner(b, w.margin, pi.x, pi.y, pi.z));
         double fx = 0.0, fy = 0.0, fz = 0.0, p[6] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
         if (q.kv > 0) {

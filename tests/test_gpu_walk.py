@@ -119,3 +119,54 @@ def test_lost_atoms_leave_their_neighbours_alone(orc, name):
     assert np.max(np.abs(d - do[rest]) / np.maximum(1.0, np.abs(do[rest]))) <= 1e-13
     assert np.max(np.abs(e - eo[rest])) <= 1e-13 * np.max(np.abs(eo[rest]))
     assert np.max(np.abs(a - ao[rest])) <= 1e-13 * np.max(aabs[rest])
+
+
+@pytest.mark.parametrize("name", ["eam-39k", "fs-130k", "cuni-41k"])
+def test_pairs_at_the_edge_of_the_window(orc, name):
+    """Hundreds of pairs at the distance where the knots in LDS begin (three eighths of the table),
+    as near to it as coordinates go, in all directions: each counts once, on whichever side of the edge
+    rounding puts it.  Bars as above, relative to the largest absolute value."""
+    box, ctrl, ft, _ = _case(name)
+    rng = np.random.default_rng(17)
+    edge = 3 * ((ft.NTAB + 2) // 8) / ft.CSI
+    r = edge * edge
+    x = box.XP.copy()
+    fc = md.MDForceClassGPU(ForceTable=ft)
+    md.Register_ForceClass(ft.PotType, fc)
+    md.Initialize_Globle_Variables_DEV(box, ctrl, fc)
+    md.Init_Forcetable_Dev(box, ctrl, fc)
+    dev = fc.Device
+    dev.build_neighbors()
+    kv, ind = dev.get_neighbors()
+    used = np.zeros(box.NPRT, dtype=bool)
+    inside = np.all((x - box.BOXLOW > 1.0) & (box.BOXLOW + box.ZL - x > 1.0), axis=1)
+    pairs = 0
+    for i in range(box.NPRT):
+        js = ind[i, :kv[i]] - 1
+        if pairs == 3000 or used[i] or not inside[i] or not kv[i] or used[js].any():
+            continue
+        j = js[np.argmin(np.sum((box.XP[js] - box.XP[i]) ** 2, axis=1))]
+        d = rng.normal(size=3)
+        x[j] = x[i] + d * (r / np.linalg.norm(d))
+        used[js] = used[i] = True
+        pairs += 1
+    assert pairs > 100
+    dev.put_atoms(x)
+    it = box.ITYP - 1
+    okv, oind = orc.nlist("full", box.XP, it, box.STATU, box.BOXLOW, box.ZL, ctrl.IFPD, ctrl.NB_RM,
+                          ctrl.NB_MXNBS)
+    ru2, t = float(np.max(ctrl.RU)) ** 2, orc.from_mdlib(ft)
+    fo, do, eo = orc.force_full(np.asfortranarray(x), it, box.STATU, okv, oind, box.ZL, ctrl.IFPD,
+                                ru2, t)
+    ao, aabs = orc.atomic_stress_full(np.asfortranarray(x), it, box.STATU, okv, oind, box.ZL,
+                                      ctrl.IFPD, ru2, t, do, with_abs=True)
+    dev.calc_force()
+    f, d = dev.get_forces(), dev.get_den()
+    dev.calc_epot()
+    e, a = dev.get_epot(), dev.calc_atomic_stress()
+    dev.close()
+    err = [np.max(np.abs(f - fo)) / np.max(np.abs(fo)), np.max(np.abs(d - do)) / np.max(np.abs(do)),
+           np.max(np.abs(e - eo)) / np.max(np.abs(eo)), np.max(np.abs(a - ao)) / np.max(aabs)]
+    print(f"{name}: {pairs} pairs at {r:.4f} A, force up to {np.max(np.abs(fo)):.3g}, errors "
+          + " ".join(f"{v:.2e}" for v in err))
+    assert err[0] <= 1e-12 and err[1] <= 1e-13 and err[2] <= 1e-13 and err[3] <= 1e-12
