@@ -344,6 +344,12 @@ int msm_set_option(msm_sim* sim, int option, int value);
  * range of its XCD's atom chunks; 1 the workgroups of an XCD take its chunks round-robin, so the
  * chunks in flight on one XCD are adjacent and share that XCD's L2. */
 #define MSM_OPT_CHUNK_SWEEP      15
+/* The density, force, energy and stress passes walk the list with 32-bit offsets below this many
+ * atoms (1 .. 2^27, the default); from there on the kernels with 64-bit offsets run. */
+#define MSM_OPT_WALK_ATOMS       16
+/* Read-only: lanes per atom of that walk's density and force pass (1 to 32); 0: another kernel. */
+#define MSM_OPT_DENSITY_WALK     17
+#define MSM_OPT_FORCE_WALK       18
 /* Read-only: the density/force kernels the current options and list select (MSM_PASS_*). */
 #define MSM_OPT_PASS_KERNEL      13
 #define MSM_PASS_BRICKS      0  /* LDS-staged positions, global table */

@@ -116,6 +116,9 @@ MSM_OPT_NLIST_KERNEL = 3
 MSM_OPT_FORCE_PATH = 4
 MSM_OPT_COMPACT_LIST = 5
 MSM_OPT_CHUNK_SWEEP = 15
+MSM_OPT_WALK_ATOMS = 16
+MSM_OPT_DENSITY_WALK = 17
+MSM_OPT_FORCE_WALK = 18
 MSM_OPT_TABLE_LDS = 6
 MSM_OPT_LT_DENSITY_BLOCK = 7
 MSM_OPT_LT_DENSITY_WGS = 8

@@ -138,6 +138,7 @@ struct msm_sim {
     int cell_brick = 1;    // cells are numbered in bricks of cell_brick^3 (1: row-major)
     msm::LtShape lt = kLtDefault;  // block / workgroups per CU of the LDS-table passes
     int auto_pass = 1;     // MSM_PATH_BY_SIZE: lanes and table placement by size (walk_plan)
+    int walk_atoms = msm::kWalkMaxAtoms;  // the list walk is for fewer atoms than this
     int compact = 0;       // global-list path: force pass reads the density pass's in-cutoff list
 
     // adjoint scratch (allocated on first use)
@@ -709,7 +710,7 @@ bool size_plan(const msm_sim* s, int force, msm::WalkPlan& p) {
 
 // The list-walk pass (msm_walk.hip) and its shape; false: another kernel runs.
 bool walk_plan(const msm_sim* s, int force, msm::WalkPlan& p) {
-    if (s->n >= msm::kWalkMaxAtoms || s->compact) return false;
+    if (s->n >= s->walk_atoms || s->compact) return false;
     const int fp = eff_path(s);
     if (fp != 1 && fp != 2 && fp != 4) return false;
     walk_geometry(s, p);
@@ -735,7 +736,7 @@ void enqueue_density(msm_sim* s);
 
 // The list walk of the energy and virial passes, which no option fixes; false: the general passes.
 bool aux_plan(const msm_sim* s, msm::WalkPlan& p) {
-    if (s->n >= msm::kWalkMaxAtoms) return false;
+    if (s->n >= s->walk_atoms) return false;
     walk_geometry(s, p);
     p.block = 1024;
     p.wgs = 1;
@@ -2301,6 +2302,12 @@ int msm_set_option(msm_sim* s, int option, int value) {
                 return set_err(s, MSM_ERR_ARG, "force lanes must be 0, 1, 2 or 4");
             set_pass(s, s->force_lanes, value);
             return MSM_OK;
+        case MSM_OPT_WALK_ATOMS:
+            if (value < 1 || value > msm::kWalkMaxAtoms)
+                return set_err(s, MSM_ERR_ARG, "list walk atoms must be 1..2^27");
+            s->walk_atoms = value;
+            clear_graphs(s);
+            return MSM_OK;
         case MSM_OPT_LT_DENSITY_BLOCK:
         case MSM_OPT_LT_FORCE_BLOCK:
             if (value != 256 && value != 512 && value != 1024)
@@ -2331,6 +2338,13 @@ static int pass_kernel(const msm_sim* s) {
     return MSM_PASS_BRICKS;
 }
 
+// Lanes per atom of the list-walk density (force: force) pass that these options select, or 0.
+static int walk_lanes(const msm_sim* s, int force) {
+    msm::WalkPlan wp{};
+    if (use_staged(s) || use_brick_table(s) || !walk_plan(s, force, wp)) return 0;
+    return wp.lanes;
+}
+
 int msm_get_option(msm_sim* s, int option, int* value) {
     if (!s || !value) return MSM_ERR_ARG;
     switch (option) {
@@ -2350,6 +2364,12 @@ int msm_get_option(msm_sim* s, int option, int* value) {
         case MSM_OPT_BRICK_LANES: *value = s->bt_lanes; return MSM_OK;
         case MSM_OPT_FORCE_LANES: *value = s->force_lanes; return MSM_OK;
         case MSM_OPT_CHUNK_SWEEP: *value = s->lt.sweep; return MSM_OK;
+        case MSM_OPT_WALK_ATOMS: *value = s->walk_atoms; return MSM_OK;
+        case MSM_OPT_DENSITY_WALK:
+        case MSM_OPT_FORCE_WALK:
+            if (!s->has_table) return set_err(s, MSM_ERR_STATE, "no force table");
+            *value = walk_lanes(s, option == MSM_OPT_FORCE_WALK);
+            return MSM_OK;
         case MSM_OPT_PASS_KERNEL:
             if (!s->has_table) return set_err(s, MSM_ERR_STATE, "no force table");
             *value = pass_kernel(s);

@@ -599,6 +599,11 @@ class DeviceMD:
         from ._lib import MSM_OPT_PASS_KERNEL, PASS_KERNELS
         return PASS_KERNELS[self.get_option(MSM_OPT_PASS_KERNEL)]
 
+    def walk_lanes(self):
+        """Lanes per atom of the list-walk (density, force) pass, 0 where another kernel runs."""
+        from ._lib import MSM_OPT_DENSITY_WALK, MSM_OPT_FORCE_WALK
+        return self.get_option(MSM_OPT_DENSITY_WALK), self.get_option(MSM_OPT_FORCE_WALK)
+
     def autotune(self, reps: int = 3) -> dict:
         """Times the kernel variants on the current atoms and list and keeps the fastest
         (msm_autotune); returns the choice and the chosen per-pass times."""
