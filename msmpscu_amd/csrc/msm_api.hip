@@ -1363,17 +1363,25 @@ int msm_get_atoms(msm_sim* s, double* xp, double* xp1, double* fp, int* statu, d
     const AtomsDev a = atoms_view(s, s->scur, s->pcur);
     const int* gid = s->set[s->scur].gid;
     void* const host[5] = {xp, xp1, fp, dis, statu};
-    // everything through one device block, or array by array where that would be large
-    const bool whole = m <= (size_t(1) << 22);
+    auto bytes_of = [&](int k) {
+        return !host[k] ? size_t(0) : k < 4 ? 3 * m * sizeof(double) : m * sizeof(int);
+    };
+    // everything through one device block, or array by array where that would be large or cannot be had
+    bool whole = m <= (size_t(1) << 22);
+    if (whole) {
+        size_t all = 0;
+        for (int k = 0; k < 5; ++k) all += bytes_of(k);
+        whole = dreserve(s, &s->d_stage, (all + 7) / 8, s->cap_stage) == MSM_OK;
+        if (!whole) (void)hipGetLastError();
+    }
     msm::CopyPart parts[5];
     int np = 0, what = 0;
     size_t total = 0;
     for (int k = 0; k < 5; ++k) {
         if (host[k]) {
-            const size_t bytes = k < 4 ? 3 * m * sizeof(double) : m * sizeof(int);
-            parts[np++] = {total, bytes, host[k]};
+            parts[np++] = {total, bytes_of(k), host[k]};
             what |= 1 << k;
-            total += bytes;
+            total += bytes_of(k);
         }
         if (!what || (whole && k < 4)) continue;
         const int rc = dreserve(s, &s->d_stage, (total + 7) / 8, s->cap_stage);

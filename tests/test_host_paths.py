@@ -256,6 +256,27 @@ def density_is_timed_once(f):
         assert (t["density"][1], t["force"][1]) == (1, 1), (compact, t)
 
 
+@case
+def copy_out_in_little_memory(f):
+    """All arrays at once leave through one block of 100 bytes an atom; where that cannot be had, one
+    after another through 24."""
+    import msmpscu_amd._lib as L
+    dev, boxes, _ = _device((16, 16, 17))
+    n = boxes[0].NPRT
+    f.fake_dev_limit(24 * n)
+    for _ in range(2):
+        assert all(set(a.tobytes()) == {0x5a} for a in dev.get_atoms())
+    dev.close()
+    dev, boxes, _ = (f.fake_dev_limit(-1), _device((16, 16, 17)))[1]
+    f.fake_dev_limit(24 * n - 1)
+    try:
+        dev.get_atoms()
+        raise AssertionError("copied through nothing")
+    except L.MSMError as e:
+        assert e.code == 3      # MSM_ERR_NOMEM
+    dev.close()
+
+
 @pytest.mark.parametrize("name", sorted(CASES))
 def test_host_path(fake, name):
     r = subprocess.run([sys.executable, os.path.abspath(__file__), name, fake],
