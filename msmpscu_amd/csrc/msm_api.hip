@@ -64,10 +64,11 @@ struct msm_sim {
     // force table
     bool has_table = false;
     TabDev tab{};
+    double* d_knots = nullptr;  // one block: knot values alone (d_f2, d_e2, d_b1 point into it)
     double* d_b1 = nullptr;
     double2 *d_b2 = nullptr, *d_f2 = nullptr, *d_e2 = nullptr;
     double4 *d_f4 = nullptr, *d_e4 = nullptr, *d_m4 = nullptr;
-    size_t cap_b1 = 0, cap_f2 = 0, cap_e2 = 0, cap_b2 = 0, cap_f4 = 0, cap_e4 = 0, cap_m4 = 0;  // elements allocated
+    size_t cap_knots = 0, cap_b2 = 0, cap_f4 = 0, cap_e4 = 0, cap_m4 = 0;  // elements allocated
     int tab_ngroup = 0;
 
     // control
@@ -1000,9 +1001,7 @@ int msm_destroy(msm_sim* s) {
     }
     for (hipEvent_t e : s->evpool) (void)hipEventDestroy(e);
     if (s->fm_ev) (void)hipEventDestroy(s->fm_ev);
-    dfree(&s->d_b1);
-    dfree(&s->d_f2);
-    dfree(&s->d_e2);
+    dfree(&s->d_knots);
     dfree(&s->d_b2);
     dfree(&s->d_f4);
     dfree(&s->d_e4);
@@ -1066,8 +1065,6 @@ int msm_set_force_table(msm_sim* s, int pot_type, int ngroup, int nkind, int nta
     };
     std::vector<double2> hb2(static_cast<size_t>(nkind) * ntab2);
     std::vector<double4> hf4(static_cast<size_t>(nkind) * ntab2), he4(hf4.size());
-    std::vector<double> hb1(hb2.size());
-    std::vector<double2> hf2(hb2.size()), hen2(hb2.size());
     for (int k = 0; k < nkind; ++k)
         for (int i = 0; i < ntab2; ++i) {
             const size_t a = static_cast<size_t>(k) * ntab2 + i;
@@ -1078,9 +1075,6 @@ int msm_set_force_table(msm_sim* s, int pot_type, int ngroup, int nkind, int nta
             hf4[a] = make_double4(fr, fr1 - fr, fb, fb1 - fb);
             const double pr = knot(potr, k, i), pr1 = knot(potr, k, i + 1);
             he4[a] = make_double4(pr, pr1 - pr, pb, pb1 - pb);
-            hb1[a] = pb;
-            hf2[a] = make_double2(fr, fb);
-            hen2[a] = make_double2(pr, pb);
         }
     TabDev t;
     std::memset(&t, 0, sizeof(t));  // byte-wise comparable with the current table
@@ -1099,16 +1093,15 @@ int msm_set_force_table(msm_sim* s, int pot_type, int ngroup, int nkind, int nta
         for (int i = 0; i < ngroup; ++i)
             if (kembd[i] < 1 || kembd[i] > nkind1)
                 return set_err(s, MSM_ERR_ARG, "KEMBD entry out of range");
-    int rc = dreserve(s, &s->d_b2, hb2.size(), s->cap_b2);
+    const size_t nkn = hb2.size();
+    int rc = dreserve(s, &s->d_b2, nkn, s->cap_b2);
     if (rc == MSM_OK) rc = dreserve(s, &s->d_f4, hf4.size(), s->cap_f4);
     if (rc == MSM_OK) rc = dreserve(s, &s->d_e4, he4.size(), s->cap_e4);
-    if (rc == MSM_OK) rc = dreserve(s, &s->d_b1, hb1.size(), s->cap_b1);
-    if (rc == MSM_OK) rc = dreserve(s, &s->d_f2, hf2.size(), s->cap_f2);
-    if (rc == MSM_OK) rc = dreserve(s, &s->d_e2, hen2.size(), s->cap_e2);
+    if (rc == MSM_OK) rc = dreserve(s, &s->d_knots, 5 * nkn, s->cap_knots);
     if (rc != MSM_OK) return rc;
-    HIPCHK(s, hipMemcpy(s->d_b1, hb1.data(), hb1.size() * sizeof(double), hipMemcpyHostToDevice));
-    HIPCHK(s, hipMemcpy(s->d_f2, hf2.data(), hf2.size() * sizeof(double2), hipMemcpyHostToDevice));
-    HIPCHK(s, hipMemcpy(s->d_e2, hen2.data(), hen2.size() * sizeof(double2), hipMemcpyHostToDevice));
+    s->d_f2 = reinterpret_cast<double2*>(s->d_knots);
+    s->d_e2 = s->d_f2 + nkn;
+    s->d_b1 = s->d_knots + 4 * nkn;
     HIPCHK(s, hipMemcpy(s->d_b2, hb2.data(), hb2.size() * sizeof(double2), hipMemcpyHostToDevice));
     HIPCHK(s, hipMemcpy(s->d_f4, hf4.data(), hf4.size() * sizeof(double4), hipMemcpyHostToDevice));
     HIPCHK(s, hipMemcpy(s->d_e4, he4.data(), he4.size() * sizeof(double4), hipMemcpyHostToDevice));
@@ -1140,6 +1133,9 @@ int msm_set_force_table(msm_sim* s, int pot_type, int ngroup, int nkind, int nta
         t.nkind1 = 1;
         t.rhod = 1.0;
     }
+    // the values alone are taken from these on the device (three copies of their own: 0.1 ms a table)
+    msm::launch_knot_values(nkn, s->d_b2, s->d_f4, s->d_e4, s->d_b1, s->d_f2, s->d_e2, s->stream);
+    HIPCHK(s, hipGetLastError());
     t.b1 = s->d_b1;
     t.f2 = s->d_f2;
     t.e2 = s->d_e2;

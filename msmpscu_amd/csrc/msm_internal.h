@@ -117,6 +117,9 @@ struct SortBufs {
 
 // ---- launchers (msm_kernels.hip) ----
 void launch_fill_int(int* p, int v, int n, hipStream_t s);
+// The knot values alone (b1, f2, e2 of TabDev) of the n knots of all kinds in b2, f4, e4.
+void launch_knot_values(size_t n, const double2* b2, const double4* f4, const double4* e4, double* b1,
+                        double2* f2, double2* e2, hipStream_t s);
 // Cell sort (msm_cells.hip): src in its current order -> dst in cell order; sb.count must hold zeros
 // (it does again afterwards).  Boxes within both limits sort in one workgroup.
 constexpr int kSortSmallAtoms = 8192, kSortSmallCells = 12288;

@@ -37,6 +37,24 @@ void launch_fill_int(int* p, int v, int n, hipStream_t s) {
     hipLaunchKernelGGL(k_fill_int, dim3(grid_for(n)), dim3(kBlock), 0, s, p, v, n);
 }
 
+__global__ void k_knot_values(size_t n, const double2* __restrict__ b2,
+                              const double4* __restrict__ f4, const double4* __restrict__ e4,
+                              double* __restrict__ b1, double2* __restrict__ f2,
+                              double2* __restrict__ e2) {
+    const size_t k = static_cast<size_t>(blockIdx.x) * blockDim.x + threadIdx.x;
+    if (k >= n) return;
+    b1[k] = b2[k].x;
+    f2[k] = make_double2(f4[k].x, f4[k].z);
+    e2[k] = make_double2(e4[k].x, e4[k].z);
+}
+
+void launch_knot_values(size_t n, const double2* b2, const double4* f4, const double4* e4, double* b1,
+                        double2* f2, double2* e2, hipStream_t s) {
+    if (n > 0)
+        hipLaunchKernelGGL(k_knot_values, dim3(static_cast<unsigned>((n + kBlock - 1) / kBlock)),
+                           dim3(kBlock), 0, s, n, b2, f4, e4, b1, f2, e2);
+}
+
 // --------------------------------------------------------------------------------------------
 // neighbour list: per-atom scan (the sort and the default list are in msm_cells.hip)
 // --------------------------------------------------------------------------------------------
