@@ -151,7 +151,9 @@ int msm_set_boxes(msm_sim* sim, int nbox, const int* natoms, const double* lo, c
 int msm_set_atoms(msm_sim* sim, int n, const double* xp, const double* xp1, const int* ityp,
                   const int* statu);
 
-/* Copy-out in the caller's atom order; any pointer may be NULL. */
+/* Copy-out in the caller's atom order; any pointer may be NULL.  Copies beyond 64 KB, in and out, go
+ * through pinned memory that the contexts of a GPU share (8 MB from the first such copy on, given back
+ * with the last context): one copy at a time, on up to eight host threads. */
 int msm_get_atoms(msm_sim* sim, double* xp, double* xp1, double* fp, int* statu, double* dis);
 /* CopyXPFrom_Host_to_Devices / CopyXP1From_Host_to_Devices (MD_Globle_Variables_GPU.F90:349-373):
  * positions and/or velocities (either may be NULL) of all atoms, (N,3) column-major in the
@@ -234,7 +236,8 @@ int msm_check_timestep(msm_sim* sim, double th, double mxd2, int* exceeded);
  * msm_dyn_damp: Do_DynDamp_Forsteps_DEV (:1809-1883) -- up to maxsteps of damping, predictor,
  * force, per-atom energy, stopping when max |EPOT_i - EPOT_i(previous)| <= mindele (before the
  * corrector), else corrector; the list is not rebuilt.  steps receives the iteration it stopped
- * at (maxsteps + 1 if it did not converge), delepot the last max |dEPOT|.
+ * at (maxsteps + 1 if it did not converge), delepot the last max |dEPOT|.  The calling thread watches
+ * for the device's note of each step without sleeping, and so occupies a host core meanwhile.
  * msm_calc_ekin, msm_scale_velocities and msm_dyn_damp need a built neighbour list (the atoms sit
  * in cell order on the device from the first msm_build_neighbors on). */
 int msm_damping(msm_sim* sim);

@@ -669,11 +669,18 @@ bool use_brick_table(const msm_sim* s) {
 }
 
 // Lanes per atom of a pass when no option fixes the kernel (s->auto_pass): enough that the pass
-// holds about 120,000 lanes (twice that for long lists), at least 2 (4).  Measured, density + force + 1/10 list per step: 2,000 W atoms
-// (26 neighbours) 37.9 us at 2 lanes, 21.2 / 19.5 / 19.2 at 8 / 16 / 32; 16,000 atoms 38.0 at 2,
-// 23.3 / 24.7 / 30.1; 54,000 atoms 30.1 / 32.0 / 38.1 at 2 / 4 / 8, 137,000 48.7 / 51.0 / 64.1;
-// Cu-Ni (86 neighbours) 42,600 atoms 131.9 / 100.5 / 93.8 at 2 / 4 / 8, 442,000 atoms 377.7 /
-// 374.8 / 421.6.
+// holds about 120,000 lanes (twice that for long lists), at least 2 (4).  Steps of msm_run with their
+// rebuilds, us, one workgroup of 1024 a CU with the knots in LDS | global memory:
+//              lanes       2      4      8  |     8     16     32
+//   W (26 neighbours)
+//    2,000              26.8      -      -  |  12.2   10.8   10.3
+//   16,000              28.1   21.6   18.5  |  14.6   16.4   22.9
+//   54,000              31.8   24.8   26.6  |  30.4      -      -
+//  138,000              38.3   42.5   50.9  |     -      -      -   (one lane 50.8)
+//   Cu-Ni (86 neighbours)
+//    4,000                 -      -      -  |  25.9   21.7   20.7
+//   42,600              99.3   66.8   59.3  |  72.5   79.0      -
+//  442,000             338.5  329.9  369.4  |     -      -      -
 int auto_lanes(const msm_sim* s) {
     const bool lng = s->kmean >= 48.0;
     int lanes = lng ? 4 : 2;
@@ -695,9 +702,12 @@ void walk_geometry(const msm_sim* s, msm::WalkPlan& p) {
 }
 
 // Lanes and table placement by size.  Filling the LDS window costs more than the global lookups it
-// saves below about 10^6 pairs: 16,000 W atoms at 8 lanes 25.6 us with it, 23.3 without; 54,000 at
-// 4 lanes 31.0, at 8 lanes from global memory 38.7; 42,600 Cu-Ni atoms at 8 lanes 93.8 with it,
-// 108.4 without.  false: a table too large for the LDS on a large box (the general passes).
+// saves below about 10^6 pairs (the table at auto_lanes: 16,000 W atoms and 54,000 on either side of it).
+// false: a table too large for the LDS on a large box, whose force pass is then one of the passes
+// without the walk (three kinds fill half a window with 6,780 knots each).  Cu-Ni, 10,000 knots,
+// steps with 8 lanes of the walk from global memory / without it: 42,600 atoms 75.9 / 91.3 us, 88,000
+// (7.5e6 pairs) 134 / 139, 187,000 239 / 256, 442,000 556 / 544: from 8e6 pairs on the two are close,
+// and the walk loses in the end.
 bool size_plan(const msm_sim* s, int force, msm::WalkPlan& p) {
     p.lanes = auto_lanes(s);
     p.tl = s->table_lds && p.lanes <= 8 && s->n * s->kmean >= 8.0e5 &&
@@ -720,11 +730,10 @@ bool walk_plan(const msm_sim* s, int force, msm::WalkPlan& p) {
     p.sweep = s->lt.sweep;
     if (s->auto_pass) {
         if (!size_plan(s, force, p)) return false;
-        // Several boxes: every lane loads its atom's box record, so one lane an atom as soon as that
-        // fills the chip (64 boxes, 428,674 W atoms, density / force 43.8 / 56.2 us with 2 lanes,
-        // 40.8 / 50.4 with 1; 12 boxes, 242,498 atoms 28.5 / 35.7 and 27.8 / 33.1).  In one box the
-        // two are equal from 265,000 atoms on, below two are better (182,250: 21.6 / 25.1 and
-        // 24.5 / 28.5).
+        // Several boxes: a lane loads its atom's box record too, so fewer lanes pay as soon as one an
+        // atom fills the chip.  Steps with 2 lanes / 1, us: 64 boxes, 432,000 W atoms 99.8 / 94.4, one
+        // box of as many 89.3 / 95.0; 12 boxes, 256,000 atoms 65.2 / 61.7, one of 265,000 61.9 / 64.9;
+        // 4 boxes, 182,000 atoms 51.7 / 57.8.
         if (p.tl && p.lanes == 2 && multibox(s) && s->n >= 200000) p.lanes = 1;
         return true;
     }

@@ -606,7 +606,8 @@ class DeviceMD:
 
     def autotune(self, reps: int = 3) -> dict:
         """Times the kernel variants on the current atoms and list and keeps the fastest
-        (msm_autotune); returns the choice and the chosen per-pass times."""
+        (msm_autotune); returns the choice (force_path -1: lanes and table placement by size) and
+        the chosen per-pass times."""
         ch = np.zeros(8, dtype=np.int32)
         ms = np.zeros(2)
         check(lib().msm_autotune(self.h, int(reps), iptr(ch), dptr(ms)), "msm_autotune", self.h)
