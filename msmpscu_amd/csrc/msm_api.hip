@@ -437,6 +437,8 @@ void enqueue_rebuild(msm_sim* s, bool keep_f = true) {
     const int nc = s->ncell_total;
     msm::launch_cell_sort(s->n, nc, s->d_boxes, a_src, s->set[src].gid, a_dst, s->set[dst].gid,
                           s->set[dst].cell, s->sb, keep_f ? 1 : 0, s->d_err, s->stream);
+    // a sort that was refused part way leaves the atoms where they are
+    if (hipPeekAtLastError() != hipSuccess) return;
     TimedScope tl(s, MSM_KCLASS_NLIST);
     if (s->nlist_kind == 1) {
         s->list_sidx = 0;
@@ -1548,8 +1550,9 @@ int msm_build_neighbors(msm_sim* s) {
     clear_flags(s);
     ready_counts(s);
     enqueue_rebuild(s);
-    s->has_list = true;
-    return read_flags(s);
+    rc = read_flags(s);
+    s->has_list = rc != MSM_ERR_HIP;
+    return rc;
 }
 
 int msm_get_neighbors(msm_sim* s, int* kvois, int* indi, int ld) {
@@ -2472,6 +2475,10 @@ int msm_autotune(msm_sim* s, int reps, int* choice, double* best_ms) {
         if ((rc = replan_bricks(s)) != MSM_OK) break;
         float ms = 0.f;
         rc = time_it([&] { enqueue_rebuild(s); }, ms);
+        if (rc == MSM_OK) {
+            const hipError_t e = hipGetLastError();
+            if (e != hipSuccess) rc = set_err(s, MSM_ERR_HIP, hipGetErrorString(e));
+        }
         if (rc != MSM_OK) break;
         if (g == 2 || ms < best_nl) {
             best_nl = ms;
@@ -2501,9 +2508,9 @@ int msm_autotune(msm_sim* s, int reps, int* choice, double* best_ms) {
             s->table_lds = 1;
             if (use_brick_table(s)) cands.push_back(c);
         }
-    // density + force passes
+    // density + force passes (one whose launch is refused is no candidate)
     float best = 0.f;
-    size_t bi = 0;
+    size_t bi = cands.size();
     for (size_t c = 0; c < cands.size() && rc == MSM_OK; ++c) {
         select(cands[c]);
         float ms = 0.f;
@@ -2511,11 +2518,12 @@ int msm_autotune(msm_sim* s, int reps, int* choice, double* best_ms) {
             enqueue_density(s);
             enqueue_force(s, 0, 1, 0.0);
         }, ms);
-        if (rc == MSM_OK && (c == 0 || ms < best)) {
+        if (hipGetLastError() == hipSuccess && rc == MSM_OK && (bi == cands.size() || ms < best)) {
             best = ms;
             bi = c;
         }
     }
+    if (rc == MSM_OK && bi == cands.size()) rc = set_err(s, MSM_ERR_HIP, "no pass could be launched");
     (void)hipEventDestroy(e0);
     (void)hipEventDestroy(e1);
     s->timing = saved_timing;
@@ -2536,7 +2544,8 @@ int msm_autotune(msm_sim* s, int reps, int* choice, double* best_ms) {
     enqueue_density(s);
     enqueue_force(s, 0, 1, 0.0);
     if (choice) {
-        const int c[8] = {w.autop ? MSM_PATH_BY_SIZE : w.fp, w.lds, w.bd, w.wd, w.bf, w.wf, s->nlist_kind, w.lanes};
+        const int c[8] = {w.autop ? MSM_PATH_BY_SIZE : w.fp, w.lds, w.bd, w.wd, w.bf, w.wf,
+                          s->nlist_kind, w.lanes};
         for (int k = 0; k < 8; ++k) choice[k] = c[k];
     }
     if (best_ms) {

@@ -40,6 +40,7 @@ int fake_launches(const char* part) {
 
 static err_t fail(err_t e) { return last = e; }
 err_t hipGetLastError(void) { err_t e = last; last = OK; return e; }
+err_t hipPeekAtLastError(void) { return last; }
 const char* hipGetErrorString(err_t e) { return e ? "fake error" : "no error"; }
 
 void** __hipRegisterFatBinary(const void* d) { static void* h; (void)d; return &h; }

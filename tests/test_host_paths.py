@@ -83,6 +83,7 @@ def refused_passes(f):
         f.fake_refuse(kernel)
         assert _hip_error(call), kernel
         f.fake_refuse(b"")
+        dev.build_neighbors()
     dev.calc_force()
     dev.run(2, ctrl.NB_UPTAB, 0, ctrl.H)
     for maxsteps in (1, 2, 3):
@@ -120,7 +121,7 @@ def sort_buffers_after_failures(f):
     for call in (dev.build_neighbors, lambda: dev.run(3, 1, 0, ctrl.H)):
         dev.build_neighbors()
         f.fake_refuse(b"k_scan_blocks")
-        assert _hip_error(dev.build_neighbors)
+        assert _hip_error(call)
         f.fake_refuse(b"")
         fills = f.fake_launches(b"k_fill_int")
         call()
@@ -275,6 +276,41 @@ def copy_out_in_little_memory(f):
     except L.MSMError as e:
         assert e.code == 3      # MSM_ERR_NOMEM
     dev.close()
+
+
+@case
+def refused_in_the_middle(f):
+    """A rebuild whose sort is refused leaves the atoms where they are (the runtime's memory is what it
+    was: nothing moved to the other buffers) and no list; a pass that is refused is no candidate of the
+    autotuner, and no error while others run; a list kernel that is, is one."""
+    import msmpscu_amd._lib as L
+    dev, boxes, ctrl = _device()
+    dev.build_neighbors()
+    for kernel in (b"k_sort_small", b"k_order_move", b"k_nlist"):
+        f.fake_refuse(kernel)
+        lists = f.fake_launches(b"k_nlist")
+        assert _hip_error(dev.build_neighbors)
+        assert f.fake_launches(b"k_nlist") == lists
+        f.fake_refuse(b"")
+        try:
+            dev.calc_force()
+            raise AssertionError("forces from no list")
+        except L.MSMError as e:
+            assert e.code == 7      # MSM_ERR_STATE
+        dev.build_neighbors()
+
+    def state():
+        return [dev.get_option(o) for o in range(L.MSM_OPT_TRACK_DIS, L.MSM_OPT_CHUNK_SWEEP + 1)]
+    before = state()
+    for kernel in (b"k_nlist_small", b"k_order_move", b"k_d"):
+        f.fake_refuse(kernel)
+        assert _hip_error(lambda: dev.autotune(1)), kernel
+        assert state() == before
+        f.fake_refuse(b"")
+        dev.build_neighbors()
+    f.fake_refuse(b"k_force_w")
+    assert dev.autotune(1)["force_path"] not in (L.MSM_PATH_BY_SIZE, 1, 2, 4)
+    dev.calc_force()
 
 
 @pytest.mark.parametrize("name", sorted(CASES))
