@@ -151,9 +151,10 @@ int msm_set_boxes(msm_sim* sim, int nbox, const int* natoms, const double* lo, c
 int msm_set_atoms(msm_sim* sim, int n, const double* xp, const double* xp1, const int* ityp,
                   const int* statu);
 
-/* Copy-out in the caller's atom order; any pointer may be NULL.  Copies beyond 64 KB, in and out, go
- * through pinned memory that the contexts of a GPU share (8 MB from the first such copy on, given back
- * with the last context): one copy at a time, on up to eight host threads. */
+/* Copy-out in the caller's atom order; any pointer may be NULL.  Copies out beyond 4 MB go through
+ * pinned memory that the contexts of a GPU share (8 MB from the first use on, given back with the last
+ * context) on eight host threads, those of several arrays below half a megabyte through it on the
+ * calling thread: one copy at a time. */
 int msm_get_atoms(msm_sim* sim, double* xp, double* xp1, double* fp, int* statu, double* dis);
 /* CopyXPFrom_Host_to_Devices / CopyXP1From_Host_to_Devices (MD_Globle_Variables_GPU.F90:349-373):
  * positions and/or velocities (either may be NULL) of all atoms, (N,3) column-major in the

@@ -367,7 +367,7 @@ void clear_flags(msm_sim* s) {
 
 // A device block (its parts in order, without gaps; total a multiple of 4) to the caller's arrays.
 // Up to 64 KB a kernel writes it into the context's pinned words, which spares the copy engine's
-// start-up; beyond, the ring of msm_copy.h.  Returns with the stream idle and the data in place, or
+// start-up; beyond, msm_copy.h.  Returns with the stream idle and the data in place, or
 // the error of a launch of this call that was refused (the pinned words then hold an earlier copy).
 hipError_t pull(msm_sim* s, const void* base, size_t total, const msm::CopyPart* parts,
                 int nparts) {
@@ -386,7 +386,7 @@ hipError_t pull(msm_sim* s, const void* base, size_t total, const msm::CopyPart*
 // the stream, the caller synchronises before the next push.
 hipError_t push(msm_sim* s, void* dst, const void* host, size_t total) {
     if (total > kSmallCopy)
-        return msm::copy_to_device(s->device, dst, host, total, s->stream);
+        return hipMemcpyAsync(dst, host, total, hipMemcpyHostToDevice, s->stream);
     std::memcpy(s->h_small, host, total);
     msm::launch_copy_words(s->d_small, dst, total, s->stream);
     return hipGetLastError();

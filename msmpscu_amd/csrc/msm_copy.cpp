@@ -67,14 +67,6 @@ void on_threads(int extra, F&& work) {
     for (int k = 0; k < n; ++k) th[k].join();
 }
 
-// Chunk size and extra threads: a thread for every half megabyte.
-void shape(size_t total, size_t& chunk, int& extra) {
-    const size_t want = (total + (kCopySlotBytes / 2) - 1) / (kCopySlotBytes / 2);
-    const int threads = static_cast<int>(std::min<size_t>(std::max<size_t>(want, 1), kCopySlots));
-    extra = threads - 1;
-    chunk = std::min(kCopySlotBytes, (((total + threads - 1) / threads) + 4095) & ~size_t(4095));
-}
-
 }  // namespace
 
 void copy_ring_acquire(int device) {
@@ -97,8 +89,9 @@ hipError_t copy_to_host(int device, const void* base, size_t total, const CopyPa
                         int nparts, hipStream_t stream) {
     // the stream's earlier work ends before the ring is taken, for other streams to use it meanwhile
     const hipError_t idle = hipStreamSynchronize(stream);
-    Ring* r = ring_of(device);
     if (idle != hipSuccess || total == 0) return idle;
+    const bool one_slot = nparts > 1 && total <= kOneSlot;
+    Ring* r = one_slot || total > kRingFrom ? ring_of(device) : nullptr;
     std::unique_lock<std::mutex> g;
     if (r) g = std::unique_lock<std::mutex>(r->mu);
     if (!r || !pinned(*r)) {
@@ -110,12 +103,12 @@ hipError_t copy_to_host(int device, const void* base, size_t total, const CopyPa
         const hipError_t done = hipStreamSynchronize(stream);
         return e != hipSuccess ? e : done;
     }
-    size_t chunk;
-    int extra;
-    shape(total, chunk, extra);
+    // an equal share a slot, in chunks of at most the slot; or all of it through the first
+    const size_t share = ((total + kCopySlots - 1) / kCopySlots + 4095) & ~size_t(4095);
+    const size_t chunk = one_slot ? total : std::min(kCopySlotBytes, share);
     std::atomic<size_t> next{0};
     std::atomic<int> err{hipSuccess};
-    on_threads(extra, [&](int slot) {
+    on_threads(one_slot ? 0 : kCopySlots - 1, [&](int slot) {
         if (slot > 0 && hipSetDevice(device) != hipSuccess) return;
         char* pin = r->base + slot * kCopySlotBytes;
         for (;;) {
@@ -136,44 +129,6 @@ hipError_t copy_to_host(int device, const void* base, size_t total, const CopyPa
                 if (lo < hi)
                     std::memcpy(static_cast<char*>(parts[k].host) + (lo - parts[k].offset),
                                 pin + (lo - a), hi - lo);
-            }
-        }
-    });
-    return static_cast<hipError_t>(err.load());
-}
-
-hipError_t copy_to_device(int device, void* dst, const void* host, size_t total,
-                          hipStream_t stream) {
-    if (total == 0) return hipSuccess;
-    Ring* r = ring_of(device);
-    std::unique_lock<std::mutex> g;
-    if (r) g = std::unique_lock<std::mutex>(r->mu);
-    if (!r || !pinned(*r)) {
-        if (r) g.unlock();
-        const hipError_t e = hipMemcpyAsync(dst, host, total, hipMemcpyHostToDevice, stream);
-        const hipError_t done = hipStreamSynchronize(stream);
-        return e != hipSuccess ? e : done;
-    }
-    size_t chunk;
-    int extra;
-    shape(total, chunk, extra);
-    std::atomic<size_t> next{0};
-    std::atomic<int> err{hipSuccess};
-    on_threads(extra, [&](int slot) {
-        if (slot > 0 && hipSetDevice(device) != hipSuccess) return;
-        char* pin = r->base + slot * kCopySlotBytes;
-        for (;;) {
-            const size_t a = next.fetch_add(chunk);
-            if (a >= total || err.load() != hipSuccess) return;
-            const size_t b = std::min(a + chunk, total);
-            std::memcpy(pin, static_cast<const char*>(host) + a, b - a);
-            hipError_t e = hipMemcpyAsync(static_cast<char*>(dst) + a, pin, b - a,
-                                          hipMemcpyHostToDevice, stream);
-            if (e == hipSuccess) e = hipEventRecord(r->ev[slot], stream);
-            if (e == hipSuccess) e = hipEventSynchronize(r->ev[slot]);
-            if (e != hipSuccess) {
-                err.store(e);
-                return;
             }
         }
     });

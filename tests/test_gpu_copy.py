@@ -1,5 +1,6 @@
-"""Copies to and from the caller's arrays: up to 64 KB through the context's pinned words, beyond
-through the shared ring in chunks.  Sizes around the 64 KB line, around one chunk and over several
+"""Copies to and from the caller's arrays: up to 64 KB through the context's pinned words, to the host
+beyond 4 MB through the shared ring in chunks and up to half a megabyte, where it is several arrays,
+through one slot of it, else plain.  Sizes around these lines, and over several
 rounds of the ring; several contexts at once.  Values come back bit for bit."""
 import threading
 
@@ -51,7 +52,8 @@ def _round_trip(cells, seed):
 
 # 2 * product atoms: one array of 3 n doubles is 64 KB at 2730.7 atoms, all five 104 n at 630.2
 @pytest.mark.parametrize("cells", [(4, 4, 4), (5, 7, 9), (3, 5, 21), (7, 13, 15), (5, 21, 13),
-                                   (21, 26, 40), (41, 41, 42)])
+                                   (21, 26, 40), (41, 41, 42), (26, 27, 29), (27, 27, 29),
+                                   (13, 14, 14), (14, 14, 14)])
 def test_round_trip(cells):
     assert _round_trip(cells, 5)
 

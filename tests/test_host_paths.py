@@ -132,15 +132,21 @@ def sort_buffers_after_failures(f):
 
 @case
 def pinned_ring(f):
-    """Creating a context pins its own few words only, and works where no more can be pinned: large
-    copies are then plain ones.  Else the first large copy pins the ring, which goes with the last
-    context."""
+    """Creating a context pins its own few words only, and works where no more can be pinned: copies
+    are then plain ones.  So are those to the device, and those to the host of one part up to
+    4 MB or of several between half a megabyte and four.  The first of the others pins the
+    ring, which goes with the last context."""
     ring = 8 << 20
     for limit in (ring - 1, -1):
         f.fake_host_limit(limit)
-        dev, boxes, _ = _device((16, 16, 17))
-        other, _, _ = _device((4, 4, 4))
+        dev, boxes, _ = _device((30, 30, 30))      # 5.1 MB (2^20) of per-atom arrays
+        other, _, _ = _device((26, 27, 29))        # 3.9
         other.get_atoms()
+        dev.put_atoms(boxes[0].XP, None)
+        few, _, _ = _device((12, 12, 14))          # 0.4
+        few.get_forces()
+        few.close()
+        dev.set_atoms(boxes[0].XP, boxes[0].XP1, boxes[0].ITYP, boxes[0].STATU)
         small = f.fake_host_bytes()
         assert small < ring // 8
         have = small + (0 if limit > 0 else ring)
@@ -157,6 +163,12 @@ def pinned_ring(f):
         assert f.fake_host_bytes() >= have - small
         other.close()
         assert f.fake_host_bytes() == 0
+    few, _, _ = _device((12, 12, 14))
+    small = f.fake_host_bytes()
+    assert all(set(a.tobytes()) == {0x5a} for a in few.get_atoms())
+    assert f.fake_host_bytes() == small + ring
+    few.close()
+    assert f.fake_host_bytes() == 0
 
 
 @case
